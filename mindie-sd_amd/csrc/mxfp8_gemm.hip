@@ -18,11 +18,26 @@
 // F+f0.., so both halves of an output element meet in the same lane and register); the kernel comment
 // below describes how the tile is walked.  LDS rows are 128 bytes; 16-byte chunk c of row r sits at
 // chunk c ^ ((r >> 1) & 7) (bank-conflict free for the 16-byte operand reads).
+#include <type_traits>
+#include <utility>
+
 #include "common.hpp"
 
 namespace msd {
 
 constexpr float kE4M3MaxMx = 448.0f;
+
+#if defined(__HIP_DEVICE_COMPILE__)
+template <int... I, class F>
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>)
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(std::make_integer_sequence<int, N>{}, f);
+}
+#endif
 
 // ---- MX quantisation of a [M][K] 16-bit matrix along K -----------------------------------------------------
 // 4 lanes share one 32-element block (8 elements = 16 bytes each).
@@ -84,6 +99,10 @@ struct GemmParams {
   int M, K, Nw, Nout;        // Nout = Nw (plain) or Nw/2 (SwiGLU)
   int tiles_m, tiles_n;
 };
+
+__device__ __forceinline__ float silu_mul(float g, float u) {
+  return g * __builtin_amdgcn_rcpf(1.0f + fast_exp2(-1.4426950408889634f * g)) * u;
+}
 
 // Work decomposition: one workgroup of 4 waves (one per SIMD, 256 accumulator registers each) owns a
 // 256 x 256 tile of (X rows) x (W rows), seen as 2 x 2 quadrants of 128 x 128; inside a quadrant every
@@ -151,7 +170,7 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
   // kind: 0 = W0, 1 = A0, 2 = A1, 3 = W1 (the order of consumption).  K blocks past the end are requested
   // through an empty descriptor: the DMA then writes zeros and costs no memory traffic, which keeps the
   // number of outstanding operations the same in every step.
-  auto load_unit = [&](int kb, auto kind_c, int slot) {
+  auto load_unit = [&](int kb, auto kind_c, int slot) __attribute__((always_inline)) {
     constexpr int KIND = decltype(kind_c)::value;
     constexpr bool IS_A = KIND == 1 || KIND == 2, SECOND = KIND >= 2;
     const bool valid = kb < k_blocks;
@@ -183,7 +202,7 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
   // Requested in every eighth step so that the number of outstanding operations repeats with the
   // unrolled loop; the request that falls in the middle of a chunk (or past the end of K) goes through
   // the empty descriptor into a scrap area and costs nothing.
-  auto load_scale_chunk = [&](int t) {  // t: multiple of 8; a chunk is requested 16 steps before its first step
+  auto load_scale_chunk = [&](int t) __attribute__((always_inline)) {  // t: multiple of 8; a chunk is requested 16 steps before its first step
     const int chunk = __builtin_amdgcn_readfirstlane((t + 16) >> 4);
     const bool real = (t & 15) == 0 && 4 * chunk < k_blocks;
     const __amdgpu_buffer_rsrc_t ar = real ? as_rsrc : none_rsrc;
@@ -201,7 +220,7 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
   struct Scales {
     int a[2][2], w[2][2];  // [half][block]: one dword = the 4 MX blocks of one K block
   };
-  auto read_scales = [&](int kb, Scales& s) {
+  auto read_scales = [&](int kb, Scales& s) __attribute__((always_inline)) {
     const int off = ((kb >> 2) & 1) * kScBuf + (kb & 3) * 4;
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf)
@@ -232,7 +251,7 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
     c_off[ks][1] = ((4 * ks + 2 + h) ^ swz) << 4;
   }
   const int a_row_off = (wm * 64 + l32) * BK, w_row_off = (wn * 64 + l32) * BK;
-  auto read_unit = [&](int slot, Frag& f, bool is_a) {
+  auto read_unit = [&](int slot, Frag& f, bool is_a) __attribute__((always_inline)) {
     MSD_LDS const char* base = smem + slot * kUnit + (is_a ? a_row_off : w_row_off);
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk)
@@ -247,7 +266,7 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
   // Workgroup barrier without the memory fence of __syncthreads(): the fence would wait for every DMA in
   // flight, the explicit counts below wait only for the unit that is needed.  The empty asm statements
   // keep the compiler from moving LDS accesses across the barrier.
-  auto wg_barrier = [] {
+  auto wg_barrier = []() __attribute__((always_inline)) {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -285,7 +304,7 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
   // ---- main loop -----------------------------------------------------------------------------------------------------
   // step t = 4 * kb + q computes quadrant q of K block kb from the register sets (fa, fw), loads unit t+2
   // from LDS into fl and requests unit t+9 (into the slot of unit t+1, read during the previous step).
-  auto step = [&](int t, auto j_c, const Frag& fa, const Frag& fw, Frag& fl) {
+  auto step = [&](int t, auto j_c, const Frag& fa, const Frag& fw, Frag& fl) __attribute__((always_inline)) {
     constexpr int J = decltype(j_c)::value;  // t % 8
     constexpr int Q = J & 3;
     constexpr int AH = (Q == 1 || Q == 2) ? 1 : 0, WH = Q >= 2 ? 1 : 0;
@@ -357,7 +376,7 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
   // the wave complete 16 bytes, the four quads and two blocks the 128-byte line).  Output columns of the
   // wave: SwiGLU: f0 + wn*64 + [0,64) (gate from w = 0, up from w = 1); plain: f0 + w*128 + wn*64 + [0,64).
   T* og = (T*)p.out;
-  auto write_tile = [&](auto bias_c) {
+  auto write_tile = [&](auto bias_c) __attribute__((always_inline)) {
     constexpr bool BIAS = decltype(bias_c)::value;
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
@@ -396,7 +415,7 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
                 for (int e = 0; e < 4; ++e) {
                   const float g = acc[a][0][mb][nb][4 * j + e] + bg[e];
                   const float u = acc[a][1][mb][nb][4 * j + e] + bu[e];
-                  v[e] = g * __builtin_amdgcn_rcpf(1.0f + fast_exp2(-1.4426950408889634f * g)) * u;
+                  v[e] = silu_mul(g, u);
                 }
               } else {
                 f32x4_t bv = {0.f, 0.f, 0.f, 0.f};
@@ -417,9 +436,226 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
 #endif
 }
 
+// ---- GEMM on smaller tiles, for grids that 256 x 256 tiles leave mostly empty -------------------------------------------
+// Same operand formats, LDS swizzle and matrix instruction as mxfp8_gemm_kernel.  4 waves own a TM x TN tile (TM, TN 64 or
+// 128; a wave TM/2 x TN/2), K is walked in blocks of 128 codes: a stage holds the block of all TM + TN rows, four stages
+// form a ring (one being read into registers, one landed, two in flight), operands of the next block are read from LDS
+// while the matrix core works on the current one (two register sets).
+//
+// What bounds it: a tile of 128 x 128 takes 0.30 us per K block where its 8 matrix instructions take 0.22 (operands in the
+// L2; with its requests in one burst at the end of the step it was 0.39), and 0.5 us when the operands come from the
+// memory-side cache: a CU alone draws 55 to 70 GB/s from there, and neither deeper prefetch into the L2 by a fifth wave nor
+// a split of K over several workgroups (fp32 sums through memory, 29 to 47 us at 512 x 5120 x 5120) was faster.  Plain GEMM,
+// M x N x K, 256 x 256 tiles before -> now: 512 x 5120 x 5120 57.5 -> 23.8 us, 128 x 5120 x 5120 51.5 -> 12.4 us,
+// 64 x 1536 x 1536 19.5 -> 4.9 us.
+template <int DT, bool SWIGLU, int TM, int TN>
+__global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_small_kernel(const GemmParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  using E = Elem<DT>;
+  using T = typename E::type;
+  constexpr int BK = 128, NS = 4, ROWS = TM + TN;
+  constexpr int MB = TM / 64, NB = TN / 64;   // 32 x 32 blocks of a wave
+  constexpr int kStage = ROWS * BK;
+  constexpr int kDma = ROWS / 32;             // DMA instructions of a wave and stage (8 rows of 128 bytes each)
+  static_assert(!SWIGLU || NB == 2, "gate and up rows of an output column are the two column blocks of a wave");
+  extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
+  MSD_LDS char* smem = (MSD_LDS char*)smem_raw;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, h = lane >> 5;
+  const int wm = wave >> 1, wn = wave & 1;
+
+  // tile order: consecutive tiles of an XCD share their W panel (X is the small operand here)
+  const int per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
+  const int lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (lin >= p.tiles_m * p.tiles_n || (int)(blockIdx.x >> 3) >= per_xcd) return;
+  const int tn = lin / p.tiles_m, tm = lin - tn * p.tiles_m;
+  const int m0 = tm * TM;
+  const int half = p.Nw >> 1;
+  const int f0 = tn * (SWIGLU ? TN / 2 : TN);
+  // W row of tile-local row r: SwiGLU takes, per wave, 32 gate rows and the matching 32 up rows
+  auto w_row = [&](int r) __attribute__((always_inline)) { return SWIGLU ? f0 + (r >> 6) * 32 + (r & 31) + ((r & 32) ? half : 0) : f0 + r; };
+
+  const int k_blocks = p.K / BK;
+
+  // Requests past the last K block keep the outstanding counts as they are: with an empty range the DMA writes zeros and
+  // costs no memory traffic.
+  auto rsrc = [](const unsigned char* base, long long bytes) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00020000);
+  };
+  const int a_bytes = p.M * p.K, w_bytes = p.Nw * p.K, kblk_row = p.K >> 5;
+
+  int voff[kDma];
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) {
+    const int row = 8 * (i * 4 + wave) + (lane >> 3);  // row of the stage: X rows, then W rows
+    const int c = (lane & 7) ^ ((row >> 1) & 7);
+    voff[i] = (i < TM / 32 ? m0 + row : w_row(row - TM)) * p.K + c * 16;
+  }
+  auto load_piece = [&](int kb, int slot, auto i_c) __attribute__((always_inline)) {
+    constexpr int I = decltype(i_c)::value;
+    const int bytes = kb < k_blocks ? (I < TM / 32 ? a_bytes : w_bytes) : 0;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(I < TM / 32 ? p.a : p.w, bytes),
+                                             (MSD_LDS void*)(smem + slot * kStage + wave * 1024 + I * 4096), 16, voff[I],
+                                             kb * BK, 0, 0);
+  };
+  // scales: 16 bytes per row = 4 K blocks, one instruction of 64 rows per wave (waves past the rows: an empty request)
+  constexpr int kScBase = NS * kStage, kScBuf = 4 * 1024;
+  const unsigned char* s_base = 64 * wave < TM ? p.as : p.ws;
+  const int s_bytes = (64 * wave < TM ? p.M : p.Nw) * kblk_row;
+  int s_voff;
+  {
+    const int row = 64 * wave + lane;
+    s_voff = (row < TM ? m0 + row : w_row(row - TM)) * kblk_row;
+  }
+  auto load_scales = [&](int chunk) __attribute__((always_inline)) {
+    const int bytes = (64 * wave < ROWS && 4 * chunk < k_blocks) ? s_bytes : 0;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(s_base, bytes), (MSD_LDS void*)(smem + kScBase + (chunk & 1) * kScBuf + wave * 1024), 16,
+                                             s_voff, chunk * 16, 0, 0);
+  };
+
+  const int swz = (l32 >> 1) & 7, sh = 8 * h;
+  int c_off[2][2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    c_off[ks][0] = ((4 * ks + h) ^ swz) << 4;
+    c_off[ks][1] = ((4 * ks + 2 + h) ^ swz) << 4;
+  }
+  struct Frag {
+    i32x8_t a[MB][2], w[NB][2];  // [block][k step]
+    int as[MB], ws[NB];
+  };
+  const int a_row = wm * (TM / 2) + l32, wr_row = TM + wn * (TN / 2) + l32;
+  // one of the 16-byte reads of a block's operands (X blocks, then W blocks; k step 0 first) or, index -1, its scales
+  constexpr int kReads = 4 * (MB + NB);
+  auto read_piece = [&](int kb, int slot, Frag& f, auto r_c) __attribute__((always_inline)) {
+    constexpr int R = decltype(r_c)::value;
+    if constexpr (R < 0) {
+      MSD_LDS const char* sb = smem + kScBase + ((kb >> 2) & 1) * kScBuf + (kb & 3) * 4;
+#pragma unroll
+      for (int b = 0; b < MB; ++b) f.as[b] = *(MSD_LDS const int*)(sb + (a_row + b * 32) * 16);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) f.ws[b] = *(MSD_LDS const int*)(sb + (wr_row + b * 32) * 16);
+    } else {
+      constexpr int KS = R / (2 * (MB + NB)), Q = R % (2 * (MB + NB)), B = Q >> 1, HL = Q & 1;
+      constexpr bool IS_A = B < MB;
+      const int row = IS_A ? a_row + B * 32 : wr_row + (B - MB) * 32;
+      const i32x4_t v = *(MSD_LDS const i32x4_t*)(smem + slot * kStage + row * BK + c_off[KS][HL]);
+      i32x8_t& d = IS_A ? f.a[IS_A ? B : 0][KS] : f.w[IS_A ? 0 : B - MB][KS];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[4 * HL + j] = v[j];
+    }
+  };
+
+  f32x16_t acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB * NB; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) (&acc[0][0])[i][r] = 0.f;
+
+  auto wg_barrier = []() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // s_waitcnt immediate: vmcnt(N) with every LDS read waited for
+#define MSD_WAIT_VM(N) __builtin_amdgcn_s_waitcnt(((N) & 15) | (((N) >> 4) << 14) | 0x0070)
+
+  load_scales(0);
+#pragma unroll
+  for (int s = 0; s < NS; ++s) static_for<kDma>([&](auto i) __attribute__((always_inline)) { load_piece(s, s, i); });
+  MSD_WAIT_VM((NS - 2) * kDma);  // the scales, stages 0 and 1
+  wg_barrier();
+  Frag fx, fy;
+  read_piece(0, 0, fx, std::integral_constant<int, -1>{});
+  static_for<kReads>([&](auto r) __attribute__((always_inline)) { read_piece(0, 0, fx, r); });
+  MSD_WAIT_VM((NS - 2) * kDma);
+  wg_barrier();
+
+  auto mfma = [&](int ks, i32x8_t w, i32x8_t a, f32x16_t c, int wsc, int asc) __attribute__((always_inline)) {
+    return ks == 0 ? __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w, a, c, 0, 0, 0, wsc, 0, asc)
+                   : __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w, a, c, 0, 0, 2, wsc, 2, asc);
+  };
+  // step kb: products of block kb, reads of block kb + 1 into the other set, request of block kb + 4
+  auto step = [&](int kb, auto j_c, Frag& f, Frag& nf) __attribute__((always_inline)) {
+    constexpr int J = decltype(j_c)::value;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < MB; ++b) f.as[b] = (int)((unsigned)f.as[b] >> sh);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) f.ws[b] = (int)((unsigned)f.ws[b] >> sh);
+    // One wave per SIMD: what is not a matrix instruction has to issue in the shadow of one (64 cycles).  The address unit of
+    // a CU takes a DMA request of 1 KiB in 16 cycles, for 128 x 128 as long in all as the matrix instructions, and a wave
+    // whose request finds the queue full stands still: so the requests are spread evenly, behind the LDS reads of their
+    // matrix instruction.  The reads end early, as their latency has to be over at the end of the step.
+    constexpr int kMfma = 2 * MB * NB, kReadOver = kMfma > 4 ? kMfma - 2 : kMfma, kPer = (kReads + kReadOver - 1) / kReadOver;
+    static_for<kMfma>([&](auto i_c) __attribute__((always_inline)) {
+      constexpr int I = decltype(i_c)::value, KS = I / (MB * NB), nb = I % (MB * NB) / MB, mb = I % MB;
+      acc[mb][nb] = mfma(KS, f.w[nb][KS], f.a[mb][KS], acc[mb][nb], f.ws[nb], f.as[mb]);
+      if constexpr (I == 0) read_piece(kb + 1, (J + 1) & 3, nf, std::integral_constant<int, -1>{});
+      constexpr int R0 = I * kPer < kReads ? I * kPer : kReads, R1 = R0 + kPer < kReads ? R0 + kPer : kReads;
+      static_for<R1 - R0>([&](auto r) __attribute__((always_inline)) {
+        read_piece(kb + 1, (J + 1) & 3, nf, std::integral_constant<int, R0 + decltype(r)::value>{});
+      });
+      if constexpr (I == 0 && J == 0) load_scales((kb >> 2) + 1);
+      constexpr int D0 = I * kDma / kMfma, D1 = (I + 1) * kDma / kMfma;
+      static_for<D1 - D0>([&](auto d) __attribute__((always_inline)) {
+        load_piece(kb + NS, J, std::integral_constant<int, D0 + decltype(d)::value>{});
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    // block kb + 2 must have landed; younger: the requests of this and the step before, with one for scales
+    MSD_WAIT_VM(2 * kDma + (J <= 1 ? 1 : 0));
+    wg_barrier();
+  };
+  for (int kb = 0; kb < k_blocks; kb += 4) {
+    step(kb, std::integral_constant<int, 0>{}, fx, fy);
+    if (kb + 1 < k_blocks) step(kb + 1, std::integral_constant<int, 1>{}, fy, fx);
+    if (kb + 2 < k_blocks) step(kb + 2, std::integral_constant<int, 2>{}, fx, fy);
+    if (kb + 3 < k_blocks) step(kb + 3, std::integral_constant<int, 3>{}, fy, fx);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // the trailing (empty) requests
+#undef MSD_WAIT_VM
+
+  // lane: X row l32 of its blocks, W rows 8 * j + 4 * h + e of its blocks: four consecutive columns per quad
+  f32x4_t bias[NB][4];
+#pragma unroll
+  for (int i = 0; i < 4 * NB; ++i) (&bias[0][0])[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (p.bias) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int row = w_row(wn * (TN / 2) + nb * 32 + 8 * j + 4 * h);  // rows past the end: never stored
+        bias[nb][j] = *(const f32x4_t*)(p.bias + (row < p.Nw ? row : 0));
+      }
+  }
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    const int m = m0 + wm * (TM / 2) + mb * 32 + l32;
+    T* orow = (T*)p.out + (long long)m * p.Nout;
+#pragma unroll
+    for (int nb = 0; nb < (SWIGLU ? 1 : NB); ++nb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int col = f0 + (SWIGLU ? wn * 32 : wn * (TN / 2) + nb * 32) + 8 * j + 4 * h;
+        T t4[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g = acc[mb][nb][4 * j + e] + bias[nb][j][e];
+          t4[e] = E::from_float(SWIGLU ? silu_mul(g, acc[mb][NB - 1][4 * j + e] + bias[NB - 1][j][e]) : g);
+        }
+        if (m < p.M && col < p.Nout) *(i32x2_t*)(orow + col) = *(const i32x2_t*)t4;
+      }
+  }
+#endif
+}
+
 }  // namespace msd
 
 using namespace msd;
+
+constexpr int kCUs = 256;
 
 extern "C" {
 
@@ -457,25 +693,37 @@ int mindiesd_mxfp8_gemm(const void* a, const void* a_scale, const void* w, const
   p.w = (const unsigned char*)w; p.ws = (const unsigned char*)w_scale;
   p.bias = bias; p.out = out;
   p.M = M; p.K = K; p.Nw = Nw; p.Nout = swiglu ? Nw / 2 : Nw;
-  p.tiles_m = (M + 255) / 256;
-  p.tiles_n = swiglu ? (Nw / 2 + 127) / 128 : (Nw + 255) / 256;
-  constexpr int kLds = 8 * 16384 + 2 * 8192 + 1024;  // ring of eight 16 KiB units + two scale chunk buffers + scrap
+  // Tile choice.  A workgroup walks all of K whatever its tile, so a launch takes (rounds over the 256 CUs) x (time of a
+  // tile): 64 x 64, 64 x 128, 128 x 128 and 256 x 256 tiles take 4.9 / 7.0 / 10 / 26 us at K 1536, 8 / 11 / 15.5 / 38.5 us at
+  // K 3072 and 12 / 17.5 / 23.5 / 57 us at K 5120.  Hence the smallest tile whose grid is one round; 128 x 128 tiles still win
+  // in two rounds against one round of 256 x 256 (M 1024, N K 5120: 47 against 58 us), not in three (M 1536: 52 against 59 us
+  // with 480 tiles, M 2048: 82 against 61 us with 640).
+  auto count = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((p.Nout + (swiglu ? tn / 2 : tn) - 1) / (swiglu ? tn / 2 : tn)); };
+  int tm = 256, tn = 256;
+  if (!swiglu && count(64, 64) <= kCUs) tm = tn = 64;
+  else if (count(64, 128) <= kCUs) tm = 64, tn = 128;
+  else if (count(128, 128) <= (count(256, 256) <= kCUs ? 2 * kCUs : kCUs)) tm = tn = 128;
+  p.tiles_m = (M + tm - 1) / tm;
+  p.tiles_n = swiglu ? (p.Nout + tn / 2 - 1) / (tn / 2) : (Nw + tn - 1) / tn;
   const int total = p.tiles_m * p.tiles_n;
   const int grid = (total + 7) / 8 * 8;
-#define MSD_LAUNCH_GEMM(DTV, SW)                                                                                   \
-  {                                                                                                                \
-    auto kern = mxfp8_gemm_kernel<DTV, SW>;                                                                        \
-    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)    \
-      return MSD_ERR_LAUNCH;                                                                                       \
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), kLds, stream, p);                                              \
-  }
-  if (out_dtype == MSD_DTYPE_BF16) {
-    if (swiglu) MSD_LAUNCH_GEMM(MSD_DTYPE_BF16, true) else MSD_LAUNCH_GEMM(MSD_DTYPE_BF16, false)
-  } else {
-    if (swiglu) MSD_LAUNCH_GEMM(MSD_DTYPE_F16, true) else MSD_LAUNCH_GEMM(MSD_DTYPE_F16, false)
-  }
-#undef MSD_LAUNCH_GEMM
-  return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
+  // 256 x 256: ring of eight 16 KiB units + two scale chunk buffers + scrap; small tiles: four stages + two chunk buffers
+  const int lds = tm == 256 ? 8 * 16384 + 2 * 8192 + 1024 : 4 * (tm + tn) * 128 + 8192;
+  auto launch = [&](auto kern) -> int {
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+      return MSD_ERR_LAUNCH;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, stream, p);
+    return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
+  };
+  auto pick = [&](auto dt) -> int {
+    constexpr int DT = decltype(dt)::value;
+    if (tm == 64 && tn == 64) return launch(mxfp8_gemm_small_kernel<DT, false, 64, 64>);
+    if (tm == 64) return swiglu ? launch(mxfp8_gemm_small_kernel<DT, true, 64, 128>) : launch(mxfp8_gemm_small_kernel<DT, false, 64, 128>);
+    if (tm == 128) return swiglu ? launch(mxfp8_gemm_small_kernel<DT, true, 128, 128>) : launch(mxfp8_gemm_small_kernel<DT, false, 128, 128>);
+    return swiglu ? launch(mxfp8_gemm_kernel<DT, true>) : launch(mxfp8_gemm_kernel<DT, false>);
+  };
+  return out_dtype == MSD_DTYPE_BF16 ? pick(std::integral_constant<int, MSD_DTYPE_BF16>{})
+                                     : pick(std::integral_constant<int, MSD_DTYPE_F16>{});
 }
 
 }  // extern "C"

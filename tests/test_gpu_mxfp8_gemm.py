@@ -64,6 +64,42 @@ def test_plain_gemm_with_bias_and_linear_module(cuda):
     assert y.shape == (2, m // 2, n) and torch.equal(y.reshape(m, n).cpu(), out)
 
 
+# one shape per tile of the GEMM's dispatch (64 x 64, 64 x 128, 128 x 128 in one and in two rounds, 256 x 256), each with rows
+# and columns past a tile's edge and K of one, of a few and of a number of blocks that four does not divide
+@pytest.mark.parametrize("m,k,nw,swiglu", [
+    (1, 128, 8, False), (65, 640, 1032, False), (64, 512, 16, True), (700, 128, 3080, False), (130, 384, 2064, True),
+    (1000, 896, 2056, False), (300, 256, 9232, True), (2100, 128, 4104, False), (1100, 640, 6160, True),
+    (4500, 128, 4104, False), (2100, 384, 8208, True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gemm_tiles_vs_oracle(cuda, m, k, nw, swiglu, dtype):
+    """Against the exact product of the quantised operands on sampled rows (all of the first and last tile's edges):
+    the matrix instruction aligns its 64 products to the largest and drops what falls below (measured with the bias set to
+    minus the exact result: 2^-13 of the largest product and instruction at K 128, less at larger K; twice that is allowed),
+    fp32 sums of K products deviate by at most K 2^-24 sum |x w|, the output rounds by 2^-9 (bf16, half an ulp) or 2^-12
+    (fp16), and silu * up carries the error of two sums."""
+    from mindiesd.layers.quant import mx_quantize, mxfp8_matmul
+    x, w, bias = _rand((m, k), 11), _rand((nw, k), 12, scale=0.05), _rand((nw,), 13, dtype=torch.float32)
+    xq, xs = mx_quantize(x.to(cuda))
+    wq, ws = mx_quantize(w.to(cuda))
+    got = mxfp8_matmul(xq, xs, wq, ws, bias.to(cuda), dtype, swiglu).double().cpu()
+    assert got.shape == (m, nw // 2 if swiglu else nw)
+    rows = torch.cat([torch.arange(0, m, max(1, m // 37)), torch.arange(max(0, m - 70), m)]).unique()
+    deq = lambda q, e: (q.float().cpu().view(q.shape[0], -1, 32) * e.float().cpu().unsqueeze(-1)).view(q.shape).double()
+    xd, wd = deq(xq, xs)[rows], deq(wq, ws)
+    want, slack = xd @ wd.T + bias.double(), k * 2.0 ** -24 * (xd.abs() @ wd.abs().T + bias.double().abs())
+    slack += k / 64 * 2.0 ** -12 * xd.abs().amax(1, keepdim=True) * wd.abs().amax(1)
+    if swiglu:
+        g, u = want.chunk(2, -1)
+        sg, su = slack.chunk(2, -1)
+        want = torch.nn.functional.silu(g) * u
+        # |silu'| <= 1.1; exp2, reciprocal and the products add a few fp32 roundings
+        slack = 1.1 * sg * (u.abs() + su) + g.abs() * su + 2.0 ** -18 * (g * u).abs()
+    err = (got[rows] - want).abs()
+    half_ulp = (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12) * 2 * want.abs()
+    tiny = 2.0 ** -25 if dtype == torch.float16 else 0.0
+    assert (err <= half_ulp * (1 + 2.0 ** -6) + slack + tiny).all(), float((err - half_ulp - slack).max())
+
+
 def test_gemm_errors(cuda):
     from mindiesd import ParametersInvalid
     from mindiesd.layers.quant import mx_quantize, mxfp8_matmul
