@@ -31,6 +31,27 @@ FA16_HD Work runs(int block, int groups, int tiles) {
 }
 inline long long runs_grid(long long groups, long long tiles) { return (groups * tiles + 7) / 8 * 8; }
 
+// Runs whose last, partial round is cut finer: of its run of tiles an XCD computes the first `full` as whole tiles, each
+// of the others as `split` workgroups of a part of its rows.
+struct Part {
+  int group;  // < 0: nothing to do
+  int tile;
+  int part;  // -1: the whole tile
+};
+FA16_HD Part runs_tail(int block, int groups, int tiles, int full, int split) {
+  const int total = groups * tiles;
+  const int per_xcd = (total + 7) / 8;
+  const int j = block >> 3;
+  const int local = j < full ? j : full + (j - full) / split;
+  const int work = (block & 7) * per_xcd + local;
+  if (work >= total || local >= per_xcd) return Part{-1, 0, -1};
+  const int group = work / tiles;
+  return Part{group, work - group * tiles, j < full ? -1 : (j - full) % split};
+}
+inline long long runs_tail_grid(long long groups, long long tiles, long long full, long long split) {
+  return 8 * (full + ((groups * tiles + 7) / 8 - full) * split);
+}
+
 // Units of one heavy and one light tile (u and tiles - 1 - u; heavy_first_index: the heavy one is the lower index,
 // as with pairs numbered by descending length, or the higher one, as with causal tiles).  An XCD takes a run of units,
 // starts all its heavy halves first and its light halves last, in reverse.

@@ -30,6 +30,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "fa16_flex.hpp"
 #include "fa_params.hpp"
 
 #ifndef FA16_AHEAD
@@ -65,16 +66,6 @@ struct FaCfg {
 };
 
 #if defined(__HIP_DEVICE_COMPILE__)
-template <int... I, class F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>)
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
-}
-
 // LDS-DMA of one K tile and one V tile: every wave issues G pairs of 1 KiB transfers.
 // Group i of a wave lies 4 * NWAVES rows below group 0 (a multiple of 16, so the swizzles are the same): one
 // per-lane offset per operand serves all groups, the rest goes into the scalar offset.
@@ -708,7 +699,8 @@ __global__ __launch_bounds__(NWAVES * 64, (QPW == 32 ? 2 : 1)) void fa_fwd_kerne
 // query operand is zero from p.head_dim on, and the lanes that would stage the 16-byte chunks of K and V past it
 // request an offset beyond the buffers' range instead, for which the DMA writes zeros without touching memory.  The
 // output columns past p.head_dim are not stored.
-template <int DT, int NWAVES = 8, bool PAIR = false, bool GATHER = false, int GEN = 0, bool DPAD = false>
+template <int DT, int NWAVES = 8, bool PAIR = false, bool GATHER = false, int GEN = 0, bool DPAD = false,
+          int TAIL = 0>
 __global__ __launch_bounds__(NWAVES * 64, 1) void fa_fwd16_kernel(const FaParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using E = Elem<DT>;
@@ -730,7 +722,25 @@ __global__ __launch_bounds__(NWAVES * 64, 1) void fa_fwd16_kernel(const FaParams
   static_assert(!gen || (!PAIR && !GATHER), "general mode: dense tensors in their own order");
   int bn, qt, b, n, Sq, Skv;
   long long q_tok0, k_tok0;  // general mode: first token of the sequence in packed tensors
-  if (!fa16_find_work<GEN, PAIR>(p, kBM, bn, qt, b, n, Sq, Skv, q_tok0, k_tok0)) return;
+  if constexpr (TAIL != 0) {
+    static_assert((GEN == 0 || GEN == 3) && !PAIR && !GATHER && !DPAD && NWAVES == 8, "dense, with or without a key mask");
+    const fa16::Part w = fa16::runs_tail(blockIdx.x, p.B * p.N, (p.Sq + kBM - 1) / kBM, p.tail_full, TAIL);
+    if (w.group < 0) return;
+    if (w.part >= 0) {
+      const int row_base = w.tile * kBM + w.part * (kBM / TAIL);
+      if (row_base < p.Sq) fa16_flex_body<DT, 8, BN, TAIL, GEN == 3>(p, smem, w.group, row_base);
+      return;
+    }
+    bn = w.group;
+    qt = w.tile;
+    b = bn / p.N;
+    n = bn - b * p.N;
+    Sq = p.Sq;
+    Skv = p.Skv;
+    q_tok0 = k_tok0 = 0;
+  } else {
+    if (!fa16_find_work<GEN, PAIR>(p, kBM, bn, qt, b, n, Sq, Skv, q_tok0, k_tok0)) return;
+  }
   const int nkv = n / (p.N / p.Nkv);
   // first query row of this wave; rows at or beyond row_end do not exist (tail of the sequence / of the block)
   int row0 = qt * kBM + wave * 32, row_end = Sq;
@@ -1274,16 +1284,43 @@ __global__ __launch_bounds__(NWAVES * 64, 1) void fa_fwd16_kernel(const FaParams
 #endif  // __HIP_DEVICE_COMPILE__
 }
 
-template <int DT, int NWAVES = 8, bool PAIR = false, bool GATHER = false, int GEN = 0, bool DPAD = false>
+template <int DT, int NWAVES = 8, bool PAIR = false, bool GATHER = false, int GEN = 0, bool DPAD = false, int TAIL = 0>
 static int launch_fa16(const FaParams& p, hipStream_t stream) {
   constexpr int kLds = 4 * 128 * 256;  // two K and two V stages of 128 keys
-  auto kern = fa_fwd16_kernel<DT, NWAVES, PAIR, GATHER, GEN, DPAD>;
+  auto kern = fa_fwd16_kernel<DT, NWAVES, PAIR, GATHER, GEN, DPAD, TAIL>;
   if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
     return MSD_ERR_LAUNCH;
-  const long long grid = fa16_grid<GEN, PAIR>(p, NWAVES * 32);
+  const long long grid = TAIL ? fa16::runs_tail_grid((long long)p.B * p.N, (p.Sq + 255) / 256, p.tail_full, TAIL)
+                              : fa16_grid<GEN, PAIR>(p, NWAVES * 32);
   if (grid > 0x7ffffff0ll) return MSD_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NWAVES * 64), kLds, stream, p);
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
+}
+
+// MINDIESD_DENSE_TILE_ROWS = 256 or 128 in the environment (0: not set): dense and causal calls run as whole tiles of
+// 256 rows, or as workgroups of 128 rows on the 4-wave kernels (the tests reach each kind at every size that way).
+static int forced_tile_rows() {
+  const char* rows = getenv("MINDIESD_DENSE_TILE_ROWS");
+  const int n = rows ? atoi(rows) : 0;
+  return n == 128 || n == 256 ? n : 0;
+}
+
+// Plain dense attention (GEN 0) or with a key mask (GEN 3): how the last round of workgroups is cut.  An XCD runs its
+// share of the 256-row tiles in rounds of 32; when the last round has at most 8 or 16 tiles, they go as four or two
+// workgroups each (fa16_flex.hpp), which still is one round: a round of quarter tiles takes 0.46, one of half tiles 0.62
+// of a round of whole ones, two rounds of either more than one (20 tiles: 140 against 110 us at 5120 keys).
+// B x N 8, keys = queries, before -> now: 4 tiles per XCD 21 -> 15 us, 16 tiles 71 -> 62 us, 32 + 1 tiles 350 -> 278 us,
+// 32 + 16 tiles 538 -> 467 us, 64 + 8 tiles 1245 -> 1042 us; 46 * 32 + 8 tiles (40 heads, 75600) 85.2 -> 84.1 ms.
+template <int DT, int GEN>
+static int launch_fa16_rounds(FaParams p, hipStream_t stream) {
+  const long long per_xcd = ((long long)p.B * p.N * ((p.Sq + 255) / 256) + 7) / 8;
+  constexpr int kCusPerXcd = 32;
+  const int rest = (int)(per_xcd % kCusPerXcd);
+  if (rest == 0 || 2 * rest > kCusPerXcd || forced_tile_rows() == 256)
+    return launch_fa16<DT, 8, false, false, GEN>(p, stream);
+  p.tail_full = (int)(per_xcd - rest);
+  if (4 * rest > kCusPerXcd) return launch_fa16<DT, 8, false, false, GEN, false, 2>(p, stream);
+  return launch_fa16<DT, 8, false, false, GEN, false, 4>(p, stream);
 }
 
 template <int DT, int NWAVES, int QPW, int BN, bool SPARSE, int SCHED, int MODE = 0, bool GATHER = false,
@@ -1461,14 +1498,13 @@ int mindiesd_block_sparse_attention_paired_fwd(const void* q, const void* k, con
                      : launch_fa<MSD_DTYPE_F16, 4, 32, 64, true, 1, 0, false, true>(p, stream);
 }
 
-// True when B x N x ceil(Sq / 256) workgroups of 256 rows would fill the chip badly (see mindiesd_flash_attention_fwd).
+// True when B x N x ceil(Sq / 256) workgroups of 256 rows would fill the 256 CUs badly - at most half of them busy, or
+// a second round for at most half of them - for the calls whose rounds launch_fa16_rounds does not cut: head dims up to
+// 64 and causal ones.  They run as 128-row workgroups of four waves, two to a CU.
 static bool prefers_half_tiles(int B, int N, int Sq) {
   const long long tiles256 = (long long)B * N * ((Sq + 255) / 256);
   bool half_tiles = 2 * tiles256 <= kCus || (tiles256 > kCus && 2 * tiles256 <= 3 * kCus);
-  if (const char* rows = getenv("MINDIESD_DENSE_TILE_ROWS")) {
-    if (atoi(rows) == 256) half_tiles = false;
-    if (atoi(rows) == 128) half_tiles = true;
-  }
+  if (const int rows = forced_tile_rows()) half_tiles = rows == 128;
   return half_tiles;
 }
 
@@ -1481,10 +1517,6 @@ int mindiesd_flash_attention_fwd(const void* q, const void* k, const void* v, vo
   const int rc = check_common(q, k, v, out, dtype, B, N, Nkv, Sq, Skv, D, st, scale, true);
   if (rc != MSD_OK) return rc;
   FaParams p = make_params(q, k, v, out, lse, B, N, Nkv, Sq, Skv, st, scale);
-  // Grids of 256-row workgroups that fill the 256 CUs badly - at most half of them busy, or a second round for at
-  // most half of them - run as 128-row workgroups of four waves, two to a CU (head dims 128 and up to 64).
-  // MINDIESD_DENSE_TILE_ROWS = 256 or 128 in the environment overrides the choice (the tests reach both kinds of
-  // kernel at every size that way).
   const bool half_tiles = prefers_half_tiles(B, N, Sq);
   if (D == 64 && fa16_d64_supported(p)) return launch_fa16_d64(p, dtype, stream, 0, half_tiles ? 128 : 256);
   // Head dims between 64 and 128 run as head_dim 128 on the 16x16x32 kernel (the part of the matrix work spent on
@@ -1504,16 +1536,13 @@ int mindiesd_flash_attention_fwd(const void* q, const void* k, const void* v, vo
   // A few key tiles per query tile (cross attention over a short text): the launch is mostly reading Q and writing O,
   // and two 4-wave workgroups per CU overlap one's memory phases with the other's tiles better than one 8-wave
   // workgroup does (75600 queries x 40 heads: 0.42 vs 0.53 ms at 77 keys, 0.62 vs 0.70 at 226, equal at 512).
-  // The same 4-wave kernel takes the grids that fill the chip badly (half_tiles above): it reaches 86 % of the 8-wave
-  // kernel's rate on a full chip, and B x N = 16: S 1024 / 1536 / 2048 31 -> 25, 43 -> 35, 56 -> 46 us, S 4608 (288
-  // workgroups of 256 rows) 218 -> 206 us; 24 heads at S 3072: 152 -> 139 us.  (In between - 129 .. 256 workgroups -
-  // and from 385 on the 8-wave kernel is faster.)
-  if (Skv <= kShortKv || half_tiles) {
+  // (Grids of whatever size on more keys than that: launch_fa16_rounds.)
+  if (Skv <= kShortKv || forced_tile_rows() == 128) {
     if (dtype == MSD_DTYPE_BF16) return launch_fa<MSD_DTYPE_BF16, 4, 32, 64, false, 1, 1>(p, stream);
     return launch_fa<MSD_DTYPE_F16, 4, 32, 64, false, 1, 1>(p, stream);
   }
-  if (dtype == MSD_DTYPE_BF16) return launch_fa16<MSD_DTYPE_BF16>(p, stream);
-  return launch_fa16<MSD_DTYPE_F16>(p, stream);
+  if (dtype == MSD_DTYPE_BF16) return launch_fa16_rounds<MSD_DTYPE_BF16, 0>(p, stream);
+  return launch_fa16_rounds<MSD_DTYPE_F16, 0>(p, stream);
 }
 
 // Block-sparse attention with an optional causal mask inside the selected blocks (queries and keys of equal
@@ -1604,8 +1633,8 @@ int mindiesd_flash_attention_general_fwd(const void* q, const void* k, const voi
   }
   if (D != 128) return launch_fa_hd(p, dtype, D, stream);
   if (key_mask && long_rows) {
-    if (dtype == MSD_DTYPE_BF16) return launch_fa16<MSD_DTYPE_BF16, 8, false, false, 3>(p, stream);
-    return launch_fa16<MSD_DTYPE_F16, 8, false, false, 3>(p, stream);
+    if (dtype == MSD_DTYPE_BF16) return launch_fa16_rounds<MSD_DTYPE_BF16, 3>(p, stream);
+    return launch_fa16_rounds<MSD_DTYPE_F16, 3>(p, stream);
   }
   if (mask) {
     if (dtype == MSD_DTYPE_BF16) return launch_fa<MSD_DTYPE_BF16, 4, 32, 64, false, 1, 2>(p, stream);

@@ -44,6 +44,23 @@ static void cover(const char* name, int groups, int tiles, long long grid, F&& f
   }
 }
 
+// runs with the last round cut: every part of every cut tile and every whole tile once
+static void cover_tail(int groups, int tiles, int full, int split) {
+  std::vector<int> seen((size_t)groups * tiles, 0);
+  for (long long block = 0; block < runs_tail_grid(groups, tiles, full, split); ++block) {
+    const Part w = runs_tail((int)block, groups, tiles, full, split);
+    if (w.group < 0) continue;
+    if (w.group >= groups || w.tile < 0 || w.tile >= tiles || w.part >= split) fail("tail", groups, tiles, (int)block);
+    const int bits = w.part < 0 ? (1 << split) - 1 : 1 << w.part;
+    int& s = seen[(size_t)w.group * tiles + w.tile];
+    if (s & bits) fail("tail", groups, tiles, (int)block);
+    s |= bits;
+    ++checks;
+  }
+  for (int s : seen)
+    if (s != (1 << split) - 1) fail("tail", groups, tiles, -1);
+}
+
 int main(int argc, char** argv) {
   if (argc != 3) return 2;
   const int groups = std::atoi(argv[1]), tiles = std::atoi(argv[2]);
@@ -60,6 +77,11 @@ int main(int argc, char** argv) {
         false);
   cover("spread, packed", groups, tiles, runs_grid(groups, tiles + 5), [&](int b) { return spread(b, groups, tiles, true); },
         false);
+  const int per_xcd = (groups * tiles + 7) / 8;
+  for (int split = 2; split <= 4; split += 2) {
+    cover_tail(groups, tiles, per_xcd / 32 * 32, split);
+    cover_tail(groups, tiles, 0, split);
+  }
   std::printf("%lld checks passed\n", checks);
   return 0;
 }

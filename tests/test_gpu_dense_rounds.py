@@ -1,0 +1,80 @@
+"""Dense attention at head_dim 128 where the last round of workgroups is cut into half or quarter tiles
+(launch_fa16_rounds): whole rounds before it or none, tiles per XCD at the edges of the rule, ragged query and key
+lengths around the 64-, 128- and 256-row and the 128-key tiles, both layouts and types, and the key-padding mask.
+
+Bounds against the float64 softmax of the same 16-bit operands: the query is rounded to 16 bits after scaling and a
+probability before the second product (a relative u = 2^-9 for bf16, 2^-12 for fp16, each), the output once more; in the
+2-norm 3 u covers their sum, an element lies within 16 u of the largest absolute value of v."""
+import pytest
+import torch
+
+import mindiesd
+
+pytestmark = pytest.mark.gpu
+U = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}
+
+
+def reference(q, k, v, mask=None):
+    out = []
+    for b in range(q.shape[0]):
+        for n in range(q.shape[1]):
+            s = q[b, n].double() @ k[b, n].double().t() * q.shape[-1] ** -0.5
+            if mask is not None:
+                s = s.masked_fill(~mask[b].view(1, -1), float("-inf"))
+            out.append(torch.softmax(s, -1) @ v[b, n].double())
+    return torch.stack(out).view(q.shape)
+
+
+def check(got, want, v, dtype):
+    err = got.double() - want
+    assert torch.isfinite(got).all()
+    assert (err.norm() / want.norm()).item() <= 3 * U[dtype]
+    assert err.abs().max().item() <= 16 * U[dtype] * v.abs().max().item()
+
+
+# heads x ceil(q_len / 256) tiles over 8 XCDs: tiles per XCD 1, 1, 8, 9, 16, 17 (no round before the last),
+# 32 + 1, 32 + 8, 32 + 9, 32 + 16, 64 + 3
+CASES = [(1, 1, 385), (3, 257, 512), (64, 129, 1000), (72, 200, 513), (43, 700, 641), (136, 256, 400),
+         (264, 193, 400), (160, 300, 577), (164, 511, 390), (128, 641, 700), (536, 65, 450)]
+
+
+@pytest.mark.parametrize("heads,q_len,kv_len", CASES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("masked", [False, True])
+def test_cut_rounds(heads, q_len, kv_len, dtype, masked):
+    if masked and q_len < 256:
+        q_len += 256                      # key masks run on this kernel from 256 query rows on
+    print("case", heads, q_len, kv_len, dtype, masked, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(heads + q_len)
+    q, k, v = (torch.randn((1, heads, s, 128), generator=g, device="cuda").to(dtype) for s in (q_len, kv_len, kv_len))
+    mask = None
+    if masked:
+        mask = torch.rand((1, kv_len), generator=g, device="cuda") < 0.5
+        mask[:, :70] = False              # the first groups of keys and all of a group's keys in the last tile hidden
+        mask[:, kv_len - kv_len % 128 - 20:] = False
+        mask[:, 200] = True
+    want = reference(q, k, v, mask)
+    m4 = None if mask is None else mask.view(1, 1, 1, kv_len)
+    check(mindiesd.attention_forward(q, k, v, attn_mask=m4, head_first=True), want, v, dtype)
+    t = [x.transpose(1, 2).contiguous() for x in (q, k, v)]
+    check(mindiesd.attention_forward(*t, attn_mask=m4, head_first=False).transpose(1, 2), want, v, dtype)
+
+
+def test_groups_of_very_different_maxima():
+    """The groups of waves that share a row keep reference maxima of their own: scores that differ by hundreds between
+    the groups' keys, rows whose scores all lie far below zero, and a NaN and an infinity that stay in their rows."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn((1, 4, s, 128), generator=g, device="cuda").bfloat16() for s in (512, 640, 640))
+    q[:, :, :, 0] = 4.0
+    k[:, :, :, 0] = torch.where(torch.arange(640, device="cuda") % 128 < 64, -900.0, -300.0).view(1, 1, -1).bfloat16()
+    q[:, 1, :, 0] = -4.0
+    q[:, 2, :, 0] = torch.where(torch.arange(512, device="cuda") % 2 == 0, 4.0, -0.5).bfloat16()
+    check(mindiesd.attention_forward(q, k, v, head_first=True), reference(q, k, v), v, torch.bfloat16)
+    clean = mindiesd.attention_forward(q, k, v, head_first=True)
+    q[0, 3, 17, 5] = float("nan")
+    q[0, 3, 300, 5] = float("inf")
+    out = mindiesd.attention_forward(q, k, v, head_first=True)
+    bad = torch.zeros_like(out, dtype=torch.bool)
+    bad[0, 3, 17] = bad[0, 3, 300] = True
+    assert torch.isnan(out[bad]).all()
+    assert torch.equal(out[~bad], clean[~bad])
