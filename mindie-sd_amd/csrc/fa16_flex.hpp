@@ -1,9 +1,11 @@
 // The body of fa_fwd16_kernel (flash_attn_fwd.hip: dense attention at head_dim 128 on the 16x16x32 matrix instruction)
-// for workgroups that own fewer query rows: NW waves of 32 rows each walk key tiles of BN keys, and with KS > 1 the
-// waves form KS groups that share the same NW / KS * 32 query rows, each taking BN / KS keys of every tile with a
-// running softmax of its own; the groups' sums and outputs are added up in LDS at the end, in 32 bits.
+// in two other shapes of work.  NW waves of 32 rows each walk key tiles of BN keys.
 //
-// Why: the launch time of fa_fwd16_kernel is rounds of 256 workgroups of 256 rows, and a round that is a quarter full
+// KS 1: a workgroup that keeps its CU and goes from one tile of rows to the next (fa16_loop_kernel states why).
+//
+// KS > 1: workgroups that own fewer query rows: the waves form KS groups that share the same NW / KS * 32 query rows, each
+// taking BN / KS keys of every tile with a running softmax of its own; the groups' sums and outputs are added up in LDS
+// at the end, in 32 bits.  Why: the launch time of fa_fwd16_kernel is rounds of 256 workgroups of 256 rows, and a round that is a quarter full
 // takes as long as a full one.  A workgroup of 128 (KS 2) or 64 rows (KS 4) has half or a quarter of the matrix and
 // vector work per tile for the same number of waves, so its walk over the keys takes about half or a third of the time
 // (the L2 -> LDS stream of a tile stays what it is, 64 KiB per 128 keys, and bounds KS 4).  No workspace, no second launch.
@@ -29,10 +31,13 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 
-// bn: (batch, head) index; row_base: first query row of the workgroup (rows at or beyond p.Sq do not exist).
-// LDS: K stages at 0 and BN * 256 bytes, V stages behind them; swizzles and operand layouts as in fa_fwd16_kernel.
+// item: the first tile of NW / KS * 32 query rows, numbered through the heads ((batch, head) * row_tiles + tile; rows at
+// or beyond p.Sq do not exist); part: KS > 1, which part of a tile of NW * 32 rows it is.  KS 1: the workgroup goes on with
+// the tiles item + 32, item + 64, ... below `end`.
+// LDS: K stages at 0 and BN * 256 bytes, V stages behind them, with KS 1 the output staging behind those; swizzles and
+// operand layouts as in fa_fwd16_kernel.
 template <int DT, int NW, int BN, int KS, bool KEYMASK>
-__device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* smem, int bn, int row_base) {
+__device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* smem, int item, int part, int end) {
   using E = Elem<DT>;
   using T = typename E::type;
   using X8 = typename E::x8;
@@ -47,21 +52,25 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   const int rg = wave % RG, kg_i = wave / RG;
-  const int b = bn / p.N, n = bn - b * p.N;
-  const int nkv = n / (p.N / p.Nkv);
+  constexpr bool LOOP = KS == 1;
   const int Sq = p.Sq, Skv = p.Skv;
-  const int row0 = row_base + rg * 32;
-
-  const T* qg = (const T*)p.q + b * p.q_sb + n * p.q_sn;
-  const T* kg = (const T*)p.k + b * p.k_sb + nkv * p.k_sn;
-  const T* vg = (const T*)p.v + b * p.v_sb + nkv * p.v_sn;
-  T* og = (T*)p.o + b * p.o_sb + n * p.o_sn;
+  const int row_tiles = (Sq + NW * 32 - 1) / (NW * 32);
+  // the tile at hand, and with LOOP the one after it
+  int b, n, row0, b_nx = 0, n_nx = 0, row0_nx = 0;
+  auto locate = [&](int it, int& ib, int& in, int& irow) __attribute__((always_inline)) {
+    const int bn = it / row_tiles;
+    ib = bn / p.N;
+    in = bn - ib * p.N;
+    irow = (it - bn * row_tiles) * (NW * 32) + part * (NW / KS * 32) + rg * 32;
+  };
+  locate(item, b, n, row0);
 
   // ---- staging (LDS-DMA) -------------------------------------------------------------------------------------
-  const __amdgpu_buffer_rsrc_t k_rsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)kg, 0, (int)(((long long)(Skv - 1) * p.k_ss + 128) * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t v_rsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)vg, 0, (int)(((long long)(Skv - 1) * p.v_ss + 128) * 2), 0x00020000);
+  const int group = p.N / p.Nkv;
+  const int k_range = (int)(((long long)(Skv - 1) * p.k_ss + 128) * 2), v_range = (int)(((long long)(Skv - 1) * p.v_ss + 128) * 2);
+  auto k_base = [&](int ib, int in) __attribute__((always_inline)) { return (const T*)p.k + ib * p.k_sb + (in / group) * p.k_sn; };
+  auto v_base = [&](int ib, int in) __attribute__((always_inline)) { return (const T*)p.v + ib * p.v_sb + (in / group) * p.v_sn; };
+  const T *kg = k_base(b, n), *vg = v_base(b, n), *kg_nx = kg, *vg_nx = vg;
   const int k_row_bytes = (int)p.k_ss * 2, v_row_bytes = (int)p.v_ss * 2;
   int k_voff, v_voff;
   {
@@ -70,7 +79,9 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     k_voff = row * k_row_bytes + ((pc ^ (row & 15)) << 4);
     v_voff = row * v_row_bytes + (((((pc >> 1) ^ (row & 7)) << 1) | (pc & 1)) << 4);
   }
-  auto load_tile = [&](int key0, int stage) __attribute__((always_inline)) {
+  auto load_tile = [&](const T* kp, const T* vp, int key0, int stage) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, k_range, 0x00020000);
+    const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, v_range, 0x00020000);
 #pragma unroll
     for (int i = 0; i < BN / 4 / NW; ++i) {
       const int grp = i * NW + wave;
@@ -81,34 +92,25 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     }
   };
 
-  // ---- Q^T operand, resident ---------------------------------------------------------------------------------
+  // ---- Q^T operand, resident: requested here, converted at the start of its tile ------------------------------------
   X8 qf[2][4];
+  auto load_q = [&](int ib, int in, int irow) __attribute__((always_inline)) {
+    const T* qg = (const T*)p.q + ib * p.q_sb + in * p.q_sn;
+    int c = lane & 15, g = lane >> 4;
+    if constexpr (LOOP) asm volatile("" : "+v"(c), "+v"(g));  // (recomputed for every tile, not kept in registers)
 #pragma unroll
-  for (int nq = 0; nq < 2; ++nq) {
-    const int qrow = row0 + nq * 16 + c;
-    const bool ok = qrow < Sq;
-    const T* src = qg + (long long)(ok ? qrow : 0) * p.q_ss + 8 * g;
+    for (int nq = 0; nq < 2; ++nq) {
+      const int qrow = irow + nq * 16 + c;
+      const T* src = qg + (long long)(qrow < Sq ? qrow : 0) * p.q_ss + 8 * g;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      X8 v = *(const X8*)(src + 32 * ks);
-      if (!ok) v = X8{0};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = E::from_float((float)v[j] * p.scale_log2);
-      qf[nq][ks] = v;
+      for (int ks = 0; ks < 4; ++ks) qf[nq][ks] = *(const X8*)(src + 32 * ks);
     }
-  }
+  };
   f32x4_t oacc[8][2], negm[2], lt[2];
   float l_run[2];
   X8 ones;
 #pragma unroll
   for (int j = 0; j < 8; ++j) ones[j] = E::from_float(1.f);
-#pragma unroll
-  for (int nq = 0; nq < 2; ++nq) {
-    l_run[nq] = 0.f;
-    negm[nq] = lt[nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int db = 0; db < 8; ++db) oacc[db][nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
 
   // per-lane parts of the LDS read addresses (the wave's keys start at row kg_i * kKeys, a multiple of 16)
   unsigned k_lds[4], v_lds[4];
@@ -121,7 +123,8 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
                 ((db ^ (4 * (g & 1) + (c >> 2))) << 5) + 8 * (c & 3);
 
   const int tiles = (Skv + BN - 1) / BN;
-  load_tile(0, 0);
+  load_q(b, n, row0);
+  load_tile(kg, vg, 0, 0);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();
   bool first = true;
@@ -129,7 +132,6 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   // ---- key mask: words of visible keys of the current tile, bit l of word j = key 4 * l + j -----------------------------
   unsigned kvis[4] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu}, kraw = 0;
   const unsigned char* mask_g = nullptr;
-  if constexpr (KEYMASK) mask_g = p.mask + b * p.m_sb + n * p.m_sn;
   auto mask_request = [&](int key0) __attribute__((always_inline)) {
     if constexpr (KEYMASK) {
       kraw = 0;
@@ -153,14 +155,12 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     }
   };
   constexpr unsigned kOwn = (unsigned)((1ull << (kKeys / 4)) - 1);
-  if constexpr (KEYMASK) {
-    mask_request(0);
-    mask_reduce();
-  }
 
-  auto tile_step = [&](auto stage_c, const int key0, const int next_key0) __attribute__((always_inline)) {
+  // next_tile: the first key of the tile to request, of the workgroup's next tile of rows with `other`; < 0: none
+  auto tile_step = [&](auto stage_c, const int key0, const int next_tile, const bool other) __attribute__((always_inline)) {
     constexpr int stage = decltype(stage_c)::value;
-    if (next_key0 >= 0) load_tile(next_key0, stage ^ 1);
+    if (next_tile >= 0) load_tile(other ? kg_nx : kg, other ? vg_nx : vg, next_tile, stage ^ 1);
+    const int next_key0 = other ? -1 : next_tile;
     const unsigned kv_all = kvis[0] & kvis[1] & kvis[2] & kvis[3] & kOwn;
     const int key_w = key0 + kg_i * kKeys;  // the wave's first key
 
@@ -232,7 +232,21 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
         for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sacc[kb][nq][i]);
       if constexpr (KEYMASK) seen = seen || __builtin_amdgcn_ballot_w64(mx > -INFINITY) != 0;
       l_run[nq] += lt[nq][0];
-      if (first || __builtin_amdgcn_ballot_w64(mx > kTau) != 0) {
+      if constexpr (NKB == 8) {  // (see cond_rescale_fa16)
+        float delta = 0.f, alpha = 1.f;
+        int moved = 0;
+        if (first || __builtin_amdgcn_ballot_w64(mx > kTau) != 0) {
+          mx = quarter_max(mx);
+          delta = first ? mx : fmaxf(mx, 0.f);
+          delta = (delta == -INFINITY) ? 0.f : delta;
+          alpha = first ? 1.f : fast_exp2(-delta);
+          moved = 1;
+        }
+        cond_rescale_fa16(__builtin_amdgcn_readfirstlane(moved), delta, alpha, l_run[nq], negm[nq], sacc[0][nq], sacc[1][nq],
+                          sacc[2][nq], sacc[3][nq], sacc[NKB - 4][nq], sacc[NKB - 3][nq], sacc[NKB - 2][nq],
+                          sacc[NKB - 1][nq], oacc[0][nq], oacc[1][nq], oacc[2][nq], oacc[3][nq], oacc[4][nq], oacc[5][nq],
+                          oacc[6][nq], oacc[7][nq]);
+      } else if (first || __builtin_amdgcn_ballot_w64(mx > kTau) != 0) {
         mx = quarter_max(mx);
         float delta = first ? mx : fmaxf(mx, 0.f);
         delta = (delta == -INFINITY) ? 0.f : delta;
@@ -305,9 +319,57 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     mask_reduce();
     __syncthreads();
   };
+  for (;;) {
+  if constexpr (KEYMASK) {
+    mask_g = p.mask + b * p.m_sb + n * p.m_sn;
+    mask_request(0);
+    mask_reduce();
+  }
+#pragma unroll
+  for (int nq = 0; nq < 2; ++nq) {
+    int cc = c;
+    if constexpr (LOOP) asm volatile("" : "+v"(cc));
+    const bool ok = row0 + nq * 16 + cc < Sq;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      X8 v = qf[nq][ks];
+      if (!ok) v = X8{0};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = E::from_float((float)v[j] * p.scale_log2);
+      qf[nq][ks] = v;
+    }
+    l_run[nq] = 0.f;
+    negm[nq] = lt[nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int db = 0; db < 8; ++db) oacc[db][nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  first = true;
+  bool more = false;
+  unsigned touched = 0;
+  if constexpr (LOOP) {
+    more = item + 32 < end;
+    if (more) {
+      locate(item + 32, b_nx, n_nx, row0_nx);
+      kg_nx = k_base(b_nx, n_nx);
+      vg_nx = v_base(b_nx, n_nx);
+      // a word of every 128-byte line of the next rows of q, so that they wait in the L2
+      const int qrow = min(row0_nx - rg * 32 + (tid >> 1), Sq - 1);
+      touched = *(const unsigned*)((const T*)p.q + b_nx * p.q_sb + n_nx * p.q_sn + (long long)qrow * p.q_ss + (tid & 1) * 64);
+    }
+  }
   for (int t = 0; t < tiles; t += 2) {
-    tile_step(std::integral_constant<int, 0>{}, t * BN, t + 1 < tiles ? (t + 1) * BN : -1);
-    if (t + 1 < tiles) tile_step(std::integral_constant<int, 1>{}, (t + 1) * BN, t + 2 < tiles ? (t + 2) * BN : -1);
+    tile_step(std::integral_constant<int, 0>{}, t * BN, t + 1 < tiles ? (t + 1) * BN : -1, false);
+    // (an even number of key tiles: the last step requests the first key tile of the next rows)
+    if (t + 1 < tiles)
+      tile_step(std::integral_constant<int, 1>{}, (t + 1) * BN, t + 2 < tiles ? (t + 2) * BN : (LOOP && more ? 0 : -1),
+                LOOP && t + 2 >= tiles);
+  }
+  if constexpr (LOOP) {
+    asm volatile("" ::"v"(touched));
+    if (more) {  // (an odd number: it goes into the stage of the last step, which no wave reads any more)
+      load_q(b_nx, n_nx, row0_nx);
+      if (tiles & 1) load_tile(kg_nx, vg_nx, 0, 0);
+    }
   }
 
   // ---- the groups' partial results (KS > 1) --------------------------------------------------------------------------
@@ -319,7 +381,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   constexpr int kStat = KS > 1 ? 4 * 256 : 0;      // m and l of two column blocks, a dword per lane
   constexpr int kORow = 2 * 16 * DB + 8;           // a row of the output staging, padded
   constexpr int kOBase = KS > 1 ? NW * (kPart + kStat) : 0;
-  static_assert(kOBase + NW * 32 * kORow <= 4 * BN * 256, "fits the tile stages");
+  static_assert(KS == 1 || kOBase + NW * 32 * kORow <= 4 * BN * 256, "fits the tile stages");
   float l_tot[2], m_tot[2];
 #pragma unroll
   for (int nq = 0; nq < 2; ++nq) {
@@ -389,6 +451,49 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   }
 
   // ---- normalise, transpose the wave's rows through LDS, coalesced store ----------------------------------------------
+  T* og = (T*)p.o + b * p.o_sb + n * p.o_sn;
+  if constexpr (LOOP) {
+    // 16 rows at a time through 4 KiB per wave behind the tile stages (which already fill with the next rows' keys):
+    // 16-byte chunk k of row r sits at chunk k ^ r
+    MSD_LDS char* ost = smem + 4 * BN * 256 + wave * 4096;
+    int c = lane & 15, g = lane >> 4;
+    asm volatile("" : "+v"(c), "+v"(g));
+#pragma unroll
+    for (int nq = 0; nq < 2; ++nq) {
+      const float inv = l_tot[nq] > 0.f ? 1.f / l_tot[nq] : 0.f;
+      const int qrow_l = row0 + nq * 16 + c;
+      if (p.lse && g == 0 && qrow_l < Sq)
+        p.lse[((long long)b * p.N + n) * Sq + qrow_l] =
+            l_tot[nq] > 0.f ? m_tot[nq] * 0.6931471805599453f + __logf(l_tot[nq]) : -INFINITY;
+#pragma unroll
+      for (int db = 0; db < 8; ++db) {
+        typename E::x4 pk;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pk[i] = E::from_float(oacc[db][nq][i] * inv);
+        *(MSD_LDS typename E::x4*)(ost + c * 256 + (((2 * db + (g >> 1)) ^ c) << 4) + 8 * (g & 1)) = pk;
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 4 * i + g, qrow = row0 + nq * 16 + row;
+        const i32x4_t v = *(MSD_LDS const i32x4_t*)(ost + row * 256 + ((c ^ row) << 4));
+        if (qrow < Sq) *(i32x4_t*)(og + (long long)qrow * p.o_ss + c * 8) = v;
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (!more) return;
+    item += 32;
+    b = b_nx;
+    n = n_nx;
+    row0 = row0_nx;
+    kg = kg_nx;
+    vg = vg_nx;
+    if (tiles & 1) {
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+      __syncthreads();
+    }
+    continue;
+  }
   MSD_LDS char* ost = smem + kOBase + wave * 32 * kORow;
 #pragma unroll
   for (int nq = 0; nq < 2; ++nq) {
@@ -415,6 +520,8 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     const i32x2_t lo = *(MSD_LDS const i32x2_t*)(ost + row * kORow + c16 * 16);
     const i32x2_t hi = *(MSD_LDS const i32x2_t*)(ost + row * kORow + c16 * 16 + 8);
     if (qrow < Sq) *(i32x4_t*)(og + (long long)qrow * p.o_ss + kg_i * (16 * DB) + c16 * 8) = i32x4_t{lo[0], lo[1], hi[0], hi[1]};
+  }
+  return;
   }
 }
 #endif

@@ -727,8 +727,8 @@ __global__ __launch_bounds__(NWAVES * 64, 1) void fa_fwd16_kernel(const FaParams
     const fa16::Part w = fa16::runs_tail(blockIdx.x, p.B * p.N, (p.Sq + kBM - 1) / kBM, p.tail_full, TAIL);
     if (w.group < 0) return;
     if (w.part >= 0) {
-      const int row_base = w.tile * kBM + w.part * (kBM / TAIL);
-      if (row_base < p.Sq) fa16_flex_body<DT, 8, BN, TAIL, GEN == 3>(p, smem, w.group, row_base);
+      if (w.tile * kBM + w.part * (kBM / TAIL) < p.Sq)
+        fa16_flex_body<DT, 8, BN, TAIL, GEN == 3>(p, smem, w.group * ((p.Sq + kBM - 1) / kBM) + w.tile, w.part, 0);
       return;
     }
     bn = w.group;
@@ -1297,6 +1297,33 @@ static int launch_fa16(const FaParams& p, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
 }
 
+// Dense attention over a few key tiles (cross attention) by one workgroup per CU that goes through its XCD's tiles of rows:
+// with four key tiles per 256 rows a launch spends 7 of 20 us per tile of rows on starting a workgroup, waiting for its
+// queries and first keys, and storing.  The last key tile's step requests the first keys of the next rows, the next
+// queries are pulled into the L2 meanwhile and requested before the output leaves.  40 heads, 32760 queries, before -> now:
+// 400 keys 384 -> 353, 512 keys 383 -> 362, 768 keys 496 -> 482 us, 1024 keys 614 -> 615; with a key mask 512 keys 414 -> 390.
+// What is left above the 12 us of the products: reading q and writing out, which all CUs do at the same moments.
+template <int DT, bool KEYMASK>
+__global__ __launch_bounds__(512, 1) void fa16_loop_kernel(const FaParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
+  const int total = p.B * p.N * ((p.Sq + 255) / 256), per_xcd = (total + 7) / 8;
+  const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int end = min(total, (x + 1) * per_xcd);
+  if (x * per_xcd + j >= end) return;
+  fa16_flex_body<DT, 8, 128, 1, KEYMASK>(p, (MSD_LDS char*)smem_raw, x * per_xcd + j, 0, end);
+#endif
+}
+template <int DT, bool KEYMASK>
+static int launch_fa16_loop(const FaParams& p, hipStream_t stream) {
+  auto kern = fa16_loop_kernel<DT, KEYMASK>;
+  constexpr int kLds = 160 * 1024;  // two K and two V stages of 128 keys, 4 KiB of output staging per wave
+  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+    return MSD_ERR_LAUNCH;
+  hipLaunchKernelGGL(kern, dim3(256), dim3(512), kLds, stream, p);
+  return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
+}
+
 // MINDIESD_DENSE_TILE_ROWS = 256 or 128 in the environment (0: not set): dense and causal calls run as whole tiles of
 // 256 rows, or as workgroups of 128 rows on the 4-wave kernels (the tests reach each kind at every size that way).
 static int forced_tile_rows() {
@@ -1311,11 +1338,16 @@ static int forced_tile_rows() {
 // of a round of whole ones, two rounds of either more than one (20 tiles: 140 against 110 us at 5120 keys).
 // B x N 8, keys = queries, before -> now: 4 tiles per XCD 21 -> 15 us, 16 tiles 71 -> 62 us, 32 + 1 tiles 350 -> 278 us,
 // 32 + 16 tiles 538 -> 467 us, 64 + 8 tiles 1245 -> 1042 us; 46 * 32 + 8 tiles (40 heads, 75600) 85.2 -> 84.1 ms.
+constexpr int kLoopKv = 768;  // keys up to which workgroups keep their CU (fa16_loop_kernel)
 template <int DT, int GEN>
 static int launch_fa16_rounds(FaParams p, hipStream_t stream) {
   const long long per_xcd = ((long long)p.B * p.N * ((p.Sq + 255) / 256) + 7) / 8;
   constexpr int kCusPerXcd = 32;
   const int rest = (int)(per_xcd % kCusPerXcd);
+  // few keys: the workgroups that keep their CU, when there are rounds enough that cutting the last one matters less
+  if (p.Skv <= kLoopKv && per_xcd >= 2 * kCusPerXcd && (rest == 0 || 2 * rest > kCusPerXcd || per_xcd >= 8 * kCusPerXcd) &&
+      per_xcd < (1 << 27) && forced_tile_rows() != 256)
+    return launch_fa16_loop<DT, GEN == 3>(p, stream);
   if (rest == 0 || 2 * rest > kCusPerXcd || forced_tile_rows() == 256)
     return launch_fa16<DT, 8, false, false, GEN>(p, stream);
   p.tail_full = (int)(per_xcd - rest);

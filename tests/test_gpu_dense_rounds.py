@@ -1,5 +1,5 @@
 """Dense attention at head_dim 128 where the last round of workgroups is cut into half or quarter tiles
-(launch_fa16_rounds): whole rounds before it or none, tiles per XCD at the edges of the rule, ragged query and key
+(launch_fa16_rounds) or, over a few key tiles, workgroups keep their CU (fa16_loop_kernel): whole rounds before it or none, tiles per XCD at the edges of the rule, ragged query and key
 lengths around the 64-, 128- and 256-row and the 128-key tiles, both layouts and types, and the key-padding mask.
 
 Bounds against the float64 softmax of the same 16-bit operands: the query is rounded to 16 bits after scaling and a
@@ -22,7 +22,7 @@ def reference(q, k, v, mask=None):
             if mask is not None:
                 s = s.masked_fill(~mask[b].view(1, -1), float("-inf"))
             out.append(torch.softmax(s, -1) @ v[b, n].double())
-    return torch.stack(out).view(q.shape)
+    return torch.stack(out).reshape(q.shape)
 
 
 def check(got, want, v, dtype):
@@ -30,6 +30,25 @@ def check(got, want, v, dtype):
     assert torch.isfinite(got).all()
     assert (err.norm() / want.norm()).item() <= 3 * U[dtype]
     assert err.abs().max().item() <= 16 * U[dtype] * v.abs().max().item()
+
+
+# (batch, heads, q_len, kv_len), 2 to 9 rounds: even and odd numbers of key tiles, ragged rows, heads that change inside
+# a workgroup's run, and the last key count of the rule
+LOOP_CASES = [(1, 40, 4200, 385), (2, 20, 3328, 513), (1, 264, 600, 640), (3, 11, 8200, 767), (1, 536, 256, 768), (1, 523, 257, 500)]
+
+
+@pytest.mark.parametrize("batch,heads,q_len,kv_len", LOOP_CASES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("masked", [False, True])
+def test_rows_in_a_loop(batch, heads, q_len, kv_len, dtype, masked):
+    print("case", batch, heads, q_len, kv_len, dtype, masked, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(heads + q_len)
+    q, k, v = (torch.randn((batch, s, heads, 128), generator=g, device="cuda").to(dtype) for s in (q_len, kv_len, kv_len))
+    mask = torch.rand((batch, kv_len), generator=g, device="cuda") < 0.5 if masked else None
+    m4 = None if mask is None else mask.view(batch, 1, 1, kv_len)
+    want = reference(*(x.transpose(1, 2) for x in (q, k, v)), mask)
+    got = mindiesd.attention_forward(q, k, v, attn_mask=m4, head_first=False)
+    check(got.transpose(1, 2), want, v, dtype)
 
 
 # heads x ceil(q_len / 256) tiles over 8 XCDs: tiles per XCD 1, 1, 8, 9, 16, 17 (no round before the last),
