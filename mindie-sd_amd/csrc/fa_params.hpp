@@ -81,6 +81,26 @@ __device__ __forceinline__ bool packed_find_tile(const int* seq_meta, int nseq, 
   return false;
 }
 
+// The same numbering with the sequences taken by descending key count (ties by index) instead of in their order; at most
+// 64 sequences, one per lane.
+__device__ __forceinline__ bool packed_find_tile_longest_first(const int* seq_meta, int nseq, int i, int& seq, int& tile,
+                                                               int rows) {
+  const int lane = threadIdx.x & 63;
+  const int t = lane < nseq ? (seq_meta[4 * lane + 1] + rows - 1) / rows : 0;
+  const int keys = lane < nseq ? seq_meta[4 * lane + 3] : -1;
+  int first = 0;  // tiles of the sequences before the lane's
+  for (int j = 0; j < nseq; ++j) {
+    const int tj = __builtin_amdgcn_readlane(t, j), kj = __builtin_amdgcn_readlane(keys, j);
+    if (kj > keys || (kj == keys && j < lane)) first += tj;
+  }
+  const unsigned long long hit = __ballot(t > 0 && i >= first && i < first + t);
+  if (hit == 0) return false;
+  const int l = __ffsll((long long)hit) - 1;  // exactly one lane holds tile i
+  seq = l;
+  tile = i - __builtin_amdgcn_readlane(first, l);
+  return true;
+}
+
 // True when the query counts of the table differ enough (the longest more than 1.25 times the mean of the non-empty
 // ones) that equal numbers of consecutive tiles per XCD would be unequal work; wave-uniform, the same in every wave.
 // `tiles`: the number of query tiles of `rows` rows that the sequences have together.
@@ -118,34 +138,45 @@ __device__ __forceinline__ bool fa16_find_work(const FaParams& p, int rows, int&
   constexpr bool packed = GEN == 2;
   int q_tiles = PAIR ? p.NP : packed ? p.packed_tiles : (p.Sq + rows - 1) / rows;
   // Sequences of unequal length (general mode with a table): workgroups are dealt to the XCDs one by one instead of in
-  // runs - tiles in descending order, the (batch, head) index fastest - so every XCD gets its share of the long ones.
-  bool spread = false;
+  // runs, so every XCD gets its share of the long ones.  A causal tile's work is its index: tiles in descending order, the
+  // (batch, head) index fastest.  Otherwise it is the sequence's key count: the longest sequence's tiles first, the head
+  // fastest, so that the launch ends on short ones (24 heads, 7 sequences of 16380 tokens together: in descending tile
+  // order, which leaves the first tile of the longest sequence to the end, 576 us, now 523; beyond 64 sequences as before).
+  bool spread = false, longest_first = false;
   if constexpr (GEN == 1 || GEN == 2) {
     if (p.seq_meta) {
       int real_tiles;
       spread = seqs_uneven(p.seq_meta, p.B, rows, real_tiles);
       // packed numbering: the grid is sized for an upper bound; the tiles that exist are what is dealt out
       if (packed) q_tiles = min(q_tiles, real_tiles);
+      longest_first = spread && !p.causal && p.B <= 64;
     }
   }
   // (fa16_work.hpp: runs of consecutive tiles per XCD; units of a heavy and a light tile - causal: tile t of a head has
   // t + 1 tiles' worth of keys, PAIR: the pairs of a head are numbered by descending length of their lists - so that
   // 12 heads on 8 XCDs are not 1.75 against 1.25 heads' worth of work; or one by one)
   const int groups = (packed ? 1 : p.B) * p.N;
-  const fa16::Work w = spread ? fa16::spread(blockIdx.x, groups, q_tiles, packed)
-                       : (PAIR || (GEN == 1 && p.causal)) ? fa16::units(blockIdx.x, groups, q_tiles, PAIR)
-                                                           : fa16::runs(blockIdx.x, groups, q_tiles);
-  if (w.group < 0) return false;
-  bn = w.group;
-  qt = w.tile;
-  if constexpr (packed) {  // bn is the head; the tile's sequence comes from the table
-    n = bn;
-    if (!packed_find_tile(p.seq_meta, p.B, qt, b, qt, rows)) return false;
-    if (p.causal) qt = (p.seq_meta[4 * b + 1] + rows - 1) / rows - 1 - qt;
+  if (longest_first) {
+    const int u = blockIdx.x / p.N;
+    n = blockIdx.x - u * p.N;
+    if (!packed_find_tile_longest_first(p.seq_meta, p.B, u, b, qt, rows)) return false;
     bn = b * p.N + n;
   } else {
-    b = bn / p.N;
-    n = bn - b * p.N;
+    const fa16::Work w = spread ? fa16::spread(blockIdx.x, groups, q_tiles, packed)
+                         : (PAIR || (GEN == 1 && p.causal)) ? fa16::units(blockIdx.x, groups, q_tiles, PAIR)
+                                                             : fa16::runs(blockIdx.x, groups, q_tiles);
+    if (w.group < 0) return false;
+    bn = w.group;
+    qt = w.tile;
+    if constexpr (packed) {  // bn is the head; the tile's sequence comes from the table
+      n = bn;
+      if (!packed_find_tile(p.seq_meta, p.B, qt, b, qt, rows)) return false;
+      if (p.causal) qt = (p.seq_meta[4 * b + 1] + rows - 1) / rows - 1 - qt;
+      bn = b * p.N + n;
+    } else {
+      b = bn / p.N;
+      n = bn - b * p.N;
+    }
   }
   Sq = p.Sq;
   Skv = p.Skv;
