@@ -20,6 +20,13 @@
 
 namespace msd {
 
+// LDS of a workgroup: the tile stages; the groups' hand-over and the output staging reuse them (KS 1: staging of its own)
+template <int D, int KS>
+constexpr int fa16_flex_lds(int nw, int bn) {
+  const int stages = 4 * bn * 2 * D, part = nw * ((D / 16 - D / 16 / KS) * 2048 + 1024) + nw * 32 * (2 * D / KS + 8);
+  return KS == 1 ? stages + nw * 4096 : stages > part ? stages : part;
+}
+
 #if defined(__HIP_DEVICE_COMPILE__)
 template <int... I, class F>
 __device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
@@ -36,12 +43,16 @@ __device__ __forceinline__ void static_for(F&& f) {
 // the tiles item + 32, item + 64, ... below `end`.
 // LDS: K stages at 0 and BN * 256 bytes, V stages behind them, with KS 1 the output staging behind those; swizzles and
 // operand layouts as in fa_fwd16_kernel.
-template <int DT, int NW, int BN, int KS, bool KEYMASK>
+//
+// D: head_dim, 128 or 64 (fa_fwd16_d64_kernel's layouts: rows of 128 bytes, K chunk p of row r at p ^ ((r >> 1) & 7), V
+// chunk p at p ^ ((r >> 1) & 3)).
+template <int DT, int NW, int BN, int KS, bool KEYMASK, int D = 128>
 __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* smem, int item, int part, int end) {
   using E = Elem<DT>;
   using T = typename E::type;
   using X8 = typename E::x8;
-  constexpr int kRowBytes = 256, kTileBytes = BN * kRowBytes;
+  static_assert(D == 128 || (D == 64 && KS > 1), "head_dim");
+  constexpr int kRowBytes = 2 * D, kDmaRows = 1024 / kRowBytes, NDB = D / 16, NKS = D / 32, kTileBytes = BN * kRowBytes;
   constexpr int RG = NW / KS;         // waves side by side over the query rows
   constexpr int kKeys = BN / KS;      // keys of a tile that one wave takes
   constexpr int NKB = kKeys / 16;     // its 16-key blocks
@@ -67,33 +78,34 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
 
   // ---- staging (LDS-DMA) -------------------------------------------------------------------------------------
   const int group = p.N / p.Nkv;
-  const int k_range = (int)(((long long)(Skv - 1) * p.k_ss + 128) * 2), v_range = (int)(((long long)(Skv - 1) * p.v_ss + 128) * 2);
+  const int k_range = (int)(((long long)(Skv - 1) * p.k_ss + D) * 2), v_range = (int)(((long long)(Skv - 1) * p.v_ss + D) * 2);
   auto k_base = [&](int ib, int in) __attribute__((always_inline)) { return (const T*)p.k + ib * p.k_sb + (in / group) * p.k_sn; };
   auto v_base = [&](int ib, int in) __attribute__((always_inline)) { return (const T*)p.v + ib * p.v_sb + (in / group) * p.v_sn; };
   const T *kg = k_base(b, n), *vg = v_base(b, n), *kg_nx = kg, *vg_nx = vg;
   const int k_row_bytes = (int)p.k_ss * 2, v_row_bytes = (int)p.v_ss * 2;
   int k_voff, v_voff;
   {
-    const int row = 4 * wave + (lane >> 4);  // groups of one wave lie 4 * NW rows apart: same swizzles
-    const int pc = lane & 15;
-    k_voff = row * k_row_bytes + ((pc ^ (row & 15)) << 4);
-    v_voff = row * v_row_bytes + (((((pc >> 1) ^ (row & 7)) << 1) | (pc & 1)) << 4);
+    const int row = kDmaRows * wave + lane / (kRowBytes / 16);  // groups of one wave lie kDmaRows * NW rows apart: same swizzles
+    const int pc = lane % (kRowBytes / 16);
+    const int ksw = D == 128 ? row & 15 : (row >> 1) & 7, vsw = D == 128 ? row & 7 : (row >> 1) & 3;
+    k_voff = row * k_row_bytes + ((pc ^ ksw) << 4);
+    v_voff = row * v_row_bytes + (((((pc >> 1) ^ vsw) << 1) | (pc & 1)) << 4);
   }
   auto load_tile = [&](const T* kp, const T* vp, int key0, int stage) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, k_range, 0x00020000);
     const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, v_range, 0x00020000);
 #pragma unroll
-    for (int i = 0; i < BN / 4 / NW; ++i) {
+    for (int i = 0; i < BN / kDmaRows / NW; ++i) {
       const int grp = i * NW + wave;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rsrc, (MSD_LDS void*)(smem + stage * kTileBytes + grp * 1024), 16, k_voff,
-                                               (key0 + i * 4 * NW) * k_row_bytes, 0, 0);
+                                               (key0 + i * kDmaRows * NW) * k_row_bytes, 0, 0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rsrc, (MSD_LDS void*)(smem + (2 + stage) * kTileBytes + grp * 1024), 16,
-                                               v_voff, (key0 + i * 4 * NW) * v_row_bytes, 0, 0);
+                                               v_voff, (key0 + i * kDmaRows * NW) * v_row_bytes, 0, 0);
     }
   };
 
   // ---- Q^T operand, resident: requested here, converted at the start of its tile ------------------------------------
-  X8 qf[2][4];
+  X8 qf[2][NKS];
   auto load_q = [&](int ib, int in, int irow) __attribute__((always_inline)) {
     const T* qg = (const T*)p.q + ib * p.q_sb + in * p.q_sn;
     int c = lane & 15, g = lane >> 4;
@@ -103,24 +115,24 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
       const int qrow = irow + nq * 16 + c;
       const T* src = qg + (long long)(qrow < Sq ? qrow : 0) * p.q_ss + 8 * g;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) qf[nq][ks] = *(const X8*)(src + 32 * ks);
+      for (int ks = 0; ks < NKS; ++ks) qf[nq][ks] = *(const X8*)(src + 32 * ks);
     }
   };
-  f32x4_t oacc[8][2], negm[2], lt[2];
+  f32x4_t oacc[NDB][2], negm[2], lt[2];
   float l_run[2];
   X8 ones;
 #pragma unroll
   for (int j = 0; j < 8; ++j) ones[j] = E::from_float(1.f);
 
   // per-lane parts of the LDS read addresses (the wave's keys start at row kg_i * kKeys, a multiple of 16)
-  unsigned k_lds[4], v_lds[4];
+  unsigned k_lds[NKS], v_lds[4];
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-    k_lds[ks] = (unsigned)(uintptr_t)smem + (kg_i * kKeys + c) * kRowBytes + (((4 * ks + g) ^ c) << 4);
+  for (int ks = 0; ks < NKS; ++ks)
+    k_lds[ks] = (unsigned)(uintptr_t)smem + (kg_i * kKeys + c) * kRowBytes + (((4 * ks + g) ^ (D == 128 ? c : c >> 1)) << 4);
 #pragma unroll
   for (int db = 0; db < 4; ++db)
     v_lds[db] = (unsigned)(uintptr_t)smem + 2 * kTileBytes + (kg_i * kKeys + 4 * g + (c >> 2)) * kRowBytes +
-                ((db ^ (4 * (g & 1) + (c >> 2))) << 5) + 8 * (c & 3);
+                ((db ^ (D == 128 ? 4 * (g & 1) + (c >> 2) : ((4 * g + (c >> 2)) >> 1) & 3)) << 5) + 8 * (c & 3);
 
   const int tiles = (Skv + BN - 1) / BN;
   load_q(b, n, row0);
@@ -166,7 +178,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
 
     // S^T = K Q^T: operand groups of 2 key blocks of one 32-wide head_dim step, kAhead groups ahead of their use
     f32x4_t sacc[NKB][2];
-    constexpr int kPer = NKB / 2, kGroups = 4 * kPer, kAhead = 3;
+    constexpr int kPer = NKB / 2, kGroups = NKS * kPer, kAhead = kGroups > 3 ? 3 : kGroups - 1;
     X8 afrag[kAhead + 1][2];
     auto k_read = [&](auto gi_c, X8(&dst)[2]) __attribute__((always_inline)) {
       constexpr int gi = decltype(gi_c)::value, ks = gi / kPer, qu = gi % kPer;
@@ -260,7 +272,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
 #pragma unroll
           for (int i = 0; i < 4; ++i) sacc[kb][nq][i] -= delta;
 #pragma unroll
-        for (int db = 0; db < 8; ++db)
+        for (int db = 0; db < NDB; ++db)
 #pragma unroll
           for (int i = 0; i < 4; ++i) oacc[db][nq][i] *= alpha;
       }
@@ -276,10 +288,11 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
       }
     }
 
+    constexpr int NH = NDB / 4;  // steps per 32 keys
     // O^T += V^T P^T: steps of (32 keys) x (4 head_dim blocks), V^T fragments requested one step ahead
     s16x4_t vf[2][8];
     auto issue = [&](auto step_c, s16x4_t(&dst)[8]) __attribute__((always_inline)) {
-      constexpr int s = decltype(step_c)::value, j = s >> 1, dbh = s & 1;
+      constexpr int s = decltype(step_c)::value, j = s / NH, dbh = s % NH;
       constexpr int off = stage * kTileBytes + 32 * j * kRowBytes;
 #pragma unroll
       for (int d4 = 0; d4 < 4; ++d4) {
@@ -292,9 +305,9 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
       if (next_key0 >= 0) mask_request(next_key0);  // lands during the second product
     }
     issue(std::integral_constant<int, 0>{}, vf[0]);
-    static_for<2 * NJ>([&](auto step_c) __attribute__((always_inline)) {
-      constexpr int s = decltype(step_c)::value, j = s >> 1, dbh = s & 1;
-      if constexpr (s + 1 < 2 * NJ) {
+    static_for<NH * NJ>([&](auto step_c) __attribute__((always_inline)) {
+      constexpr int s = decltype(step_c)::value, j = s / NH, dbh = s % NH;
+      if constexpr (s + 1 < NH * NJ) {
         issue(std::integral_constant<int, s + 1>{}, vf[(s + 1) & 1]);
         lds_wait_tr<8>(vf[s & 1]);
       } else {
@@ -331,7 +344,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     if constexpr (LOOP) asm volatile("" : "+v"(cc));
     const bool ok = row0 + nq * 16 + cc < Sq;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
+    for (int ks = 0; ks < NKS; ++ks) {
       X8 v = qf[nq][ks];
       if (!ok) v = X8{0};
 #pragma unroll
@@ -341,7 +354,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     l_run[nq] = 0.f;
     negm[nq] = lt[nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int db = 0; db < 8; ++db) oacc[db][nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < NDB; ++db) oacc[db][nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
   first = true;
   bool more = false;
@@ -373,15 +386,15 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   }
 
   // ---- the groups' partial results (KS > 1) --------------------------------------------------------------------------
-  // Every wave ends up with all 32 rows of its row group and 8 / KS of the output's 16-wide blocks: it hands the other
+  // Every wave ends up with all 32 rows of its row group and NDB / KS of the output's 16-wide blocks: it hands the other
   // blocks to the waves that own them (16 bytes per lane and block, the accumulator layout as it is) together with its
   // reference maxima and sums.  A group that saw no key has sum 0 and no say in the maximum.
-  constexpr int DB = 8 / KS;                       // output blocks a wave stores
-  constexpr int kPart = (8 - DB) * 2 * 1024;       // bytes a wave hands out
+  constexpr int DB = NDB / KS;                       // output blocks a wave stores
+  constexpr int kPart = (NDB - DB) * 2 * 1024;       // bytes a wave hands out
   constexpr int kStat = KS > 1 ? 4 * 256 : 0;      // m and l of two column blocks, a dword per lane
   constexpr int kORow = 2 * 16 * DB + 8;           // a row of the output staging, padded
   constexpr int kOBase = KS > 1 ? NW * (kPart + kStat) : 0;
-  static_assert(KS == 1 || kOBase + NW * 32 * kORow <= 4 * BN * 256, "fits the tile stages");
+  static_assert(KS == 1 || kOBase + NW * 32 * kORow <= fa16_flex_lds<D, KS>(NW, BN), "fits");
   float l_tot[2], m_tot[2];
 #pragma unroll
   for (int nq = 0; nq < 2; ++nq) {
@@ -392,7 +405,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     MSD_LDS char* mine = smem + wave * (kPart + kStat);
     // block db belongs to group db / DB; slot of a block that is not the writer's: the blocks in order, its own left out
 #pragma unroll
-    for (int db = 0; db < 8; ++db) {
+    for (int db = 0; db < NDB; ++db) {
       const int owner = db / DB;
       const int slot = owner < kg_i ? db : db - DB;
       if (owner != kg_i) {

@@ -28,22 +28,13 @@
 #include <utility>
 
 #include "common.hpp"
+#include "fa16_flex.hpp"
 #include "fa_params.hpp"
 
 namespace msd {
 
 #if defined(__HIP_DEVICE_COMPILE__)
 namespace d64 {
-template <int... I, class F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>)
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
-}
-
 // Rescale of one 16-query column block when its reference maximum moves: l *= alpha, the seed and the 8 score blocks
 // -= delta, the 4 output blocks *= alpha - 53 registers updated in place by asm blocks that skip themselves when the
 // wave-uniform flag is zero (the same construction as cond_rescale_fa16 in common.hpp, which explains why the test
@@ -127,7 +118,8 @@ constexpr int kD64Ahead = 3;                          // K operand groups reques
 // the buffers' range (the DMA writes zeros for them without touching memory), output columns past it are not stored.
 // NW: waves per workgroup, 32 query rows each - 8 (one workgroup per CU), or 4 (two per CU: for grids that fill the
 // chip badly as 256-row workgroups).
-template <int DT, int GEN = 0, bool DPAD = false, int NW = kD64Waves>
+// TAIL as in fa_fwd16_kernel: the tiles of the last round in 2 or 4 parts.
+template <int DT, int GEN = 0, bool DPAD = false, int NW = kD64Waves, int TAIL = 0>
 __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void fa_fwd16_d64_kernel(const FaParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using namespace d64;
@@ -150,7 +142,25 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void fa_fwd16_d64_kernel(
   const int hd = DPAD ? p.head_dim : 64;
   int bn, qt, b, n, Sq, Skv;
   long long q_tok0, k_tok0;  // general mode: first token of the sequence in packed tensors
-  if (!fa16_find_work<GEN, false>(p, kBM, bn, qt, b, n, Sq, Skv, q_tok0, k_tok0)) return;
+  if constexpr (TAIL != 0) {
+    static_assert((GEN == 0 || GEN == 3) && !DPAD && NW == 8, "dense, with or without a key mask");
+    const fa16::Part w = fa16::runs_tail(blockIdx.x, p.B * p.N, (p.Sq + kBM - 1) / kBM, p.tail_full, TAIL);
+    if (w.group < 0) return;
+    if (w.part >= 0) {
+      if (w.tile * kBM + w.part * (kBM / TAIL) < p.Sq)
+        fa16_flex_body<DT, 8, BN, TAIL, GEN == 3, 64>(p, smem, w.group * ((p.Sq + kBM - 1) / kBM) + w.tile, w.part, 0);
+      return;
+    }
+    bn = w.group;
+    qt = w.tile;
+    b = bn / p.N;
+    n = bn - b * p.N;
+    Sq = p.Sq;
+    Skv = p.Skv;
+    q_tok0 = k_tok0 = 0;
+  } else {
+    if (!fa16_find_work<GEN, false>(p, kBM, bn, qt, b, n, Sq, Skv, q_tok0, k_tok0)) return;
+  }
   const int nkv = n / (p.N / p.Nkv);
   const int row0 = qt * kBM + wave * 32;  // first query row of this wave
 
@@ -491,14 +501,16 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void fa_fwd16_d64_kernel(
 }
 
 
-template <int DT, int GEN, bool DPAD = false, int NW = kD64Waves>
+template <int DT, int GEN, bool DPAD = false, int NW = kD64Waves, int TAIL = 0>
 static int launch_d64(const FaParams& p, hipStream_t stream) {
-  auto kern = fa_fwd16_d64_kernel<DT, GEN, DPAD, NW>;
-  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kD64Lds) != hipSuccess)
+  auto kern = fa_fwd16_d64_kernel<DT, GEN, DPAD, NW, TAIL>;
+  constexpr int kLds = TAIL ? fa16_flex_lds<64, TAIL ? TAIL : 2>(8, kD64BN) : kD64Lds;
+  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
     return MSD_ERR_LAUNCH;
-  const long long grid = fa16_grid<GEN, false>(p, NW * 32);
+  const long long grid = TAIL ? fa16::runs_tail_grid((long long)p.B * p.N, (p.Sq + 255) / 256, p.tail_full, TAIL)
+                              : fa16_grid<GEN, false>(p, NW * 32);
   if (grid > 0x7ffffff0ll) return MSD_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), kD64Lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), kLds, stream, p);
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
 }
 
@@ -524,9 +536,19 @@ int launch_fa16_d64_padded(const FaParams& p, int dtype, int D, hipStream_t stre
   }
 }
 
-int launch_fa16_d64(const FaParams& p, int dtype, hipStream_t stream, int gen, int rows) {
+template <int GEN>
+static int launch_d64_tail(FaParams p, int dtype, hipStream_t stream, int split) {
+  const bool bf = dtype == MSD_DTYPE_BF16;
+  if (split == 2)
+    return bf ? launch_d64<MSD_DTYPE_BF16, GEN, false, 8, 2>(p, stream) : launch_d64<MSD_DTYPE_F16, GEN, false, 8, 2>(p, stream);
+  return bf ? launch_d64<MSD_DTYPE_BF16, GEN, false, 8, 4>(p, stream) : launch_d64<MSD_DTYPE_F16, GEN, false, 8, 4>(p, stream);
+}
+
+int launch_fa16_d64(const FaParams& p, int dtype, hipStream_t stream, int gen, int rows, int split) {
   if (!fa16_d64_supported(p) || gen < 0 || gen > 3) return MSD_ERR_UNSUPPORTED;
   if (rows != 256 && !(rows == 128 && gen == 0)) return MSD_ERR_UNSUPPORTED;
+  if (split != 0 && (gen == 0 || gen == 3))
+    return gen == 3 ? launch_d64_tail<3>(p, dtype, stream, split) : launch_d64_tail<0>(p, dtype, stream, split);
   const bool bf = dtype == MSD_DTYPE_BF16;
   if (rows == 128)
     return bf ? launch_d64<MSD_DTYPE_BF16, 0, false, 4>(p, stream) : launch_d64<MSD_DTYPE_F16, 0, false, 4>(p, stream);

@@ -1317,7 +1317,7 @@ __global__ __launch_bounds__(512, 1) void fa16_loop_kernel(const FaParams p) {
 template <int DT, bool KEYMASK>
 static int launch_fa16_loop(const FaParams& p, hipStream_t stream) {
   auto kern = fa16_loop_kernel<DT, KEYMASK>;
-  constexpr int kLds = 160 * 1024;  // two K and two V stages of 128 keys, 4 KiB of output staging per wave
+  constexpr int kLds = fa16_flex_lds<128, 1>(8, 128);
   if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
     return MSD_ERR_LAUNCH;
   hipLaunchKernelGGL(kern, dim3(256), dim3(512), kLds, stream, p);
@@ -1332,27 +1332,35 @@ static int forced_tile_rows() {
   return n == 128 || n == 256 ? n : 0;
 }
 
-// Plain dense attention (GEN 0) or with a key mask (GEN 3): how the last round of workgroups is cut.  An XCD runs its
-// share of the 256-row tiles in rounds of 32; when the last round has at most 8 or 16 tiles, they go as four or two
+// Plain dense attention or with a key mask, head dims 128 and 64: how the last round of workgroups is cut.  An XCD runs
+// its share of the 256-row tiles in rounds of 32; when the last round has at most 8 or 16 tiles, they go as four or two
 // workgroups each (fa16_flex.hpp), which still is one round: a round of quarter tiles takes 0.46, one of half tiles 0.62
 // of a round of whole ones, two rounds of either more than one (20 tiles: 140 against 110 us at 5120 keys).
-// B x N 8, keys = queries, before -> now: 4 tiles per XCD 21 -> 15 us, 16 tiles 71 -> 62 us, 32 + 1 tiles 350 -> 278 us,
-// 32 + 16 tiles 538 -> 467 us, 64 + 8 tiles 1245 -> 1042 us; 46 * 32 + 8 tiles (40 heads, 75600) 85.2 -> 84.1 ms.
+// B x N 8, keys = queries, before -> now, head_dim 128: 4 tiles per XCD 21 -> 15 us, 16 tiles 71 -> 62 us, 32 + 1 tiles
+// 350 -> 278 us, 32 + 16 tiles 538 -> 467 us, 64 + 8 tiles 1245 -> 1042 us; 46 * 32 + 8 tiles (40 heads, 75600) 85.2 -> 84.1
+// ms.  Head_dim 64: 8 tiles 24 -> 16 us, 16 tiles 45 -> 40, 32 + 8 tiles 251 -> 213, 64 + 4 tiles 749 -> 614 us, 13 * 32 + 4
+// tiles (48 heads, 17776) 3.74 -> 3.60 ms.
+// Returns the number of parts (0: no cut) and sets p.tail_full.
+static int fa16_split(FaParams& p) {
+  constexpr int kCusPerXcd = 32;
+  const long long per_xcd = ((long long)p.B * p.N * ((p.Sq + 255) / 256) + 7) / 8;
+  const int rest = (int)(per_xcd % kCusPerXcd);
+  if (rest == 0 || 2 * rest > kCusPerXcd || forced_tile_rows() != 0 || per_xcd >= (1 << 27)) return 0;
+  p.tail_full = (int)(per_xcd - rest);
+  return 4 * rest > kCusPerXcd ? 2 : 4;
+}
+
 constexpr int kLoopKv = 768;  // keys up to which workgroups keep their CU (fa16_loop_kernel)
 template <int DT, int GEN>
 static int launch_fa16_rounds(FaParams p, hipStream_t stream) {
   const long long per_xcd = ((long long)p.B * p.N * ((p.Sq + 255) / 256) + 7) / 8;
-  constexpr int kCusPerXcd = 32;
-  const int rest = (int)(per_xcd % kCusPerXcd);
+  const int split = fa16_split(p);
   // few keys: the workgroups that keep their CU, when there are rounds enough that cutting the last one matters less
-  if (p.Skv <= kLoopKv && per_xcd >= 2 * kCusPerXcd && (rest == 0 || 2 * rest > kCusPerXcd || per_xcd >= 8 * kCusPerXcd) &&
-      per_xcd < (1 << 27) && forced_tile_rows() != 256)
+  if (p.Skv <= kLoopKv && per_xcd >= 64 && (split == 0 || per_xcd >= 256) && per_xcd < (1 << 27) && forced_tile_rows() == 0)
     return launch_fa16_loop<DT, GEN == 3>(p, stream);
-  if (rest == 0 || 2 * rest > kCusPerXcd || forced_tile_rows() == 256)
-    return launch_fa16<DT, 8, false, false, GEN>(p, stream);
-  p.tail_full = (int)(per_xcd - rest);
-  if (4 * rest > kCusPerXcd) return launch_fa16<DT, 8, false, false, GEN, false, 2>(p, stream);
-  return launch_fa16<DT, 8, false, false, GEN, false, 4>(p, stream);
+  if (split == 2) return launch_fa16<DT, 8, false, false, GEN, false, 2>(p, stream);
+  if (split == 4) return launch_fa16<DT, 8, false, false, GEN, false, 4>(p, stream);
+  return launch_fa16<DT, 8, false, false, GEN>(p, stream);
 }
 
 template <int DT, int NWAVES, int QPW, int BN, bool SPARSE, int SCHED, int MODE = 0, bool GATHER = false,
@@ -1531,8 +1539,8 @@ int mindiesd_block_sparse_attention_paired_fwd(const void* q, const void* k, con
 }
 
 // True when B x N x ceil(Sq / 256) workgroups of 256 rows would fill the 256 CUs badly - at most half of them busy, or
-// a second round for at most half of them - for the calls whose rounds launch_fa16_rounds does not cut: head dims up to
-// 64 and causal ones.  They run as 128-row workgroups of four waves, two to a CU.
+// a second round for at most half of them - for the calls whose last round fa16_split does not cut: head dims below 64,
+// causal ones, and some at head_dim 64.  They run as 128-row workgroups of four waves, two to a CU.
 static bool prefers_half_tiles(int B, int N, int Sq) {
   const long long tiles256 = (long long)B * N * ((Sq + 255) / 256);
   bool half_tiles = 2 * tiles256 <= kCus || (tiles256 > kCus && 2 * tiles256 <= 3 * kCus);
@@ -1550,7 +1558,13 @@ int mindiesd_flash_attention_fwd(const void* q, const void* k, const void* v, vo
   if (rc != MSD_OK) return rc;
   FaParams p = make_params(q, k, v, out, lse, B, N, Nkv, Sq, Skv, st, scale);
   const bool half_tiles = prefers_half_tiles(B, N, Sq);
-  if (D == 64 && fa16_d64_supported(p)) return launch_fa16_d64(p, dtype, stream, 0, half_tiles ? 128 : 256);
+  if (D == 64 && fa16_d64_supported(p)) {
+    // (one round and a half of tiles over few keys: the 4-wave workgroups, 19.5 against 21.4 us at 512 keys, B x N 8,
+    // S 12288; the cut round gains 1.25 us per 1024 keys on them and is ahead from 2048 keys on, 295 against 308 us at 12288)
+    int split = fa16_split(p);
+    if (split == 2 && half_tiles && p.tail_full > 0 && Skv < 2048) split = 0;
+    return launch_fa16_d64(p, dtype, stream, 0, half_tiles ? 128 : 256, split);
+  }
   // Head dims between 64 and 128 run as head_dim 128 on the 16x16x32 kernel (the part of the matrix work spent on
   // the padding costs less than the general kernel's staging through registers: 72 -> 580 vs 730 TFLOP/s of real
   // work, 112 -> 800 vs 1130), when the 256-byte rows the DMA fetches stay inside the kernel's 32-bit offsets.
@@ -1651,7 +1665,7 @@ int mindiesd_flash_attention_general_fwd(const void* q, const void* k, const voi
   const bool long_rows = Sq >= kGen16MinRows && (D != 128 || Skv > kShortKv);
   if (long_rows && (!mask || key_mask)) {  // head dims up to 128 on the 16x16x32 kernels, padded where need be
     const int gen = key_mask ? 3 : 1;
-    if (D == 64 && fa16_d64_supported(p)) return launch_fa16_d64(p, dtype, stream, gen);
+    if (D == 64 && fa16_d64_supported(p)) return launch_fa16_d64(p, dtype, stream, gen, 256, key_mask ? fa16_split(p) : 0);
     if (D < 64 && fa16_d64_supported(p)) return launch_fa16_d64_padded(p, dtype, D, stream, gen);
     if (D > 64 && D < 128 && (long long)Skv * k_ss * 2 < 0x7fffff00ll && (long long)Skv * v_ss * 2 < 0x7fffff00ll) {
       p.head_dim = D;

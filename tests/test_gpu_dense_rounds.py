@@ -1,5 +1,5 @@
-"""Dense attention at head_dim 128 where the last round of workgroups is cut into half or quarter tiles
-(launch_fa16_rounds) or, over a few key tiles, workgroups keep their CU (fa16_loop_kernel): whole rounds before it or none, tiles per XCD at the edges of the rule, ragged query and key
+"""Dense attention at head dims 128 and 64 where the last round of workgroups is cut into half or quarter tiles
+(fa16_split) or, over a few key tiles, workgroups keep their CU (fa16_loop_kernel): whole rounds before it or none, tiles per XCD at the edges of the rule, ragged query and key
 lengths around the 64-, 128- and 256-row and the 128-key tiles, both layouts and types, and the key-padding mask.
 
 Bounds against the float64 softmax of the same 16-bit operands: the query is rounded to 16 bits after scaling and a
@@ -53,19 +53,20 @@ def test_rows_in_a_loop(batch, heads, q_len, kv_len, dtype, masked):
 
 # heads x ceil(q_len / 256) tiles over 8 XCDs: tiles per XCD 1, 1, 8, 9, 16, 17 (no round before the last),
 # 32 + 1, 32 + 8, 32 + 9, 32 + 16, 64 + 3
-CASES = [(1, 1, 385), (3, 257, 512), (64, 129, 1000), (72, 200, 513), (43, 700, 641), (136, 256, 400),
+CASES = [(1, 1, 385), (3, 257, 512), (64, 129, 1000), (72, 200, 513), (43, 700, 641), (136, 256, 400), (8, 2300, 2100), (264, 300, 2050),
          (264, 193, 400), (160, 300, 577), (164, 511, 390), (128, 641, 700), (536, 65, 450)]
 
 
 @pytest.mark.parametrize("heads,q_len,kv_len", CASES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("masked", [False, True])
-def test_cut_rounds(heads, q_len, kv_len, dtype, masked):
+@pytest.mark.parametrize("d", [128, 64])
+def test_cut_rounds(heads, q_len, kv_len, dtype, masked, d):
     if masked and q_len < 256:
         q_len += 256                      # key masks run on this kernel from 256 query rows on
-    print("case", heads, q_len, kv_len, dtype, masked, flush=True)
+    print("case", heads, q_len, kv_len, dtype, masked, d, flush=True)
     g = torch.Generator(device="cuda").manual_seed(heads + q_len)
-    q, k, v = (torch.randn((1, heads, s, 128), generator=g, device="cuda").to(dtype) for s in (q_len, kv_len, kv_len))
+    q, k, v = (torch.randn((1, heads, s, d), generator=g, device="cuda").to(dtype) for s in (q_len, kv_len, kv_len))
     mask = None
     if masked:
         mask = torch.rand((1, kv_len), generator=g, device="cuda") < 0.5
@@ -79,11 +80,12 @@ def test_cut_rounds(heads, q_len, kv_len, dtype, masked):
     check(mindiesd.attention_forward(*t, attn_mask=m4, head_first=False).transpose(1, 2), want, v, dtype)
 
 
-def test_groups_of_very_different_maxima():
+@pytest.mark.parametrize("d", [128, 64])
+def test_groups_of_very_different_maxima(d):
     """The groups of waves that share a row keep reference maxima of their own: scores that differ by hundreds between
     the groups' keys, rows whose scores all lie far below zero, and a NaN and an infinity that stay in their rows."""
     g = torch.Generator(device="cuda").manual_seed(5)
-    q, k, v = (torch.randn((1, 4, s, 128), generator=g, device="cuda").bfloat16() for s in (512, 640, 640))
+    q, k, v = (torch.randn((1, 4, s, d), generator=g, device="cuda").bfloat16() for s in (512, 640, 640))
     q[:, :, :, 0] = 4.0
     k[:, :, :, 0] = torch.where(torch.arange(640, device="cuda") % 128 < 64, -900.0, -300.0).view(1, 1, -1).bfloat16()
     q[:, 1, :, 0] = -4.0
