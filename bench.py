@@ -196,7 +196,7 @@ def extra_head_dims(device, steps, warmup):
 
 def extra_mid_size_grids(device, steps, warmup):
     """Dense calls whose grid fills the 256 CUs badly as 256-row workgroups (few heads, a few thousand tokens): the
-    entry point runs them as 128-row workgroups; both choices timed (MINDIESD_DENSE_TILE_ROWS forces either)."""
+    entry point cuts their last round into smaller workgroups; timed beside whole tiles (MINDIESD_DENSE_TILE_ROWS)."""
     import os
     import torch
     import mindiesd
