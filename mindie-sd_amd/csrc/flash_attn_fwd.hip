@@ -1337,15 +1337,16 @@ static int forced_tile_rows() {
 // workgroups each (fa16_flex.hpp), which still is one round: a round of quarter tiles takes 0.46, one of half tiles 0.62
 // of a round of whole ones, two rounds of either more than one (20 tiles: 140 against 110 us at 5120 keys).
 // B x N 8, keys = queries, before -> now, head_dim 128: 4 tiles per XCD 21 -> 15 us, 16 tiles 71 -> 62 us, 32 + 1 tiles
-// 350 -> 278 us, 32 + 16 tiles 538 -> 467 us, 64 + 8 tiles 1245 -> 1042 us; 46 * 32 + 8 tiles (40 heads, 75600) 85.2 -> 84.1
-// ms.  Head_dim 64: 8 tiles 24 -> 16 us, 16 tiles 45 -> 40, 32 + 8 tiles 251 -> 213, 64 + 4 tiles 749 -> 614 us, 13 * 32 + 4
+// 350 -> 278 us, 32 + 16 tiles 538 -> 467 us, 64 + 8 tiles 1245 -> 1042 us.  From 16 whole rounds on the cut would gain 3 %
+// and less (46 rounds, 40 heads at 75600 tokens: 85.2 -> 84.1 ms) and is left out: there a call's bits do not depend on how
+// many problems its batch holds.  Head_dim 64: 8 tiles 24 -> 16 us, 16 tiles 45 -> 40, 32 + 8 tiles 251 -> 213, 64 + 4 tiles 749 -> 614 us, 13 * 32 + 4
 // tiles (48 heads, 17776) 3.74 -> 3.60 ms.
 // Returns the number of parts (0: no cut) and sets p.tail_full.
 static int fa16_split(FaParams& p) {
   constexpr int kCusPerXcd = 32;
   const long long per_xcd = ((long long)p.B * p.N * ((p.Sq + 255) / 256) + 7) / 8;
   const int rest = (int)(per_xcd % kCusPerXcd);
-  if (rest == 0 || 2 * rest > kCusPerXcd || forced_tile_rows() != 0 || per_xcd >= (1 << 27)) return 0;
+  if (rest == 0 || 2 * rest > kCusPerXcd || forced_tile_rows() != 0 || per_xcd >= 16 * kCusPerXcd) return 0;
   p.tail_full = (int)(per_xcd - rest);
   return 4 * rest > kCusPerXcd ? 2 : 4;
 }
