@@ -1,17 +1,19 @@
-// The body of fa_fwd16_kernel (flash_attn_fwd.hip: dense attention at head_dim 128 on the 16x16x32 matrix instruction)
-// in two other shapes of work.  NW waves of 32 rows each walk key tiles of BN keys.
+// The body of fa_fwd16_kernel and fa_fwd16_d64_kernel (dense attention at head_dim 128 and 64 on the 16x16x32 matrix
+// instruction) in two other shapes of work.  Eight waves walk key tiles of 128 keys as there, a wave owns NQ blocks of 16
+// query rows.  The arithmetic of a block of 16 rows - the chains of matrix instructions, when its reference maximum moves,
+// the rounding of its probabilities - is that of the kernels' whole tiles, so a row has the same bits in either.
 //
-// KS 1: a workgroup that keeps its CU and goes from one tile of rows to the next (fa16_loop_kernel states why).
+// LOOP (NQ 2): a workgroup that keeps its CU and goes from one tile of 256 rows to the next (fa16_loop_kernel states why).
 //
-// KS > 1: workgroups that own fewer query rows: the waves form KS groups that share the same NW / KS * 32 query rows, each
-// taking BN / KS keys of every tile with a running softmax of its own; the groups' sums and outputs are added up in LDS
-// at the end, in 32 bits.  Why: the launch time of fa_fwd16_kernel is rounds of 256 workgroups of 256 rows, and a round
-// that is a quarter full takes as long as a full one.  A workgroup of 128 (KS 2) or 64 rows (KS 4) has half or a quarter
-// of the matrix and vector work per tile for the same number of waves: its walk over the keys takes 0.62 or 0.46 of the
-// time (KS 4: 1.3 us per 128 keys, the L2 -> LDS stream of 64 KiB at 50 GB/s per CU; whole tiles: 3.0 us, matrix and
-// vector issue).  No workspace, no second launch.
+// Otherwise (NQ 1): a workgroup that owns part_rows (128 or 64) of a tile's 256 rows, 16 per wave; waves beyond them, or
+// beyond the last row, only stage keys.  Why: the launch time of the kernels is rounds of 256 workgroups of 256 rows, and a
+// round that is a quarter full takes as long as a full one.  What bounds it: every wave reads the whole key tile from LDS for
+// its 16 rows, 512 KiB per 128 keys and half tile (1.75 us at 128 bytes a cycle; it takes 1.96, a whole tile 3.15 us of matrix
+// and vector issue); a quarter tile takes 1.23 us, the L2 -> LDS stream of 64 KiB at 50 GB/s per CU.  (Head_dim 64: 1.15, 0.78 and
+// 1.91 us.)  Groups of waves that split the keys of 32 rows read less and take 1.82 and 1.16 us, but add a row up in another order
+// than the whole tiles of the same launch, so that equal problems of one batch came out with different bits.
 //
-// KEYMASK: a boolean mask row shared by all queries of a (batch, head), as GEN 3 of fa_fwd16_kernel.
+// KEYMASK: a boolean mask row shared by all queries of a (batch, head), as GEN 3 of the kernels.
 #pragma once
 #include <type_traits>
 #include <utility>
@@ -21,12 +23,8 @@
 
 namespace msd {
 
-// LDS of a workgroup: the tile stages; the groups' hand-over and the output staging reuse them (KS 1: staging of its own)
-template <int D, int KS>
-constexpr int fa16_flex_lds(int nw, int bn) {
-  const int stages = 4 * bn * 2 * D, part = nw * ((D / 16 - D / 16 / KS) * 2048 + 1024) + nw * 32 * (2 * D / KS + 8);
-  return KS == 1 ? stages + nw * 4096 : stages > part ? stages : part;
-}
+// LDS of fa16_loop_kernel: the tile stages and the output staging behind them
+constexpr int kFa16LoopLds = 4 * 128 * 256 + 8 * 16 * 256;
 
 #if defined(__HIP_DEVICE_COMPILE__)
 template <int... I, class F>
@@ -39,50 +37,72 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 
-// item: the first tile of NW / KS * 32 query rows, numbered through the heads ((batch, head) * row_tiles + tile; rows at
-// or beyond p.Sq do not exist); part: KS > 1, which part of a tile of NW * 32 rows it is.  KS 1: the workgroup goes on with
-// the tiles item + 32, item + 64, ... below `end`.
-// LDS: K stages at 0 and BN * 256 bytes, V stages behind them, with KS 1 the output staging behind those; swizzles and
-// operand layouts as in fa_fwd16_kernel.
-//
-// D: head_dim, 128 or 64 (fa_fwd16_d64_kernel's layouts: rows of 128 bytes, K chunk p of row r at p ^ ((r >> 1) & 7), V
-// chunk p at p ^ ((r >> 1) & 3)).
-template <int DT, int NW, int BN, int KS, bool KEYMASK, int D = 128>
-__device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* smem, int item, int part, int end) {
+// the rescale of column block nq when its reference maximum moves (see cond_rescale_fa16)
+template <int NQ>
+__device__ __forceinline__ void fa16_rescale(int flag, float delta, float alpha, float& l, f32x4_t& negm, f32x4_t& s0, f32x4_t& s1,
+                                             f32x4_t& s2, f32x4_t& s3, f32x4_t& s4, f32x4_t& s5, f32x4_t& s6, f32x4_t& s7,
+                                             f32x4_t (&o)[8][NQ], int nq) {
+  cond_rescale_fa16(flag, delta, alpha, l, negm, s0, s1, s2, s3, s4, s5, s6, s7, o[0][nq], o[1][nq], o[2][nq], o[3][nq], o[4][nq],
+                    o[5][nq], o[6][nq], o[7][nq]);
+}
+template <int NQ>
+__device__ __forceinline__ void fa16_rescale(int flag, float delta, float alpha, float& l, f32x4_t& negm, f32x4_t& s0, f32x4_t& s1,
+                                             f32x4_t& s2, f32x4_t& s3, f32x4_t& s4, f32x4_t& s5, f32x4_t& s6, f32x4_t& s7,
+                                             f32x4_t (&o)[4][NQ], int nq) {
+  if (flag) {
+    l *= alpha;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      negm[i] -= delta;
+      s0[i] -= delta; s1[i] -= delta; s2[i] -= delta; s3[i] -= delta;
+      s4[i] -= delta; s5[i] -= delta; s6[i] -= delta; s7[i] -= delta;
+      o[0][nq][i] *= alpha; o[1][nq][i] *= alpha; o[2][nq][i] *= alpha; o[3][nq][i] *= alpha;
+    }
+  }
+}
+
+// item: the tile of 256 query rows, numbered through the heads ((batch, head) * row_tiles + tile; rows at or beyond p.Sq
+// do not exist); LOOP: the first one, the workgroup goes on with item + 32, item + 64, ... below `end`.  Otherwise the
+// workgroup owns rows first_row .. first_row + part_rows of the tile.
+// LDS: K stages at 0 and one tile, V stages behind them, with LOOP the output staging behind those; swizzles and operand
+// layouts as in fa_fwd16_kernel (D 128) and fa_fwd16_d64_kernel (D 64: rows of 128 bytes, K chunk p of row r at
+// p ^ ((r >> 1) & 7), V chunk p at p ^ ((r >> 1) & 3)).
+template <int DT, bool LOOP, bool KEYMASK, int D>
+__device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* smem, int item, int first_row, int part_rows,
+                                               int end) {
   using E = Elem<DT>;
   using T = typename E::type;
   using X8 = typename E::x8;
-  static_assert(D == 128 || (D == 64 && KS > 1), "head_dim");
+  static_assert(D == 128 || (D == 64 && !LOOP), "head_dim");
+  constexpr int NW = 8, BN = 128, NQ = LOOP ? 2 : 1;
   constexpr int kRowBytes = 2 * D, kDmaRows = 1024 / kRowBytes, NDB = D / 16, NKS = D / 32, kTileBytes = BN * kRowBytes;
-  constexpr int RG = NW / KS;         // waves side by side over the query rows
-  constexpr int kKeys = BN / KS;      // keys of a tile that one wave takes
-  constexpr int NKB = kKeys / 16;     // its 16-key blocks
-  constexpr int NJ = kKeys / 32;      // its 32-key steps of the second product
-  static_assert(NKB % 2 == 0 && NW % KS == 0 && (4 * NW) % 16 == 0, "whole operand groups");
+  constexpr int NKB = BN / 16, NJ = BN / 32;  // 16-key blocks of the first product, 32-key steps of the second
+  constexpr int kWaveRows = 16 * NQ;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  const int rg = wave % RG, kg_i = wave / RG;
-  constexpr bool LOOP = KS == 1;
   const int Sq = p.Sq, Skv = p.Skv;
-  const int row_tiles = (Sq + NW * 32 - 1) / (NW * 32);
-  // the tile at hand, and with LOOP the one after it
-  int b, n, row0, b_nx = 0, n_nx = 0, row0_nx = 0;
+  const int row_tiles = (Sq + 255) / 256;
+  int b, n, row0;  // the tile at hand: batch entry, head, first query row of the wave
   auto locate = [&](int it, int& ib, int& in, int& irow) __attribute__((always_inline)) {
     const int bn = it / row_tiles;
     ib = bn / p.N;
     in = bn - ib * p.N;
-    irow = (it - bn * row_tiles) * (NW * 32) + part * (NW / KS * 32) + rg * 32;
+    irow = (it - bn * row_tiles) * 256 + first_row + wave * kWaveRows;
   };
   locate(item, b, n, row0);
+  const bool busy = LOOP || (wave * kWaveRows < part_rows && row0 < Sq);
 
   // ---- staging (LDS-DMA) -------------------------------------------------------------------------------------
   const int group = p.N / p.Nkv;
   const int k_range = (int)(((long long)(Skv - 1) * p.k_ss + D) * 2), v_range = (int)(((long long)(Skv - 1) * p.v_ss + D) * 2);
-  auto k_base = [&](int ib, int in) __attribute__((always_inline)) { return (const T*)p.k + ib * p.k_sb + (in / group) * p.k_sn; };
-  auto v_base = [&](int ib, int in) __attribute__((always_inline)) { return (const T*)p.v + ib * p.v_sb + (in / group) * p.v_sn; };
-  const T *kg = k_base(b, n), *vg = v_base(b, n), *kg_nx = kg, *vg_nx = vg;
+  const T *kg, *vg;
+  auto point_at_keys = [&](int ib, int in) __attribute__((always_inline)) {
+    kg = (const T*)p.k + ib * p.k_sb + (in / group) * p.k_sn;
+    vg = (const T*)p.v + ib * p.v_sb + (in / group) * p.v_sn;
+  };
+  point_at_keys(b, n);
   const int k_row_bytes = (int)p.k_ss * 2, v_row_bytes = (int)p.v_ss * 2;
   int k_voff, v_voff;
   {
@@ -92,9 +112,9 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     k_voff = row * k_row_bytes + ((pc ^ ksw) << 4);
     v_voff = row * v_row_bytes + (((((pc >> 1) ^ vsw) << 1) | (pc & 1)) << 4);
   }
-  auto load_tile = [&](const T* kp, const T* vp, int key0, int stage) __attribute__((always_inline)) {
-    const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, k_range, 0x00020000);
-    const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, v_range, 0x00020000);
+  auto load_tile = [&](int key0, int stage) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)kg, 0, k_range, 0x00020000);
+    const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)vg, 0, v_range, 0x00020000);
 #pragma unroll
     for (int i = 0; i < BN / kDmaRows / NW; ++i) {
       const int grp = i * NW + wave;
@@ -106,38 +126,38 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   };
 
   // ---- Q^T operand, resident: requested here, converted at the start of its tile ------------------------------------
-  X8 qf[2][NKS];
+  X8 qf[NQ][NKS];
   auto load_q = [&](int ib, int in, int irow) __attribute__((always_inline)) {
     const T* qg = (const T*)p.q + ib * p.q_sb + in * p.q_sn;
-    int c = lane & 15, g = lane >> 4;
-    if constexpr (LOOP) asm volatile("" : "+v"(c), "+v"(g));  // (recomputed for every tile, not kept in registers)
+    int qc = lane & 15, qgr = lane >> 4;
+    if constexpr (LOOP) asm volatile("" : "+v"(qc), "+v"(qgr));  // (recomputed for every tile, not kept in registers)
 #pragma unroll
-    for (int nq = 0; nq < 2; ++nq) {
-      const int qrow = irow + nq * 16 + c;
-      const T* src = qg + (long long)(qrow < Sq ? qrow : 0) * p.q_ss + 8 * g;
+    for (int nq = 0; nq < NQ; ++nq) {
+      const int qrow = irow + nq * 16 + qc;
+      const T* src = qg + (long long)(qrow < Sq ? qrow : 0) * p.q_ss + 8 * qgr;
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) qf[nq][ks] = *(const X8*)(src + 32 * ks);
     }
   };
-  f32x4_t oacc[NDB][2], negm[2], lt[2];
-  float l_run[2];
+  f32x4_t oacc[NDB][NQ], negm[NQ], lt[NQ];
+  float l_run[NQ];
   X8 ones;
 #pragma unroll
   for (int j = 0; j < 8; ++j) ones[j] = E::from_float(1.f);
 
-  // per-lane parts of the LDS read addresses (the wave's keys start at row kg_i * kKeys, a multiple of 16)
+  // per-lane parts of the LDS read addresses
   unsigned k_lds[NKS], v_lds[4];
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks)
-    k_lds[ks] = (unsigned)(uintptr_t)smem + (kg_i * kKeys + c) * kRowBytes + (((4 * ks + g) ^ (D == 128 ? c : c >> 1)) << 4);
+    k_lds[ks] = (unsigned)(uintptr_t)smem + c * kRowBytes + (((4 * ks + g) ^ (D == 128 ? c : c >> 1)) << 4);
 #pragma unroll
   for (int db = 0; db < 4; ++db)
-    v_lds[db] = (unsigned)(uintptr_t)smem + 2 * kTileBytes + (kg_i * kKeys + 4 * g + (c >> 2)) * kRowBytes +
+    v_lds[db] = (unsigned)(uintptr_t)smem + 2 * kTileBytes + (4 * g + (c >> 2)) * kRowBytes +
                 ((db ^ (D == 128 ? 4 * (g & 1) + (c >> 2) : ((4 * g + (c >> 2)) >> 1) & 3)) << 5) + 8 * (c & 3);
 
   const int tiles = (Skv + BN - 1) / BN;
   load_q(b, n, row0);
-  load_tile(kg, vg, 0, 0);
+  load_tile(0, 0);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();
   bool first = true;
@@ -163,23 +183,19 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   auto mask_reduce = [&]() __attribute__((always_inline)) {
     if constexpr (KEYMASK) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)  // the wave's own keys, from bit 0 on
-        kvis[j] = (unsigned)__builtin_amdgcn_ballot_w64(lane < BN / 4 && ((kraw >> (8 * j)) & 0xffu) != 0) >> (kg_i * (kKeys / 4));
+      for (int j = 0; j < 4; ++j)
+        kvis[j] = (unsigned)__builtin_amdgcn_ballot_w64(lane < BN / 4 && ((kraw >> (8 * j)) & 0xffu) != 0);
     }
   };
-  constexpr unsigned kOwn = (unsigned)((1ull << (kKeys / 4)) - 1);
 
-  // next_tile: the first key of the tile to request, of the workgroup's next tile of rows with `other`; < 0: none
-  auto tile_step = [&](auto stage_c, const int key0, const int next_tile, const bool other) __attribute__((always_inline)) {
+  // the products of the tile whose keys start at key0; next_mask0: first key of the mask bytes to request, < 0: none
+  auto compute = [&](auto stage_c, const int key0, const int next_mask0) __attribute__((always_inline)) {
     constexpr int stage = decltype(stage_c)::value;
-    if (next_tile >= 0) load_tile(other ? kg_nx : kg, other ? vg_nx : vg, next_tile, stage ^ 1);
-    const int next_key0 = other ? -1 : next_tile;
-    const unsigned kv_all = kvis[0] & kvis[1] & kvis[2] & kvis[3] & kOwn;
-    const int key_w = key0 + kg_i * kKeys;  // the wave's first key
+    const unsigned kv_all = kvis[0] & kvis[1] & kvis[2] & kvis[3];
 
     // S^T = K Q^T: operand groups of 2 key blocks of one 32-wide head_dim step, kAhead groups ahead of their use
-    f32x4_t sacc[NKB][2];
-    constexpr int kPer = NKB / 2, kGroups = NKS * kPer, kAhead = kGroups > 3 ? 3 : kGroups - 1;
+    f32x4_t sacc[NKB][NQ];
+    constexpr int kPer = NKB / 2, kGroups = NKS * kPer, kAhead = 3;
     X8 afrag[kAhead + 1][2];
     auto k_read = [&](auto gi_c, X8(&dst)[2]) __attribute__((always_inline)) {
       constexpr int gi = decltype(gi_c)::value, ks = gi / kPer, qu = gi % kPer;
@@ -195,7 +211,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int nq = 0; nq < 2; ++nq)
+        for (int nq = 0; nq < NQ; ++nq)
           sacc[2 * qu + i][nq] =
               E::mfma16(afrag[gi % (kAhead + 1)][i], qf[nq][ks], ks == 0 ? negm[nq] : sacc[2 * qu + i][nq]);
     });
@@ -203,80 +219,60 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
 #pragma unroll
     for (int gi = 0; gi < kGroups - kAhead; ++gi) {
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 2 * NQ, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 4 * kAhead, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 2 * NQ * kAhead, 0);
     __builtin_amdgcn_sched_barrier(0);
 
-    if (key_w + kKeys > Skv) {  // keys past the end of the sequence (last tile only)
+    if (key0 + BN > Skv) {  // keys past the end of the sequence (last tile only)
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (key_w + 16 * kb + 4 * g + i >= Skv) {
-            sacc[kb][0][i] = -INFINITY;
-            sacc[kb][1][i] = -INFINITY;
+          if (key0 + 16 * kb + 4 * g + i >= Skv) {
+#pragma unroll
+            for (int nq = 0; nq < NQ; ++nq) sacc[kb][nq][i] = -INFINITY;
           }
     }
     if constexpr (KEYMASK) {
-      if (kv_all != kOwn) {
+      if (kv_all != 0xffffffffu) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const unsigned w = kvis[i] >> g;  // key 16 * kb + 4 * g + i is bit 4 * kb + g of word i
 #pragma unroll
           for (int kb = 0; kb < NKB; ++kb)
             if (!((w >> (4 * kb)) & 1u)) {
-              sacc[kb][0][i] = -INFINITY;
-              sacc[kb][1][i] = -INFINITY;
+#pragma unroll
+              for (int nq = 0; nq < NQ; ++nq) sacc[kb][nq][i] = -INFINITY;
             }
         }
       }
     }
 
     // online softmax (exp2 domain, lazily moved reference maximum; see fa_fwd_kernel)
-    X8 pf[2][NJ];
+    X8 pf[NQ][NJ];
     bool seen = !KEYMASK;
 #pragma unroll
-    for (int nq = 0; nq < 2; ++nq) {
+    for (int nq = 0; nq < NQ; ++nq) {
       float mx = sacc[0][nq][0];
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sacc[kb][nq][i]);
       if constexpr (KEYMASK) seen = seen || __builtin_amdgcn_ballot_w64(mx > -INFINITY) != 0;
-      l_run[nq] += lt[nq][0];
-      if constexpr (NKB == 8) {  // (see cond_rescale_fa16)
-        float delta = 0.f, alpha = 1.f;
-        int moved = 0;
-        if (first || __builtin_amdgcn_ballot_w64(mx > kTau) != 0) {
-          mx = quarter_max(mx);
-          delta = first ? mx : fmaxf(mx, 0.f);
-          delta = (delta == -INFINITY) ? 0.f : delta;
-          alpha = first ? 1.f : fast_exp2(-delta);
-          moved = 1;
-        }
-        cond_rescale_fa16(__builtin_amdgcn_readfirstlane(moved), delta, alpha, l_run[nq], negm[nq], sacc[0][nq], sacc[1][nq],
-                          sacc[2][nq], sacc[3][nq], sacc[NKB - 4][nq], sacc[NKB - 3][nq], sacc[NKB - 2][nq],
-                          sacc[NKB - 1][nq], oacc[0][nq], oacc[1][nq], oacc[2][nq], oacc[3][nq], oacc[4][nq], oacc[5][nq],
-                          oacc[6][nq], oacc[7][nq]);
-      } else if (first || __builtin_amdgcn_ballot_w64(mx > kTau) != 0) {
+      float delta = 0.f, alpha = 1.f;
+      int moved = 0;
+      if (first || __builtin_amdgcn_ballot_w64(mx > kTau) != 0) {
         mx = quarter_max(mx);
-        float delta = first ? mx : fmaxf(mx, 0.f);
+        delta = first ? mx : fmaxf(mx, 0.f);
         delta = (delta == -INFINITY) ? 0.f : delta;
         // (first tile: sums and outputs are still zero; 2^-delta would overflow for rows far below zero and 0 * inf is NaN)
-        const float alpha = first ? 1.f : fast_exp2(-delta);
-        l_run[nq] *= alpha;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) negm[nq][i] -= delta;
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) sacc[kb][nq][i] -= delta;
-#pragma unroll
-        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) oacc[db][nq][i] *= alpha;
+        alpha = first ? 1.f : fast_exp2(-delta);
+        moved = 1;
       }
+      l_run[nq] += lt[nq][0];
+      fa16_rescale(__builtin_amdgcn_readfirstlane(moved), delta, alpha, l_run[nq], negm[nq], sacc[0][nq], sacc[1][nq],
+                   sacc[2][nq], sacc[3][nq], sacc[4][nq], sacc[5][nq], sacc[6][nq], sacc[7][nq], oacc, nq);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         X8 pk;
@@ -302,9 +298,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
         dst[2 * d4 + 1] = lds_read_tr16_async<off + 16 * kRowBytes>(a);
       }
     };
-    if constexpr (KEYMASK) {
-      if (next_key0 >= 0) mask_request(next_key0);  // lands during the second product
-    }
+    if (next_mask0 >= 0) mask_request(next_mask0);  // lands during the second product
     issue(std::integral_constant<int, 0>{}, vf[0]);
     static_for<NH * NJ>([&](auto step_c) __attribute__((always_inline)) {
       constexpr int s = decltype(step_c)::value, j = s / NH, dbh = s % NH;
@@ -320,222 +314,126 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
         u.s2[0] = vf[s & 1][2 * d4];
         u.s2[1] = vf[s & 1][2 * d4 + 1];
 #pragma unroll
-        for (int nq = 0; nq < 2; ++nq) oacc[4 * dbh + d4][nq] = E::mfma16(u.x, pf[nq][j], oacc[4 * dbh + d4][nq]);
+        for (int nq = 0; nq < NQ; ++nq) oacc[4 * dbh + d4][nq] = E::mfma16(u.x, pf[nq][j], oacc[4 * dbh + d4][nq]);
       }
       if constexpr (dbh == 0) {
 #pragma unroll
-        for (int nq = 0; nq < 2; ++nq)
+        for (int nq = 0; nq < NQ; ++nq)
           lt[nq] = E::mfma16(ones, pf[nq][j], j == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : lt[nq]);
       }
     });
     first = first && !seen;
+  };
+  // one key tile; next_key0: the first key of the tile to request (of the rows that kg and vg point at), < 0: none;
+  // other_rows: it belongs to the workgroup's next tile of rows
+  auto tile_step = [&](auto stage_c, const int key0, const int next_key0, const bool other_rows) __attribute__((always_inline)) {
+    if (next_key0 >= 0) load_tile(next_key0, decltype(stage_c)::value ^ 1);
+    if (busy) compute(stage_c, key0, other_rows ? -1 : next_key0);
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's part of the next tile has landed
     mask_reduce();
     __syncthreads();
   };
+
   for (;;) {
-  if constexpr (KEYMASK) {
-    mask_g = p.mask + b * p.m_sb + n * p.m_sn;
-    mask_request(0);
-    mask_reduce();
-  }
-#pragma unroll
-  for (int nq = 0; nq < 2; ++nq) {
-    int cc = c;
-    if constexpr (LOOP) asm volatile("" : "+v"(cc));
-    const bool ok = row0 + nq * 16 + cc < Sq;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      X8 v = qf[nq][ks];
-      if (!ok) v = X8{0};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = E::from_float((float)v[j] * p.scale_log2);
-      qf[nq][ks] = v;
+    if constexpr (KEYMASK) {
+      mask_g = p.mask + b * p.m_sb + n * p.m_sn;
+      mask_request(0);
+      mask_reduce();
     }
-    l_run[nq] = 0.f;
-    negm[nq] = lt[nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) oacc[db][nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-  first = true;
-  bool more = false;
-  unsigned touched = 0;
-  if constexpr (LOOP) {
-    more = item + 32 < end;
-    if (more) {
+    for (int nq = 0; nq < NQ; ++nq) {
+      int qc = c;
+      if constexpr (LOOP) asm volatile("" : "+v"(qc));
+      const bool ok = row0 + nq * 16 + qc < Sq;
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+        X8 v = qf[nq][ks];
+        if (!ok) v = X8{0};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = E::from_float((float)v[j] * p.scale_log2);
+        qf[nq][ks] = v;
+      }
+      l_run[nq] = 0.f;
+      negm[nq] = lt[nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) oacc[db][nq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    first = true;
+    const bool more = LOOP && item + 32 < end;
+    int b_nx = 0, n_nx = 0, row0_nx = 0;
+    unsigned touched = 0;
+    if (LOOP && more) {
       locate(item + 32, b_nx, n_nx, row0_nx);
-      kg_nx = k_base(b_nx, n_nx);
-      vg_nx = v_base(b_nx, n_nx);
       // a word of every 128-byte line of the next rows of q, so that they wait in the L2
-      const int qrow = min(row0_nx - rg * 32 + (tid >> 1), Sq - 1);
+      const int qrow = min(row0_nx - wave * kWaveRows + (tid >> 1), Sq - 1);
       touched = *(const unsigned*)((const T*)p.q + b_nx * p.q_sb + n_nx * p.q_sn + (long long)qrow * p.q_ss + (tid & 1) * 64);
     }
-  }
-  for (int t = 0; t < tiles; t += 2) {
-    tile_step(std::integral_constant<int, 0>{}, t * BN, t + 1 < tiles ? (t + 1) * BN : -1, false);
-    // (an even number of key tiles: the last step requests the first key tile of the next rows)
-    if (t + 1 < tiles)
-      tile_step(std::integral_constant<int, 1>{}, (t + 1) * BN, t + 2 < tiles ? (t + 2) * BN : (LOOP && more ? 0 : -1),
-                LOOP && t + 2 >= tiles);
-  }
-  if constexpr (LOOP) {
-    asm volatile("" ::"v"(touched));
-    if (more) {  // (an odd number: it goes into the stage of the last step, which no wave reads any more)
-      load_q(b_nx, n_nx, row0_nx);
-      if (tiles & 1) load_tile(kg_nx, vg_nx, 0, 0);
-    }
-  }
-
-  // ---- the groups' partial results (KS > 1) --------------------------------------------------------------------------
-  // Every wave ends up with all 32 rows of its row group and NDB / KS of the output's 16-wide blocks: it hands the other
-  // blocks to the waves that own them (16 bytes per lane and block, the accumulator layout as it is) together with its
-  // reference maxima and sums.  A group that saw no key has sum 0 and no say in the maximum.
-  constexpr int DB = NDB / KS;                       // output blocks a wave stores
-  constexpr int kPart = (NDB - DB) * 2 * 1024;       // bytes a wave hands out
-  constexpr int kStat = KS > 1 ? 4 * 256 : 0;      // m and l of two column blocks, a dword per lane
-  constexpr int kORow = 2 * 16 * DB + 8;           // a row of the output staging, padded
-  constexpr int kOBase = KS > 1 ? NW * (kPart + kStat) : 0;
-  static_assert(KS == 1 || kOBase + NW * 32 * kORow <= fa16_flex_lds<D, KS>(NW, BN), "fits");
-  float l_tot[2], m_tot[2];
-#pragma unroll
-  for (int nq = 0; nq < 2; ++nq) {
-    l_tot[nq] = l_run[nq] + lt[nq][0];
-    m_tot[nq] = -negm[nq][0];
-  }
-  if constexpr (KS > 1) {
-    MSD_LDS char* mine = smem + wave * (kPart + kStat);
-    // block db belongs to group db / DB; slot of a block that is not the writer's: the blocks in order, its own left out
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) {
-      const int owner = db / DB;
-      const int slot = owner < kg_i ? db : db - DB;
-      if (owner != kg_i) {
-#pragma unroll
-        for (int nq = 0; nq < 2; ++nq) *(MSD_LDS f32x4_t*)(mine + (slot * 2 + nq) * 1024 + lane * 16) = oacc[db][nq];
+    for (int t = 0; t < tiles; t += 2) {
+      tile_step(std::integral_constant<int, 0>{}, t * BN, t + 1 < tiles ? (t + 1) * BN : -1, false);
+      if (t + 1 < tiles) {
+        // (an even number of key tiles: the last step requests the first key tile of the next rows)
+        const bool other_rows = LOOP && more && t + 2 >= tiles;
+        if (other_rows) point_at_keys(b_nx, n_nx);
+        tile_step(std::integral_constant<int, 1>{}, (t + 1) * BN, t + 2 < tiles ? (t + 2) * BN : (other_rows ? 0 : -1), other_rows);
       }
     }
-#pragma unroll
-    for (int nq = 0; nq < 2; ++nq) {
-      *(MSD_LDS float*)(mine + kPart + (2 * nq) * 256 + lane * 4) = m_tot[nq];
-      *(MSD_LDS float*)(mine + kPart + (2 * nq + 1) * 256 + lane * 4) = l_tot[nq];
-    }
-    __syncthreads();
-    f32x4_t own[DB][2];
-#pragma unroll
-    for (int k = 0; k < KS; ++k)
-      if (k == kg_i) {
-#pragma unroll
-        for (int d = 0; d < DB; ++d)
-#pragma unroll
-          for (int nq = 0; nq < 2; ++nq) own[d][nq] = oacc[k * DB + d][nq];
-      }
-#pragma unroll
-    for (int nq = 0; nq < 2; ++nq) {
-      float mk[KS], lk[KS], m = -INFINITY, l = 0.f;
-#pragma unroll
-      for (int k = 0; k < KS; ++k) {
-        MSD_LDS const char* st = smem + (k * RG + rg) * (kPart + kStat) + kPart + (2 * nq) * 256 + lane * 4;
-        mk[k] = *(MSD_LDS const float*)st;
-        lk[k] = *(MSD_LDS const float*)(st + 256);
-        if (lk[k] != 0.f) m = fmaxf(m, mk[k]);
-      }
-      f32x4_t sum[DB];
-#pragma unroll
-      for (int d = 0; d < DB; ++d) sum[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int k = 0; k < KS; ++k) {
-        const float w = lk[k] != 0.f ? fast_exp2(mk[k] - m) : 0.f;
-        l += w * lk[k];
-        MSD_LDS const char* from = smem + (k * RG + rg) * (kPart + kStat);
-#pragma unroll
-        for (int d = 0; d < DB; ++d) {
-          const int db = kg_i * DB + d;
-          const int slot = kg_i < k ? db : db - DB;
-          f32x4_t v = own[d][nq];
-          if (k != kg_i) v = *(MSD_LDS const f32x4_t*)(from + (slot * 2 + nq) * 1024 + lane * 16);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) sum[d][i] += w * v[i];
+    if constexpr (LOOP) {
+      asm volatile("" ::"v"(touched));
+      if (more) {  // (an odd number: it goes into the stage of the last step, which no wave reads any more)
+        load_q(b_nx, n_nx, row0_nx);
+        if (tiles & 1) {
+          point_at_keys(b_nx, n_nx);
+          load_tile(0, 0);
         }
       }
-#pragma unroll
-      for (int d = 0; d < DB; ++d) oacc[d][nq] = sum[d];
-      l_tot[nq] = l;
-      m_tot[nq] = m;
     }
-  }
 
-  // ---- normalise, transpose the wave's rows through LDS, coalesced store ----------------------------------------------
-  T* og = (T*)p.o + b * p.o_sb + n * p.o_sn;
-  if constexpr (LOOP) {
-    // 16 rows at a time through 4 KiB per wave behind the tile stages (which already fill with the next rows' keys):
-    // 16-byte chunk k of row r sits at chunk k ^ r
-    MSD_LDS char* ost = smem + 4 * BN * 256 + wave * 4096;
-    int c = lane & 15, g = lane >> 4;
-    asm volatile("" : "+v"(c), "+v"(g));
+    // ---- normalise, transpose 16 rows at a time through LDS (16-byte chunk k of row r at chunk k ^ r), coalesced store ------
+    // LOOP: behind the tile stages, which already fill with the next rows' keys; otherwise in them: no wave reads them any more
+    if (busy) {
+      constexpr int kChunks = D / 8, kSwz = kChunks - 1;
+      T* og = (T*)p.o + b * p.o_sb + n * p.o_sn;
+      MSD_LDS char* ost = smem + (LOOP ? 4 * kTileBytes : 0) + wave * 16 * kRowBytes;
+      int oc = lane & 15, ogr = lane >> 4, ol = lane;
+      if constexpr (LOOP) asm volatile("" : "+v"(oc), "+v"(ogr), "+v"(ol));
 #pragma unroll
-    for (int nq = 0; nq < 2; ++nq) {
-      const float inv = l_tot[nq] > 0.f ? 1.f / l_tot[nq] : 0.f;
-      const int qrow_l = row0 + nq * 16 + c;
-      if (p.lse && g == 0 && qrow_l < Sq)
-        p.lse[((long long)b * p.N + n) * Sq + qrow_l] =
-            l_tot[nq] > 0.f ? m_tot[nq] * 0.6931471805599453f + __logf(l_tot[nq]) : -INFINITY;
+      for (int nq = 0; nq < NQ; ++nq) {
+        const float l_tot = l_run[nq] + lt[nq][0];
+        const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+        const int qrow_l = row0 + nq * 16 + oc;
+        if (p.lse && ogr == 0 && qrow_l < Sq)
+          p.lse[((long long)b * p.N + n) * Sq + qrow_l] =
+              l_tot > 0.f ? -negm[nq][0] * 0.6931471805599453f + __logf(l_tot) : -INFINITY;
 #pragma unroll
-      for (int db = 0; db < 8; ++db) {
-        typename E::x4 pk;
+        for (int db = 0; db < NDB; ++db) {
+          typename E::x4 pk;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) pk[i] = E::from_float(oacc[db][nq][i] * inv);
-        *(MSD_LDS typename E::x4*)(ost + c * 256 + (((2 * db + (g >> 1)) ^ c) << 4) + 8 * (g & 1)) = pk;
+          for (int i = 0; i < 4; ++i) pk[i] = E::from_float(oacc[db][nq][i] * inv);
+          *(MSD_LDS typename E::x4*)(ost + oc * kRowBytes + (((2 * db + (ogr >> 1)) ^ (oc & kSwz)) << 4) + 8 * (ogr & 1)) = pk;
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < kChunks / 4; ++i) {
+          const int row = i * (64 / kChunks) + ol / kChunks, ch = ol % kChunks, qrow = row0 + nq * 16 + row;
+          const i32x4_t v = *(MSD_LDS const i32x4_t*)(ost + row * kRowBytes + ((ch ^ (row & kSwz)) << 4));
+          if (qrow < Sq) *(i32x4_t*)(og + (long long)qrow * p.o_ss + ch * 8) = v;
+        }
+        __builtin_amdgcn_wave_barrier();
       }
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = 4 * i + g, qrow = row0 + nq * 16 + row;
-        const i32x4_t v = *(MSD_LDS const i32x4_t*)(ost + row * 256 + ((c ^ row) << 4));
-        if (qrow < Sq) *(i32x4_t*)(og + (long long)qrow * p.o_ss + c * 8) = v;
+    }
+    if constexpr (LOOP) {
+      if (!more) return;
+      item += 32;
+      b = b_nx;
+      n = n_nx;
+      row0 = row0_nx;
+      if (tiles & 1) {
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        __syncthreads();
       }
-      __builtin_amdgcn_wave_barrier();
+    } else {
+      return;
     }
-    if (!more) return;
-    item += 32;
-    b = b_nx;
-    n = n_nx;
-    row0 = row0_nx;
-    kg = kg_nx;
-    vg = vg_nx;
-    if (tiles & 1) {
-      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-      __syncthreads();
-    }
-    continue;
-  }
-  MSD_LDS char* ost = smem + kOBase + wave * 32 * kORow;
-#pragma unroll
-  for (int nq = 0; nq < 2; ++nq) {
-    const float inv = l_tot[nq] > 0.f ? 1.f / l_tot[nq] : 0.f;
-    const int qrow_l = row0 + nq * 16 + c;
-    if (p.lse && kg_i == 0 && g == 0 && qrow_l < Sq)
-      p.lse[((long long)b * p.N + n) * Sq + qrow_l] =
-          l_tot[nq] > 0.f ? m_tot[nq] * 0.6931471805599453f + __logf(l_tot[nq]) : -INFINITY;
-#pragma unroll
-    for (int d = 0; d < DB; ++d) {
-      typename E::x4 pk;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) pk[i] = E::from_float(oacc[d][nq][i] * inv);
-      *(MSD_LDS typename E::x4*)(ost + (nq * 16 + c) * kORow + (16 * d + 4 * g) * 2) = pk;
-    }
-  }
-  __builtin_amdgcn_wave_barrier();
-  constexpr int kChunks = 2 * DB;  // 16-byte chunks of a row
-#pragma unroll
-  for (int i = 0; i < 32 * kChunks / 64; ++i) {
-    const int ch = i * 64 + lane;
-    const int row = ch / kChunks, c16 = ch % kChunks;
-    const int qrow = row0 + row;
-    const i32x2_t lo = *(MSD_LDS const i32x2_t*)(ost + row * kORow + c16 * 16);
-    const i32x2_t hi = *(MSD_LDS const i32x2_t*)(ost + row * kORow + c16 * 16 + 8);
-    if (qrow < Sq) *(i32x4_t*)(og + (long long)qrow * p.o_ss + kg_i * (16 * DB) + c16 * 8) = i32x4_t{lo[0], lo[1], hi[0], hi[1]};
-  }
-  return;
   }
 }
 #endif

@@ -147,8 +147,10 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void fa_fwd16_d64_kernel(
     const fa16::Part w = fa16::runs_tail(blockIdx.x, p.B * p.N, (p.Sq + kBM - 1) / kBM, p.tail_full, TAIL);
     if (w.group < 0) return;
     if (w.part >= 0) {
-      if (w.tile * kBM + w.part * (kBM / TAIL) < p.Sq)
-        fa16_flex_body<DT, 8, BN, TAIL, GEN == 3, 64>(p, smem, w.group * ((p.Sq + kBM - 1) / kBM) + w.tile, w.part, 0);
+      constexpr int kPartRows = kBM / TAIL;
+      if (w.tile * kBM + w.part * kPartRows < p.Sq)
+        fa16_flex_body<DT, false, GEN == 3, 64>(p, smem, w.group * ((p.Sq + kBM - 1) / kBM) + w.tile, w.part * kPartRows,
+                                                kPartRows, 0);
       return;
     }
     bn = w.group;
@@ -504,13 +506,12 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void fa_fwd16_d64_kernel(
 template <int DT, int GEN, bool DPAD = false, int NW = kD64Waves, int TAIL = 0>
 static int launch_d64(const FaParams& p, hipStream_t stream) {
   auto kern = fa_fwd16_d64_kernel<DT, GEN, DPAD, NW, TAIL>;
-  constexpr int kLds = TAIL ? fa16_flex_lds<64, TAIL ? TAIL : 2>(8, kD64BN) : kD64Lds;
-  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kD64Lds) != hipSuccess)
     return MSD_ERR_LAUNCH;
   const long long grid = TAIL ? fa16::runs_tail_grid((long long)p.B * p.N, (p.Sq + 255) / 256, p.tail_full, TAIL)
                               : fa16_grid<GEN, false>(p, NW * 32);
   if (grid > 0x7ffffff0ll) return MSD_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), kLds, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), kD64Lds, stream, p);
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
 }
 

@@ -727,8 +727,10 @@ __global__ __launch_bounds__(NWAVES * 64, 1) void fa_fwd16_kernel(const FaParams
     const fa16::Part w = fa16::runs_tail(blockIdx.x, p.B * p.N, (p.Sq + kBM - 1) / kBM, p.tail_full, TAIL);
     if (w.group < 0) return;
     if (w.part >= 0) {
-      if (w.tile * kBM + w.part * (kBM / TAIL) < p.Sq)
-        fa16_flex_body<DT, 8, BN, TAIL, GEN == 3>(p, smem, w.group * ((p.Sq + kBM - 1) / kBM) + w.tile, w.part, 0);
+      constexpr int kPartRows = kBM / TAIL;
+      if (w.tile * kBM + w.part * kPartRows < p.Sq)
+        fa16_flex_body<DT, false, GEN == 3, 128>(p, smem, w.group * ((p.Sq + kBM - 1) / kBM) + w.tile, w.part * kPartRows,
+                                                 kPartRows, 0);
       return;
     }
     bn = w.group;
@@ -1311,16 +1313,15 @@ __global__ __launch_bounds__(512, 1) void fa16_loop_kernel(const FaParams p) {
   const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
   const int end = min(total, (x + 1) * per_xcd);
   if (x * per_xcd + j >= end) return;
-  fa16_flex_body<DT, 8, 128, 1, KEYMASK>(p, (MSD_LDS char*)smem_raw, x * per_xcd + j, 0, end);
+  fa16_flex_body<DT, true, KEYMASK, 128>(p, (MSD_LDS char*)smem_raw, x * per_xcd + j, 0, 256, end);
 #endif
 }
 template <int DT, bool KEYMASK>
 static int launch_fa16_loop(const FaParams& p, hipStream_t stream) {
   auto kern = fa16_loop_kernel<DT, KEYMASK>;
-  constexpr int kLds = fa16_flex_lds<128, 1>(8, 128);
-  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kFa16LoopLds) != hipSuccess)
     return MSD_ERR_LAUNCH;
-  hipLaunchKernelGGL(kern, dim3(256), dim3(512), kLds, stream, p);
+  hipLaunchKernelGGL(kern, dim3(256), dim3(512), kFa16LoopLds, stream, p);
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
 }
 
@@ -1334,13 +1335,12 @@ static int forced_tile_rows() {
 
 // Plain dense attention or with a key mask, head dims 128 and 64: how the last round of workgroups is cut.  An XCD runs
 // its share of the 256-row tiles in rounds of 32; when the last round has at most 8 or 16 tiles, they go as four or two
-// workgroups each (fa16_flex.hpp), which still is one round: a round of quarter tiles takes 0.46, one of half tiles 0.62
-// of a round of whole ones, two rounds of either more than one (20 tiles: 140 against 110 us at 5120 keys).
-// B x N 8, keys = queries, before -> now, head_dim 128: 4 tiles per XCD 21 -> 15 us, 16 tiles 71 -> 62 us, 32 + 1 tiles
-// 350 -> 278 us, 32 + 16 tiles 538 -> 467 us, 64 + 8 tiles 1245 -> 1042 us.  From 16 whole rounds on the cut would gain 3 %
-// and less (46 rounds, 40 heads at 75600 tokens: 85.2 -> 84.1 ms) and is left out: there a call's bits do not depend on how
-// many problems its batch holds.  Head_dim 64: 8 tiles 24 -> 16 us, 16 tiles 45 -> 40, 32 + 8 tiles 251 -> 213, 64 + 4 tiles 749 -> 614 us, 13 * 32 + 4
-// tiles (48 heads, 17776) 3.74 -> 3.60 ms.
+// workgroups each (fa16_flex.hpp), which still is one round: a round of quarter tiles takes 0.39, one of half tiles 0.62
+// of a round of whole ones, two rounds of half tiles more than one.  A row has the same bits in whole and in cut tiles.
+// B x N 8, keys = queries, before -> now, head_dim 128: 4 tiles per XCD 21 -> 14 us, 16 tiles 71 -> 65 us, 32 + 1 tiles
+// 353 -> 283 us, 32 + 16 tiles 540 -> 482 us, 64 + 8 tiles 1257 -> 1064 us.  From 16 whole rounds on, where it could gain 3 %
+// and less, the launch stays whole.  Head_dim 64: 8 tiles 24 -> 16 us, 16 tiles 45 -> 39, 32 + 8 tiles 247 -> 213, 64 + 4
+// tiles 738 -> 608 us, 13 * 32 + 4 tiles (48 heads, 17776) 3.65 -> 3.55 ms.
 // Returns the number of parts (0: no cut) and sets p.tail_full.
 static int fa16_split(FaParams& p) {
   constexpr int kCusPerXcd = 32;
@@ -1560,10 +1560,10 @@ int mindiesd_flash_attention_fwd(const void* q, const void* k, const void* v, vo
   FaParams p = make_params(q, k, v, out, lse, B, N, Nkv, Sq, Skv, st, scale);
   const bool half_tiles = prefers_half_tiles(B, N, Sq);
   if (D == 64 && fa16_d64_supported(p)) {
-    // (one round and a half of tiles over few keys: the 4-wave workgroups, 19.5 against 21.4 us at 512 keys, B x N 8,
-    // S 12288; the cut round gains 1.25 us per 1024 keys on them and is ahead from 2048 keys on, 295 against 308 us at 12288)
+    // (one round and a half of tiles over few keys: the 4-wave workgroups, 19.4 against 19.9 us at 512 and 30.5 against 30.8
+    // at 1024 keys, B x N 8, S 12288; the cut round is ahead from 1280 keys on, 36.1 against 36.5, and 290 against 302 at 12288)
     int split = fa16_split(p);
-    if (split == 2 && half_tiles && p.tail_full > 0 && Skv < 2048) split = 0;
+    if (split == 2 && half_tiles && p.tail_full > 0 && Skv < 1280) split = 0;
     return launch_fa16_d64(p, dtype, stream, 0, half_tiles ? 128 : 256, split);
   }
   // Head dims between 64 and 128 run as head_dim 128 on the 16x16x32 kernel (the part of the matrix work spent on

@@ -9,6 +9,7 @@ import pytest
 import torch
 
 import mindiesd
+from mindiesd.layers.flash_attn.hip_flash_attn import flash_attention
 
 pytestmark = pytest.mark.gpu
 U = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}
@@ -80,10 +81,32 @@ def test_cut_rounds(heads, q_len, kv_len, dtype, masked, d):
     check(mindiesd.attention_forward(*t, attn_mask=m4, head_first=False).transpose(1, 2), want, v, dtype)
 
 
+# equal problems side by side: 32 + 1 and 32 + 12 tiles per XCD, 32 + 19, 64 + 2 with ragged rows, 64 without a rest and few keys
+EQUAL = [(8, 8448, 640), (8, 11264, 1536), (8, 12800, 900), (264, 300, 450), (8, 16384, 512), (24, 1101, 1101)]
+
+
+@pytest.mark.parametrize("heads,q_len,kv_len", EQUAL)
+@pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (128, torch.float16), (64, torch.float16)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_equal_problems_have_equal_bits(monkeypatch, heads, q_len, kv_len, d, dtype, masked):
+    """The heads of a call hold the same problem: whichever kind of tile computes a row, its output and log-sum-exp have the
+    same bits, those of a launch in whole tiles of 256 rows."""
+    g = torch.Generator(device="cuda").manual_seed(kv_len)
+    q, k, v = (torch.randn((1, 1, s, d), generator=g, device="cuda").to(dtype).expand(1, heads, s, d).contiguous()
+               for s in (q_len, kv_len, kv_len))
+    mask = (torch.rand((1, 1, 1, kv_len), generator=g, device="cuda") < 0.5) if masked else None
+    out, lse = flash_attention(q, k, v, d ** -0.5, return_lse=True, attn_mask=mask)
+    assert torch.equal(out, out[:, :1].expand_as(out)) and torch.equal(lse, lse[:, :1].expand_as(lse))
+    assert torch.equal(out, flash_attention(q, k, v, d ** -0.5, attn_mask=mask))
+    monkeypatch.setenv("MINDIESD_DENSE_TILE_ROWS", "256")
+    whole, whole_lse = flash_attention(q, k, v, d ** -0.5, return_lse=True, attn_mask=mask)
+    assert torch.equal(out, whole) and torch.equal(lse, whole_lse)
+
+
 @pytest.mark.parametrize("d", [128, 64])
-def test_groups_of_very_different_maxima(d):
-    """The groups of waves that share a row keep reference maxima of their own: scores that differ by hundreds between
-    the groups' keys, rows whose scores all lie far below zero, and a NaN and an infinity that stay in their rows."""
+def test_very_different_maxima(d):
+    """Scores that differ by hundreds between the halves of every key tile, rows whose scores all lie far below zero, and a
+    NaN and an infinity that stay in their rows."""
     g = torch.Generator(device="cuda").manual_seed(5)
     q, k, v = (torch.randn((1, 4, s, d), generator=g, device="cuda").bfloat16() for s in (512, 640, 640))
     q[:, :, :, 0] = 4.0
