@@ -1351,6 +1351,16 @@ static int fa16_split(FaParams& p) {
   return 4 * rest > kCusPerXcd ? 2 : 4;
 }
 
+// Dense calls at head_dim 128 of one whole round and a cut one over few keys that end in the first half of a 128-key tile: the
+// 4-wave kernel (128-row workgroups, two per CU, 64-key tiles) walks half a tile less.  B x N 8, S 12288 (16 cut tiles per XCD)
+// and 8448 (1), cut against 4-wave: 448 keys 32.2 / 29.5 and 27.9 / 27.2 us, 576 keys 36.8 / 34.7 and 31.6 / 32.0, 832 keys
+// 46.1 / 45.0, 960 keys 50.9 / 50.4 but 48.5 / 48.9 at 12 tiles.  Keys that fill their tiles: 512 keys 31.6 / 31.9 and 27.4 / 29.6,
+// 896 keys 45.6 / 47.7; with a second whole round the 4-wave kernel is 10 % and more behind (400 keys, S 16640: 47.4 / 56.2).
+static bool rest_on_four_waves(FaParams p) {
+  const int split = fa16_split(p), tiles64 = (p.Skv + 63) / 64;
+  return split != 0 && p.tail_full == 32 && (tiles64 & 1) != 0 && tiles64 <= (split == 2 ? 13 : 7);
+}
+
 constexpr int kLoopKv = 768;  // keys up to which workgroups keep their CU (fa16_loop_kernel)
 template <int DT, int GEN>
 static int launch_fa16_rounds(FaParams p, hipStream_t stream) {
@@ -1583,8 +1593,8 @@ int mindiesd_flash_attention_fwd(const void* q, const void* k, const void* v, vo
   // A few key tiles per query tile (cross attention over a short text): the launch is mostly reading Q and writing O,
   // and two 4-wave workgroups per CU overlap one's memory phases with the other's tiles better than one 8-wave
   // workgroup does (75600 queries x 40 heads: 0.42 vs 0.53 ms at 77 keys, 0.62 vs 0.70 at 226, equal at 512).
-  // (Grids of whatever size on more keys than that: launch_fa16_rounds.)
-  if (Skv <= kShortKv || forced_tile_rows() == 128) {
+  // (More keys than that: launch_fa16_rounds, but for the grids that rest_on_four_waves describes.)
+  if (Skv <= kShortKv || forced_tile_rows() == 128 || rest_on_four_waves(p)) {
     if (dtype == MSD_DTYPE_BF16) return launch_fa<MSD_DTYPE_BF16, 4, 32, 64, false, 1, 1>(p, stream);
     return launch_fa<MSD_DTYPE_F16, 4, 32, 64, false, 1, 1>(p, stream);
   }

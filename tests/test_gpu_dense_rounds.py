@@ -103,6 +103,25 @@ def test_equal_problems_have_equal_bits(monkeypatch, heads, q_len, kv_len, d, dt
     assert torch.equal(out, whole) and torch.equal(lse, whole_lse)
 
 
+# one whole round and a rest per XCD (1, 8, 9, 16 tiles, B x N 8) on few keys: the 4-wave kernel where the last 128-key tile is at
+# most half full, below 449 keys for rests up to 8 and below 833 above; a second whole round, a full last tile: never
+@pytest.mark.parametrize("q_len,kv_len,four_waves", [
+    (8448, 385, True), (10240, 448, True), (10240, 449, False), (10496, 448, True), (12288, 448, True), (12288, 449, False),
+    (10240, 576, False), (10496, 520, True), (12288, 832, True), (12288, 833, False), (12288, 900, False), (12544, 448, False),
+    (8192, 448, False), (16640, 448, False)])
+def test_kernel_of_one_round_and_a_rest(monkeypatch, q_len, kv_len, four_waves):
+    """The two kernels add a row up in different orders, so their bits tell which one ran."""
+    g = torch.Generator(device="cuda").manual_seed(q_len + kv_len)
+    q, k, v = (torch.randn((1, 8, s, 128), generator=g, device="cuda").bfloat16() for s in (q_len, kv_len, kv_len))
+    out = {}
+    for rows in (None, "256", "128"):
+        if rows:
+            monkeypatch.setenv("MINDIESD_DENSE_TILE_ROWS", rows)
+        out[rows] = mindiesd.attention_forward(q, k, v, head_first=True)
+    assert not torch.equal(out["128"], out["256"])
+    assert torch.equal(out[None], out["128" if four_waves else "256"])
+
+
 @pytest.mark.parametrize("d", [128, 64])
 def test_very_different_maxima(d):
     """Scores that differ by hundreds between the halves of every key tile, rows whose scores all lie far below zero, and a
