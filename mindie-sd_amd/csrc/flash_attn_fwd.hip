@@ -1361,13 +1361,19 @@ static bool rest_on_four_waves(FaParams p) {
   return split != 0 && p.tail_full == 32 && (tiles64 & 1) != 0 && tiles64 <= (split == 2 ? 13 : 7);
 }
 
-constexpr int kLoopKv = 768;  // keys up to which workgroups keep their CU (fa16_loop_kernel)
+// When workgroups keep their CU (fa16_loop_kernel): up to 768 keys (where its gain ends, see there), from two rounds on when the
+// last one is not cut, from eight on when it would be.  The loop cannot cut its last round, and what it saves grows with the rounds.
+// B x N 8, loop against whole or cut tiles:
+//   32 + 24 tiles per XCD 36.8 / 37.7 us at 400 keys, 42.5 / 42.9 at 640; 64: 39.4 / 40.5, 45.0 / 46.0; 96: 56.2 / 59.4, 66.5 / 67.6
+//   64 + 8 (quarter tiles) 52.6 / 47.5, 61.6 / 54.0; 128 + 8: 85.9 / 84.4, 104.3 / 96.8; 192 + 8: 118.0 / 120.3, 144.0 / 139.9;
+//   256 + 8: 152.5 / 157.3, 184.6 / 183.1; 256 + 16 (half tiles) 157.1 / 165.3, 189.1 / 191.2; 320 + 2: 192.5 / 199.1, 232.1 / 228.6
+constexpr int kLoopKv = 768, kLoopRounds = 2, kLoopRoundsCut = 8;
 template <int DT, int GEN>
 static int launch_fa16_rounds(FaParams p, hipStream_t stream) {
   const long long per_xcd = ((long long)p.B * p.N * ((p.Sq + 255) / 256) + 7) / 8;
   const int split = fa16_split(p);
-  // few keys: the workgroups that keep their CU, when there are rounds enough that cutting the last one matters less
-  if (p.Skv <= kLoopKv && per_xcd >= 64 && (split == 0 || per_xcd >= 256) && per_xcd < (1 << 27) && forced_tile_rows() == 0)
+  if (p.Skv <= kLoopKv && per_xcd >= 32 * (split == 0 ? kLoopRounds : kLoopRoundsCut) && per_xcd < (1 << 27) &&
+      forced_tile_rows() == 0)
     return launch_fa16_loop<DT, GEN == 3>(p, stream);
   if (split == 2) return launch_fa16<DT, 8, false, false, GEN, false, 2>(p, stream);
   if (split == 4) return launch_fa16<DT, 8, false, false, GEN, false, 4>(p, stream);
