@@ -1,6 +1,7 @@
-"""Dense attention at head dims 128 and 64 where the last round of workgroups is cut into half or quarter tiles
-(fa16_split) or, over a few key tiles, workgroups keep their CU (fa16_loop_kernel): whole rounds before it or none, tiles per XCD at the edges of the rule, ragged query and key
-lengths around the 64-, 128- and 256-row and the 128-key tiles, both layouts and types, and the key-padding mask.
+"""Dense attention at head dims 128 and 64 where the last round of workgroups is cut into half or quarter tiles (fa16_split) or,
+over a few key tiles, workgroups keep their CU (fa16_loop_kernel): whole rounds before it or none, tiles per XCD at the edges of
+the rules, ragged query and key lengths around the 64-, 128- and 256-row and the 128-key tiles, both layouts and types, the
+key-padding mask, and the bits of equal rows.
 
 Bounds against the float64 softmax of the same 16-bit operands: the query is rounded to 16 bits after scaling and a
 probability before the second product (a relative u = 2^-9 for bf16, 2^-12 for fp16, each), the output once more; in the
@@ -33,45 +34,72 @@ def check(got, want, v, dtype):
     assert err.abs().max().item() <= 16 * U[dtype] * v.abs().max().item()
 
 
-# (batch, heads, q_len, kv_len), 2 to 9 rounds: even and odd numbers of key tiles, ragged rows, heads that change inside
-# a workgroup's run, and the last key count of the rule
-LOOP_CASES = [(1, 40, 4200, 385), (2, 20, 3328, 513), (1, 264, 600, 640), (3, 11, 8200, 767), (1, 536, 256, 768), (1, 523, 257, 500)]
+def kind(problems, q_len, kv_len, d=128, masked=False):
+    """What runs a dense call without or with a key mask, as the library's dispatch has it: "loop", "4 waves", or the number of
+    parts a tile of the last round is cut into (0: whole tiles)."""
+    per_xcd = -(-problems * -(-q_len // 256) // 8)
+    rounds, rest = divmod(per_xcd, 32)
+    parts = 0 if rest == 0 or rest > 16 or rounds >= 16 else 2 if rest > 8 else 4
+    keys64 = -(-kv_len // 64)
+    if d == 128 and kv_len <= 768 and rounds >= (8 if parts else 2):
+        return "loop"
+    if not masked and rounds == 1 and parts and (kv_len < 1280 and parts == 2 if d == 64 else
+                                                 keys64 % 2 and keys64 <= (13 if parts == 2 else 7)):
+        return "4 waves"
+    return parts
 
 
-@pytest.mark.parametrize("batch,heads,q_len,kv_len", LOOP_CASES)
+# (batch, heads, heads of k and v, q_len, kv_len), 2 to 8 rounds: 4, 5 and 6 key tiles, ragged rows, batch entries and (shared)
+# heads that change inside a workgroup's run, the first and the last key count of the rule, eight rounds and a rest
+LOOP_CASES = [(1, 40, 40, 4200, 385), (2, 21, 7, 4097, 513), (1, 225, 45, 600, 640), (3, 11, 11, 5400, 767), (1, 680, 68, 250, 768),
+              (1, 350, 350, 257, 500), (1, 2100, 210, 256, 600)]
+
+
+@pytest.mark.parametrize("batch,heads,kv_heads,q_len,kv_len", LOOP_CASES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("masked", [False, True])
-def test_rows_in_a_loop(batch, heads, q_len, kv_len, dtype, masked):
-    print("case", batch, heads, q_len, kv_len, dtype, masked, flush=True)
+def test_rows_in_a_loop(batch, heads, kv_heads, q_len, kv_len, dtype, masked):
+    """Output and log-sum-exp.  Bound of the latter: a score moves by at most u times the sum of its products' absolute values
+    (the query's second rounding), the log-sum-exp by at most the largest of these, plus the 32-bit sums."""
+    if masked and q_len < 256:
+        q_len = 256                       # key masks run on this kernel from 256 query rows on
+    assert kind(batch * heads, q_len, kv_len, masked=masked) == "loop"
     g = torch.Generator(device="cuda").manual_seed(heads + q_len)
-    q, k, v = (torch.randn((batch, s, heads, 128), generator=g, device="cuda").to(dtype) for s in (q_len, kv_len, kv_len))
+    q, k, v = (torch.randn((batch, s, h, 128), generator=g, device="cuda").to(dtype)
+               for s, h in ((q_len, heads), (kv_len, kv_heads), (kv_len, kv_heads)))
     mask = torch.rand((batch, kv_len), generator=g, device="cuda") < 0.5 if masked else None
-    m4 = None if mask is None else mask.view(batch, 1, 1, kv_len)
-    want = reference(*(x.transpose(1, 2) for x in (q, k, v)), mask)
-    got = mindiesd.attention_forward(q, k, v, attn_mask=m4, head_first=False)
-    check(got.transpose(1, 2), want, v, dtype)
+    got, lse = flash_attention(q, k, v, 128 ** -0.5, layout="BSND", return_lse=True,
+                               attn_mask=None if mask is None else mask.view(batch, 1, 1, kv_len))
+    qt, kt, vt = (x.transpose(1, 2).repeat_interleave(heads // x.shape[2], 1) for x in (q, k, v))
+    check(got.transpose(1, 2), reference(qt, kt, vt, mask), v, dtype)
+    for b, n in {(0, 0), (batch - 1, heads // 2), (batch - 1, heads - 1)}:
+        qd, kd = qt[b, n].double(), kt[b, n].double()
+        s, slack = qd @ kd.t() * 128 ** -0.5, (qd.abs() @ kd.abs().t() * 128 ** -0.5).amax(-1) * U[dtype] + 1e-5
+        want = torch.logsumexp(s if mask is None else s.masked_fill(~mask[b].view(1, -1), float("-inf")), -1)
+        assert ((lse[b, n].double() - want).abs() <= slack).all()
 
 
-# heads x ceil(q_len / 256) tiles over 8 XCDs: tiles per XCD 1, 1, 8, 9, 16, 17 (no round before the last),
-# 32 + 1, 32 + 8, 32 + 9, 32 + 16, 64 + 3
-CASES = [(1, 1, 385), (3, 257, 512), (64, 129, 1000), (72, 200, 513), (43, 700, 641), (136, 256, 400), (8, 2300, 2100), (264, 300, 2050),
-         (264, 193, 400), (160, 300, 577), (164, 511, 390), (128, 641, 700), (536, 65, 450)]
+# heads, q_len, kv_len, parts; heads x ceil(q_len / 256) tiles over 8 XCDs: tiles per XCD 1, 1, 8, 9, 16, 16, 17, 9 (no round
+# before the last), 64 + 2, 32 + 1, 32 + 8, 32 + 9, 32 + 16, 64 + 3
+CASES = [(1, 1, 385, 4), (3, 257, 512, 4), (64, 129, 1000, 4), (72, 200, 513, 2), (42, 700, 641, 2), (128, 250, 400, 2),
+         (136, 256, 400, 0), (8, 2300, 2100, 2), (264, 300, 2050, 4), (264, 193, 500, 4), (160, 300, 577, 4), (164, 511, 1300, 2),
+         (128, 641, 1400, 2), (536, 65, 450, 4)]
 
 
-@pytest.mark.parametrize("heads,q_len,kv_len", CASES)
+@pytest.mark.parametrize("heads,q_len,kv_len,parts", CASES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("d", [128, 64])
-def test_cut_rounds(heads, q_len, kv_len, dtype, masked, d):
+def test_cut_rounds(heads, q_len, kv_len, parts, dtype, masked, d):
     if masked and q_len < 256:
-        q_len += 256                      # key masks run on this kernel from 256 query rows on
-    print("case", heads, q_len, kv_len, dtype, masked, d, flush=True)
+        q_len = 256                       # key masks run on this kernel from 256 query rows on
+    assert kind(heads, q_len, kv_len, d, masked) == parts
     g = torch.Generator(device="cuda").manual_seed(heads + q_len)
     q, k, v = (torch.randn((1, heads, s, d), generator=g, device="cuda").to(dtype) for s in (q_len, kv_len, kv_len))
     mask = None
     if masked:
         mask = torch.rand((1, kv_len), generator=g, device="cuda") < 0.5
-        mask[:, :70] = False              # the first groups of keys and all of a group's keys in the last tile hidden
+        mask[:, :70] = False              # the first half of the first key tile and the last keys hidden
         mask[:, kv_len - kv_len % 128 - 20:] = False
         mask[:, 200] = True
     want = reference(q, k, v, mask)
@@ -81,7 +109,21 @@ def test_cut_rounds(heads, q_len, kv_len, dtype, masked, d):
     check(mindiesd.attention_forward(*t, attn_mask=m4, head_first=False).transpose(1, 2), want, v, dtype)
 
 
-# equal problems side by side: 32 + 1 and 32 + 12 tiles per XCD, 32 + 19, 64 + 2 with ragged rows, 64 without a rest and few keys
+# the cut ends at 16 whole rounds: 15 rounds and 16 tiles per XCD, 16 rounds and one (key heads shared by 128 and 152 heads)
+@pytest.mark.parametrize("heads,kv_heads,parts", [(3968, 31, 2), (4104, 27, 0)])
+@pytest.mark.parametrize("d", [128, 64])
+def test_last_cut_round(heads, kv_heads, parts, d):
+    assert kind(heads, 70, 900, d) == parts
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    q, k, v = (torch.randn((1, n, s, d), generator=g, device="cuda").bfloat16()
+               for n, s in ((heads, 70), (kv_heads, 900), (kv_heads, 900)))
+    got = flash_attention(q, k, v, d ** -0.5)
+    some = torch.arange(0, heads, 31, device="cuda")
+    kv = some // (heads // kv_heads)
+    check(got[:, some], reference(q[:, some], k[:, kv], v[:, kv]), v, torch.bfloat16)
+
+
+# equal problems side by side: 32 + 1 and 32 + 12 tiles per XCD, 32 + 18, 64 + 2 with ragged rows, 64 without a rest and few keys
 EQUAL = [(8, 8448, 640), (8, 11264, 1536), (8, 12800, 900), (264, 300, 450), (8, 16384, 512), (24, 1101, 1101)]
 
 

@@ -15,7 +15,6 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nseq", [2, 7, 64, 65])
 @pytest.mark.parametrize("on_gpu", [False, True])
 def test_longest_first(nseq, d, on_gpu):
-    print("case", nseq, d, on_gpu, flush=True)
     lens_q = [(257, 900, 1300, 256, 900, 511, 1)[i % 7] for i in range(nseq)]
     lens_k = [(700, 400, 513, 1500, 400, 0, 640)[i % 7] for i in range(nseq)]
     if nseq > 8:
