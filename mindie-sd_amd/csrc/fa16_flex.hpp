@@ -37,6 +37,15 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 
+// The kernel's argument block (its only argument), to be read where it is needed: the compiler loads what it sees as one block
+// up front and keeps it, and the bodies below then spill scalar registers into vector registers that their loops need.
+typedef const __attribute__((address_space(4))) FaParams* FaArgs;
+__device__ __forceinline__ FaArgs fa_args_here() {
+  FaArgs a = (FaArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return a;
+}
+
 // the rescale of column block nq when its reference maximum moves (see cond_rescale_fa16)
 template <int NQ>
 __device__ __forceinline__ void fa16_rescale(int flag, float delta, float alpha, float& l, f32x4_t& negm, f32x4_t& s0, f32x4_t& s1,
@@ -82,28 +91,44 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  const int Sq = p.Sq, Skv = p.Skv;
+  // the lane's number for the rarely run parts; LOOP, whose products need the registers: computed anew in each of them
+  auto lane_here = [&]() __attribute__((always_inline)) {
+    int l = lane;
+    if constexpr (LOOP) {
+      l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+      asm volatile("" : "+v"(l));
+    }
+    return l;
+  };
+  // (where the mask and head_dim 128 leave no vector register for spilled scalar ones; elsewhere a load of its own wait costs more)
+  auto args_here = [&]() __attribute__((always_inline)) {
+    if constexpr (KEYMASK && D == 128) return fa_args_here();
+    else return &p;
+  };
+  const auto a0 = args_here();
+  const int Sq = a0->Sq, Skv = a0->Skv;
+  const float scale_log2 = a0->scale_log2;
   const int row_tiles = (Sq + 255) / 256;
   int b, n, row0;  // the tile at hand: batch entry, head, first query row of the wave
-  auto locate = [&](int it, int& ib, int& in, int& irow) __attribute__((always_inline)) {
-    const int bn = it / row_tiles;
-    ib = bn / p.N;
-    in = bn - ib * p.N;
+  auto locate = [&](auto a, int it, int& ib, int& in, int& irow) __attribute__((always_inline)) {
+    const int bn = it / row_tiles, heads = a->N;
+    ib = bn / heads;
+    in = bn - ib * heads;
     irow = (it - bn * row_tiles) * 256 + first_row + wave * kWaveRows;
   };
-  locate(item, b, n, row0);
+  locate(a0, item, b, n, row0);
   const bool busy = LOOP || (wave * kWaveRows < part_rows && row0 < Sq);
 
   // ---- staging (LDS-DMA) -------------------------------------------------------------------------------------
-  const int group = p.N / p.Nkv;
-  const int k_range = (int)(((long long)(Skv - 1) * p.k_ss + D) * 2), v_range = (int)(((long long)(Skv - 1) * p.v_ss + D) * 2);
+  const int k_row_bytes = (int)a0->k_ss * 2, v_row_bytes = (int)a0->v_ss * 2;
+  const int k_range = (int)(((long long)(Skv - 1) * a0->k_ss + D) * 2), v_range = (int)(((long long)(Skv - 1) * a0->v_ss + D) * 2);
   const T *kg, *vg;
-  auto point_at_keys = [&](int ib, int in) __attribute__((always_inline)) {
-    kg = (const T*)p.k + ib * p.k_sb + (in / group) * p.k_sn;
-    vg = (const T*)p.v + ib * p.v_sb + (in / group) * p.v_sn;
+  auto point_at_keys = [&](auto a, int ib, int in) __attribute__((always_inline)) {
+    const int ikv = in / (a->N / a->Nkv);
+    kg = (const T*)a->k + ib * a->k_sb + ikv * a->k_sn;
+    vg = (const T*)a->v + ib * a->v_sb + ikv * a->v_sn;
   };
-  point_at_keys(b, n);
-  const int k_row_bytes = (int)p.k_ss * 2, v_row_bytes = (int)p.v_ss * 2;
+  point_at_keys(a0, b, n);
   int k_voff, v_voff;
   {
     const int row = kDmaRows * wave + lane / (kRowBytes / 16);  // groups of one wave lie kDmaRows * NW rows apart: same swizzles
@@ -127,14 +152,13 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
 
   // ---- Q^T operand, resident: requested here, converted at the start of its tile ------------------------------------
   X8 qf[NQ][NKS];
-  auto load_q = [&](int ib, int in, int irow) __attribute__((always_inline)) {
-    const T* qg = (const T*)p.q + ib * p.q_sb + in * p.q_sn;
-    int qc = lane & 15, qgr = lane >> 4;
-    if constexpr (LOOP) asm volatile("" : "+v"(qc), "+v"(qgr));  // (recomputed for every tile, not kept in registers)
+  auto load_q = [&](auto a, int ib, int in, int irow) __attribute__((always_inline)) {
+    const T* qg = (const T*)a->q + ib * a->q_sb + in * a->q_sn;
+    const int ql = lane_here(), qc = ql & 15, qgr = ql >> 4;
 #pragma unroll
     for (int nq = 0; nq < NQ; ++nq) {
       const int qrow = irow + nq * 16 + qc;
-      const T* src = qg + (long long)(qrow < Sq ? qrow : 0) * p.q_ss + 8 * qgr;
+      const T* src = qg + (long long)(qrow < Sq ? qrow : 0) * a->q_ss + 8 * qgr;
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) qf[nq][ks] = *(const X8*)(src + 32 * ks);
     }
@@ -156,7 +180,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
                 ((db ^ (D == 128 ? 4 * (g & 1) + (c >> 2) : ((4 * g + (c >> 2)) >> 1) & 3)) << 5) + 8 * (c & 3);
 
   const int tiles = (Skv + BN - 1) / BN;
-  load_q(b, n, row0);
+  load_q(a0, b, n, row0);
   load_tile(0, 0);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();
@@ -168,7 +192,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   auto mask_request = [&](int key0) __attribute__((always_inline)) {
     if constexpr (KEYMASK) {
       kraw = 0;
-      const int k4 = key0 + 4 * (lane & (BN / 4 - 1));
+      const int k4 = key0 + 4 * (lane_here() & (BN / 4 - 1));
       if (key0 + BN <= Skv) {
         __builtin_memcpy(&kraw, mask_g + k4, 4);  // (any alignment)
       } else {
@@ -183,8 +207,8 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
   auto mask_reduce = [&]() __attribute__((always_inline)) {
     if constexpr (KEYMASK) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        kvis[j] = (unsigned)__builtin_amdgcn_ballot_w64(lane < BN / 4 && ((kraw >> (8 * j)) & 0xffu) != 0);
+      for (int j = 0; j < 4; ++j)  // (lanes 0 .. 31; the others hold the same bytes again)
+        kvis[j] = (unsigned)__builtin_amdgcn_ballot_w64(((kraw >> (8 * j)) & 0xffu) != 0);
     }
   };
 
@@ -225,20 +249,22 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     __builtin_amdgcn_sched_barrier(0);
 
     if (key0 + BN > Skv) {  // keys past the end of the sequence (last tile only)
+      const int g4 = 4 * (lane_here() >> 4);
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (key0 + 16 * kb + 4 * g + i >= Skv) {
+          if (key0 + 16 * kb + g4 + i >= Skv) {
 #pragma unroll
             for (int nq = 0; nq < NQ; ++nq) sacc[kb][nq][i] = -INFINITY;
           }
     }
     if constexpr (KEYMASK) {
       if (kv_all != 0xffffffffu) {
+        const int mg = lane_here() >> 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const unsigned w = kvis[i] >> g;  // key 16 * kb + 4 * g + i is bit 4 * kb + g of word i
+          const unsigned w = kvis[i] >> mg;  // key 16 * kb + 4 * g + i is bit 4 * kb + g of word i
 #pragma unroll
           for (int kb = 0; kb < NKB; ++kb)
             if (!((w >> (4 * kb)) & 1u)) {
@@ -336,21 +362,21 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
 
   for (;;) {
     if constexpr (KEYMASK) {
-      mask_g = p.mask + b * p.m_sb + n * p.m_sn;
+      const auto a = args_here();
+      mask_g = a->mask + b * a->m_sb + n * a->m_sn;
       mask_request(0);
       mask_reduce();
     }
 #pragma unroll
     for (int nq = 0; nq < NQ; ++nq) {
-      int qc = c;
-      if constexpr (LOOP) asm volatile("" : "+v"(qc));
+      const int qc = lane_here() & 15;
       const bool ok = row0 + nq * 16 + qc < Sq;
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) {
         X8 v = qf[nq][ks];
         if (!ok) v = X8{0};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = E::from_float((float)v[j] * p.scale_log2);
+        for (int j = 0; j < 8; ++j) v[j] = E::from_float((float)v[j] * scale_log2);
         qf[nq][ks] = v;
       }
       l_run[nq] = 0.f;
@@ -363,26 +389,27 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     int b_nx = 0, n_nx = 0, row0_nx = 0;
     unsigned touched = 0;
     if (LOOP && more) {
-      locate(item + 32, b_nx, n_nx, row0_nx);
+      const auto a = args_here();
+      locate(a, item + 32, b_nx, n_nx, row0_nx);
       // a word of every 128-byte line of the next rows of q, so that they wait in the L2
-      const int qrow = min(row0_nx - wave * kWaveRows + (tid >> 1), Sq - 1);
-      touched = *(const unsigned*)((const T*)p.q + b_nx * p.q_sb + n_nx * p.q_sn + (long long)qrow * p.q_ss + (tid & 1) * 64);
+      const int qrow = min(row0_nx + (lane_here() >> 1), Sq - 1);
+      touched = *(const unsigned*)((const T*)a->q + b_nx * a->q_sb + n_nx * a->q_sn + (long long)qrow * a->q_ss + (lane_here() & 1) * 64);
     }
     for (int t = 0; t < tiles; t += 2) {
       tile_step(std::integral_constant<int, 0>{}, t * BN, t + 1 < tiles ? (t + 1) * BN : -1, false);
       if (t + 1 < tiles) {
         // (an even number of key tiles: the last step requests the first key tile of the next rows)
         const bool other_rows = LOOP && more && t + 2 >= tiles;
-        if (other_rows) point_at_keys(b_nx, n_nx);
+        if (other_rows) point_at_keys(args_here(), b_nx, n_nx);
         tile_step(std::integral_constant<int, 1>{}, (t + 1) * BN, t + 2 < tiles ? (t + 2) * BN : (other_rows ? 0 : -1), other_rows);
       }
     }
     if constexpr (LOOP) {
       asm volatile("" ::"v"(touched));
       if (more) {  // (an odd number: it goes into the stage of the last step, which no wave reads any more)
-        load_q(b_nx, n_nx, row0_nx);
+        load_q(args_here(), b_nx, n_nx, row0_nx);
         if (tiles & 1) {
-          point_at_keys(b_nx, n_nx);
+          point_at_keys(args_here(), b_nx, n_nx);
           load_tile(0, 0);
         }
       }
@@ -392,18 +419,19 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
     // LOOP: behind the tile stages, which already fill with the next rows' keys; otherwise in them: no wave reads them any more
     if (busy) {
       constexpr int kChunks = D / 8, kSwz = kChunks - 1;
-      T* og = (T*)p.o + b * p.o_sb + n * p.o_sn;
+      const auto a = args_here();
+      T* og = (T*)a->o + b * a->o_sb + n * a->o_sn;
+      float* lse = a->lse ? a->lse + ((long long)b * a->N + n) * Sq : nullptr;
+      const long long o_ss = a->o_ss;
       MSD_LDS char* ost = smem + (LOOP ? 4 * kTileBytes : 0) + wave * 16 * kRowBytes;
-      int oc = lane & 15, ogr = lane >> 4, ol = lane;
-      if constexpr (LOOP) asm volatile("" : "+v"(oc), "+v"(ogr), "+v"(ol));
+      const int ol = lane_here(), oc = ol & 15, ogr = ol >> 4;
 #pragma unroll
       for (int nq = 0; nq < NQ; ++nq) {
         const float l_tot = l_run[nq] + lt[nq][0];
         const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
         const int qrow_l = row0 + nq * 16 + oc;
-        if (p.lse && ogr == 0 && qrow_l < Sq)
-          p.lse[((long long)b * p.N + n) * Sq + qrow_l] =
-              l_tot > 0.f ? -negm[nq][0] * 0.6931471805599453f + __logf(l_tot) : -INFINITY;
+        if (lse && ogr == 0 && qrow_l < Sq)
+          lse[qrow_l] = l_tot > 0.f ? -negm[nq][0] * 0.6931471805599453f + __logf(l_tot) : -INFINITY;
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
           typename E::x4 pk;
@@ -416,7 +444,7 @@ __device__ __forceinline__ void fa16_flex_body(const FaParams& p, MSD_LDS char* 
         for (int i = 0; i < kChunks / 4; ++i) {
           const int row = i * (64 / kChunks) + ol / kChunks, ch = ol % kChunks, qrow = row0 + nq * 16 + row;
           const i32x4_t v = *(MSD_LDS const i32x4_t*)(ost + row * kRowBytes + ((ch ^ (row & kSwz)) << 4));
-          if (qrow < Sq) *(i32x4_t*)(og + (long long)qrow * p.o_ss + ch * 8) = v;
+          if (qrow < Sq) *(i32x4_t*)(og + (long long)qrow * o_ss + ch * 8) = v;
         }
         __builtin_amdgcn_wave_barrier();
       }

@@ -1302,9 +1302,11 @@ static int launch_fa16(const FaParams& p, hipStream_t stream) {
 // Dense attention over a few key tiles (cross attention) by one workgroup per CU that goes through its XCD's tiles of rows:
 // with four key tiles per 256 rows a launch spends 7 of 20 us per tile of rows on starting a workgroup, waiting for its
 // queries and first keys, and storing.  The last key tile's step requests the first keys of the next rows, the next
-// queries are pulled into the L2 meanwhile and requested before the output leaves.  40 heads, 32760 queries, before -> now:
-// 400 keys 384 -> 353, 512 keys 383 -> 362, 768 keys 496 -> 482 us, 1024 keys 614 -> 615; with a key mask 512 keys 414 -> 390.
-// What is left above the 12 us of the products: reading q and writing out, which all CUs do at the same moments.
+// queries are pulled into the L2 meanwhile and requested before the output leaves.  40 heads, 32760 queries, one workgroup per
+// tile -> this on one box: 400 keys 397 -> 362, 512 keys 397 -> 367, 640 keys 458 -> 448, 768 keys 517 -> 489 us, 1024 keys equal;
+// with a key mask 428 -> 385, 428 -> 380, 545 -> 502 at 400, 512, 768 keys.  Registers: the masked form reads its arguments and the
+// lane's number where it needs them, so that no vector register is spilled (6 otherwise, 386 us at 512 keys); scalar ones are, 8 of
+// them, without a mask 27, all outside the products.  What is left above the 12 us of the products per tile: reading q, writing out.
 template <int DT, bool KEYMASK>
 __global__ __launch_bounds__(512, 1) void fa16_loop_kernel(const FaParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
