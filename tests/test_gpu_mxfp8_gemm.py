@@ -64,20 +64,38 @@ def test_plain_gemm_with_bias_and_linear_module(cuda):
     assert y.shape == (2, m // 2, n) and torch.equal(y.reshape(m, n).cpu(), out)
 
 
-# one shape per tile of the GEMM's dispatch (64 x 64, 64 x 128, 128 x 128 in one and in two rounds, 256 x 256), each with rows
-# and columns past a tile's edge and K of one, of a few and of a number of blocks that four does not divide
-@pytest.mark.parametrize("m,k,nw,swiglu", [
-    (1, 128, 8, False), (65, 640, 1032, False), (64, 512, 16, True), (700, 128, 3080, False), (130, 384, 2064, True),
-    (1000, 896, 2056, False), (300, 256, 9232, True), (2100, 128, 4104, False), (1100, 640, 6160, True),
-    (4500, 128, 4104, False), (2100, 384, 8208, True)])
+def tile(m, nw, swiglu):
+    """The tile the GEMM takes, as its dispatch has it: the smallest whose grid is one round over 256 compute units, 128 x 128
+    also in two rounds against one of 256 x 256; SwiGLU halves the columns a tile covers."""
+    def count(tm, tn):
+        return -(-m // tm) * -(-(nw // 2 if swiglu else nw) // (tn // 2 if swiglu else tn))
+    if not swiglu and count(64, 64) <= 256:
+        return 64, 64
+    if count(64, 128) <= 256:
+        return 64, 128
+    return (128, 128) if count(128, 128) <= (512 if count(256, 256) <= 256 else 256) else (256, 256)
+
+
+# shapes of every tile, plain and SwiGLU, 128 x 128 in one and in two rounds; rows and columns past a tile's edge; K of one block,
+# of a few, and of 9, 11 or 13 (more than two chunks of scales, a number four does not divide)
+@pytest.mark.parametrize("m,k,nw,swiglu,want_tile", [
+    (1, 128, 8, False, (64, 64)), (65, 640, 1032, False, (64, 64)), (200, 1152, 1000, False, (64, 64)),
+    (320, 640, 3600, False, (64, 128)), (130, 1152, 6000, False, (64, 128)),
+    (64, 512, 16, True, (64, 128)), (130, 384, 2064, True, (64, 128)), (70, 1664, 1040, True, (64, 128)),
+    (700, 128, 3080, False, (128, 128)), (1000, 896, 2056, False, (128, 128)), (700, 1152, 3080, False, (128, 128)),
+    (1536, 1408, 5000, False, (128, 128)),
+    (300, 256, 9232, True, (128, 128)), (300, 1408, 9232, True, (128, 128)), (1100, 640, 6160, True, (128, 128)),
+    (2100, 128, 4104, False, (256, 256)), (4500, 128, 4104, False, (256, 256)), (2100, 640, 4104, False, (256, 256)),
+    (2305, 1152, 4616, False, (256, 256)), (2100, 384, 8208, True, (256, 256)), (2100, 1664, 8208, True, (256, 256))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_gemm_tiles_vs_oracle(cuda, m, k, nw, swiglu, dtype):
+def test_gemm_tiles_vs_oracle(cuda, m, k, nw, swiglu, want_tile, dtype):
     """Against the exact product of the quantised operands on sampled rows (all of the first and last tile's edges):
     the matrix instruction aligns its 64 products to the largest and drops what falls below (measured with the bias set to
     minus the exact result: 2^-13 of the largest product and instruction at K 128, less at larger K; twice that is allowed),
     fp32 sums of K products deviate by at most K 2^-24 sum |x w|, the output rounds by 2^-9 (bf16, half an ulp) or 2^-12
     (fp16), and silu * up carries the error of two sums."""
     from mindiesd.layers.quant import mx_quantize, mxfp8_matmul
+    assert tile(m, nw, swiglu) == want_tile
     x, w, bias = _rand((m, k), 11), _rand((nw, k), 12, scale=0.05), _rand((nw,), 13, dtype=torch.float32)
     xq, xs = mx_quantize(x.to(cuda))
     wq, ws = mx_quantize(w.to(cuda))
