@@ -696,8 +696,8 @@ int mindiesd_mxfp8_gemm(const void* a, const void* a_scale, const void* w, const
   // Tile choice.  A workgroup walks all of K whatever its tile, so a launch takes (rounds over the 256 CUs) x (time of a
   // tile): 64 x 64, 64 x 128, 128 x 128 and 256 x 256 tiles take 4.9 / 7.0 / 10 / 26 us at K 1536, 8 / 11 / 15.5 / 38.5 us at
   // K 3072 and 12 / 17.5 / 23.5 / 57 us at K 5120.  Hence the smallest tile whose grid is one round; 128 x 128 tiles still win
-  // in two rounds against one round of 256 x 256 (M 1024, N K 5120: 47 against 58 us), not in three (M 1536: 52 against 59 us
-  // with 480 tiles, M 2048: 82 against 61 us with 640).
+  // in two rounds against one round of 256 x 256 (N K 5120, M 1024: 47 against 58 us, M 1536, 480 tiles: 52 against 59), not in
+  // three (M 2048, 640 tiles: 82 against 61 us).
   auto count = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((p.Nout + (swiglu ? tn / 2 : tn) - 1) / (swiglu ? tn / 2 : tn)); };
   int tm = 256, tn = 256;
   if (!swiglu && count(64, 64) <= kCUs) tm = tn = 64;
