@@ -27,16 +27,6 @@ namespace msd {
 constexpr int kFa16LoopLds = 4 * 128 * 256 + 8 * 16 * 256;
 
 #if defined(__HIP_DEVICE_COMPILE__)
-template <int... I, class F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>)
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
-}
-
 // The kernel's argument block (its only argument), to be read where it is needed: the compiler loads what it sees as one block
 // up front and keeps it, and the bodies below then spill scalar registers into vector registers that their loops need.
 typedef const __attribute__((address_space(4))) FaParams* FaArgs;

@@ -32,20 +32,6 @@
 
 namespace msd {
 
-#if defined(__HIP_DEVICE_COMPILE__)
-namespace d256 {
-template <int... I, class F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>)
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
-}
-}  // namespace d256
-#endif
-
 constexpr int kD256Waves = 8, kD256BN = 64, kD256RowBytes = 512;
 constexpr int kD256TileBytes = kD256BN * kD256RowBytes;  // 32 KiB
 constexpr int kD256Lds = 4 * kD256TileBytes;              // two K and two V stages
@@ -59,7 +45,6 @@ constexpr int kD256Ahead = FA16_D256_AHEAD;               // K operand groups re
 template <int DT, bool DPAD, int GEN = 0>
 __global__ __launch_bounds__(kD256Waves * 64, 1) void fa_fwd16_d256_kernel(const FaParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  using namespace d256;
   using E = Elem<DT>;
   using T = typename E::type;
   using X8 = typename E::x8;

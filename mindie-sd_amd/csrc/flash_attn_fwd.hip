@@ -1417,7 +1417,6 @@ extern "C" {
 #ifndef MSD_SHORT_KV
 #define MSD_SHORT_KV 384
 #endif
-constexpr int kCus = 256;  // compute units of the MI355X
 constexpr int kShortKv = MSD_SHORT_KV;  // dense calls with at most this many keys run on the 4-wave kernel (see below)
 // general mode: query rows (of the longest sequence; packed: of the average one) from which the 8-wave kernel is used
 #ifndef MSD_GEN16_MIN_ROWS

@@ -27,18 +27,6 @@ namespace msd {
 
 constexpr float kE4M3MaxMx = 448.0f;
 
-#if defined(__HIP_DEVICE_COMPILE__)
-template <int... I, class F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>)
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
-}
-#endif
-
 // ---- MX quantisation of a [M][K] 16-bit matrix along K -----------------------------------------------------
 // 4 lanes share one 32-element block (8 elements = 16 bytes each).
 template <int DT>
@@ -655,8 +643,6 @@ __global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_smal
 
 using namespace msd;
 
-constexpr int kCUs = 256;
-
 extern "C" {
 
 int mindiesd_mx_quant(const void* x, void* q, void* e8m0, int dtype, long long M, int K, long long x_stride,
@@ -700,9 +686,9 @@ int mindiesd_mxfp8_gemm(const void* a, const void* a_scale, const void* w, const
   // three (M 2048, 640 tiles: 82 against 61 us).
   auto count = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((p.Nout + (swiglu ? tn / 2 : tn) - 1) / (swiglu ? tn / 2 : tn)); };
   int tm = 256, tn = 256;
-  if (!swiglu && count(64, 64) <= kCUs) tm = tn = 64;
-  else if (count(64, 128) <= kCUs) tm = 64, tn = 128;
-  else if (count(128, 128) <= (count(256, 256) <= kCUs ? 2 * kCUs : kCUs)) tm = tn = 128;
+  if (!swiglu && count(64, 64) <= kCus) tm = tn = 64;
+  else if (count(64, 128) <= kCus) tm = 64, tn = 128;
+  else if (count(128, 128) <= (count(256, 256) <= kCus ? 2 * kCus : kCus)) tm = tn = 128;
   p.tiles_m = (M + tm - 1) / tm;
   p.tiles_n = swiglu ? (p.Nout + tn / 2 - 1) / (tn / 2) : (Nw + tn - 1) / tn;
   const int total = p.tiles_m * p.tiles_n;
