@@ -431,11 +431,12 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
 // while the matrix core works on the current one (two register sets).
 //
 // What bounds it: a tile of 128 x 128 takes 0.30 us per K block where its 8 matrix instructions take 0.22 (operands in the
-// L2; with its requests in one burst at the end of the step it was 0.39), and 0.5 us when the operands come from the
-// memory-side cache: a CU alone draws 55 to 70 GB/s from there, and neither deeper prefetch into the L2 by a fifth wave nor
-// a split of K over several workgroups (fp32 sums through memory, 29 to 47 us at 512 x 5120 x 5120) was faster.  Plain GEMM,
-// M x N x K, 256 x 256 tiles before -> now: 512 x 5120 x 5120 57.5 -> 23.8 us, 128 x 5120 x 5120 51.5 -> 12.4 us,
-// 64 x 1536 x 1536 19.5 -> 4.9 us.
+// L2; with its requests in one burst at the end of the step it was 0.39), and 0.5 us when the operands come from behind it:
+// 512 x 5120 x 5120 draws 55 GB/s through its L2 on each of 160 CUs, 18 % of the requests miss (48.8 MB for 29.7 MB of operands),
+// the matrix pipe is busy 30 % of those CUs' cycles.  Neither deeper prefetch into the L2 by a fifth wave nor a split of K over
+// several workgroups (fp32 sums through memory, 29 to 47 us) was faster.  Plain GEMM, M x N x K, 256 x 256 tiles before -> now:
+// 512 x 5120 x 5120 57.5 -> 23.8 us, 128 x 5120 x 5120 51.5 -> 12.4 us, 64 x 1536 x 1536 19.5 -> 4.9 us, the weights in the
+// memory-side cache; the layer with its quantisation 62.7 -> 29.6 us at 512 x 5120 x 5120, and 70.7 -> 37.4 with weights in no cache.
 template <int DT, bool SWIGLU, int TM, int TN>
 __global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_small_kernel(const GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
