@@ -699,6 +699,8 @@ __global__ __launch_bounds__(NWAVES * 64, (QPW == 32 ? 2 : 1)) void fa_fwd_kerne
 // query operand is zero from p.head_dim on, and the lanes that would stage the 16-byte chunks of K and V past it
 // request an offset beyond the buffers' range instead, for which the DMA writes zeros without touching memory.  The
 // output columns past p.head_dim are not stored.
+//
+// TAIL (GEN 0 and 3): the tiles of an XCD's run from p.tail_full on go as TAIL (2 or 4) workgroups each (fa16_flex.hpp).
 template <int DT, int NWAVES = 8, bool PAIR = false, bool GATHER = false, int GEN = 0, bool DPAD = false,
           int TAIL = 0>
 __global__ __launch_bounds__(NWAVES * 64, 1) void fa_fwd16_kernel(const FaParams p) {
@@ -1303,7 +1305,7 @@ static int launch_fa16(const FaParams& p, hipStream_t stream) {
 // with four key tiles per 256 rows a launch spends 7 of 20 us per tile of rows on starting a workgroup, waiting for its
 // queries and first keys, and storing.  The last key tile's step requests the first keys of the next rows, the next
 // queries are pulled into the L2 meanwhile and requested before the output leaves.  40 heads, 32760 queries, one workgroup per
-// tile -> this on one box: 400 keys 397 -> 362, 512 keys 397 -> 367, 640 keys 458 -> 448, 768 keys 517 -> 489 us, 1024 keys equal;
+// tile -> this on one card: 400 keys 397 -> 362, 512 keys 397 -> 367, 640 keys 458 -> 448, 768 keys 517 -> 489 us, 1024 keys equal;
 // with a key mask 428 -> 385, 428 -> 380, 545 -> 502 at 400, 512, 768 keys.  Registers: the masked form reads its arguments and the
 // lane's number where it needs them, so that no vector register is spilled (6 otherwise, 386 us at 512 keys); scalar ones are, 8 of
 // them, without a mask 27, all outside the products.  What is left above the 12 us of the products per tile: reading q, writing out.
