@@ -322,6 +322,14 @@ int mindiesd_mx_quant(const void* x, void* q, void* e8m0, int dtype, long long M
 int mindiesd_mxfp8_gemm(const void* a, const void* a_scale, const void* w, const void* w_scale, const float* bias,
                         void* out, int out_dtype, int M, int K, int Nw, int swiglu, hipStream_t stream);
 
+/* mindiesd_mx_quant of x [M][K] (16-bit, row stride x_stride) into a / a_scale, then mindiesd_mxfp8_gemm on them: the
+ * linear layer with dynamically quantised activations (W8A8MXFP8QuantLinear, mindiesd/quantization/layer.py:334-361) as
+ * one call.  a (M * K bytes) and a_scale (M * K/32 bytes) are scratch; nothing is launched unless both calls' arguments
+ * are in order. */
+int mindiesd_mxfp8_linear(const void* x, int x_dtype, long long x_stride, void* a, void* a_scale, const void* w,
+                          const void* w_scale, const float* bias, void* out, int out_dtype, int M, int K, int Nw,
+                          int swiglu, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

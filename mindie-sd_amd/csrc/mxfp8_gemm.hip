@@ -646,11 +646,16 @@ using namespace msd;
 
 extern "C" {
 
-int mindiesd_mx_quant(const void* x, void* q, void* e8m0, int dtype, long long M, int K, long long x_stride,
-                      hipStream_t stream) {
+static int check_mx_quant(const void* x, const void* q, const void* e8m0, int dtype, long long M, int K, long long x_stride) {
   if (!x || !q || !e8m0 || M <= 0 || K <= 0) return MSD_ERR_BAD_ARG;
   if (K % 32 != 0 || x_stride % 8 != 0 || ((uintptr_t)x & 15) || ((uintptr_t)q & 7)) return MSD_ERR_BAD_ARG;
-  if (dtype != MSD_DTYPE_BF16 && dtype != MSD_DTYPE_F16) return MSD_ERR_BAD_ARG;
+  return dtype == MSD_DTYPE_BF16 || dtype == MSD_DTYPE_F16 ? MSD_OK : MSD_ERR_BAD_ARG;
+}
+
+int mindiesd_mx_quant(const void* x, void* q, void* e8m0, int dtype, long long M, int K, long long x_stride,
+                      hipStream_t stream) {
+  const int rc = check_mx_quant(x, q, e8m0, dtype, M, K, x_stride);
+  if (rc != MSD_OK) return rc;
   const long long chunks = M * (K / 8);
   const unsigned grid = (unsigned)((chunks + 255) / 256);
   if (dtype == MSD_DTYPE_BF16)
@@ -662,19 +667,25 @@ int mindiesd_mx_quant(const void* x, void* q, void* e8m0, int dtype, long long M
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
 }
 
-// out[M][Nout] = act(X W^T + bias); swiglu != 0: W = [gate rows | up rows], Nout = Nw/2,
-// out = silu(gate) * up; otherwise Nout = Nw.
-int mindiesd_mxfp8_gemm(const void* a, const void* a_scale, const void* w, const void* w_scale, const float* bias,
-                        void* out, int out_dtype, int M, int K, int Nw, int swiglu, hipStream_t stream) {
+static int check_gemm(const void* a, const void* a_scale, const void* w, const void* w_scale, const void* out, int out_dtype,
+                      int M, int K, int Nw, int swiglu) {
   if (!a || !a_scale || !w || !w_scale || !out || M <= 0 || K <= 0 || Nw <= 0) return MSD_ERR_BAD_ARG;
   if (K % 128 != 0) return MSD_ERR_UNSUPPORTED;
-  if (swiglu && (Nw % 16 != 0)) return MSD_ERR_UNSUPPORTED;
-  if (!swiglu && (Nw % 8 != 0)) return MSD_ERR_UNSUPPORTED;
+  if (Nw % (swiglu ? 16 : 8) != 0) return MSD_ERR_UNSUPPORTED;
   if (out_dtype != MSD_DTYPE_BF16 && out_dtype != MSD_DTYPE_F16) return MSD_ERR_BAD_ARG;
   if (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) return MSD_ERR_BAD_ARG;
   if (((uintptr_t)a_scale | (uintptr_t)w_scale) & 3) return MSD_ERR_BAD_ARG;
   // 32-bit buffer offsets
   if ((long long)(M + 256) * K >= (1ll << 31) || (long long)(Nw + 256) * K >= (1ll << 31)) return MSD_ERR_UNSUPPORTED;
+  return MSD_OK;
+}
+
+// out[M][Nout] = act(X W^T + bias); swiglu != 0: W = [gate rows | up rows], Nout = Nw/2,
+// out = silu(gate) * up; otherwise Nout = Nw.
+int mindiesd_mxfp8_gemm(const void* a, const void* a_scale, const void* w, const void* w_scale, const float* bias,
+                        void* out, int out_dtype, int M, int K, int Nw, int swiglu, hipStream_t stream) {
+  const int rc = check_gemm(a, a_scale, w, w_scale, out, out_dtype, M, K, Nw, swiglu);
+  if (rc != MSD_OK) return rc;
   GemmParams p{};
   p.a = (const unsigned char*)a; p.as = (const unsigned char*)a_scale;
   p.w = (const unsigned char*)w; p.ws = (const unsigned char*)w_scale;
@@ -711,6 +722,16 @@ int mindiesd_mxfp8_gemm(const void* a, const void* a_scale, const void* w, const
   };
   return out_dtype == MSD_DTYPE_BF16 ? pick(std::integral_constant<int, MSD_DTYPE_BF16>{})
                                      : pick(std::integral_constant<int, MSD_DTYPE_F16>{});
+}
+
+int mindiesd_mxfp8_linear(const void* x, int x_dtype, long long x_stride, void* a, void* a_scale, const void* w,
+                          const void* w_scale, const float* bias, void* out, int out_dtype, int M, int K, int Nw,
+                          int swiglu, hipStream_t stream) {
+  int rc = check_mx_quant(x, a, a_scale, x_dtype, M, K, x_stride);
+  if (rc == MSD_OK) rc = check_gemm(a, a_scale, w, w_scale, out, out_dtype, M, K, Nw, swiglu);
+  if (rc == MSD_OK) rc = mindiesd_mx_quant(x, a, a_scale, x_dtype, M, K, x_stride, stream);
+  if (rc == MSD_OK) rc = mindiesd_mxfp8_gemm(a, a_scale, w, w_scale, bias, out, out_dtype, M, K, Nw, swiglu, stream);
+  return rc;
 }
 
 }  // extern "C"

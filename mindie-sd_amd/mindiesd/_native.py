@@ -52,6 +52,7 @@ SIGNATURES = {
     "mindiesd_fp8_attention_fwd": (c_int, [c_p] * 7 + [c_int] * 6 + [c_ll] * 3 + [c_f, c_int, c_p]),
     "mindiesd_mx_quant": (c_int, [c_p, c_p, c_p, c_int, c_ll, c_int, c_ll, c_p]),
     "mindiesd_mxfp8_gemm": (c_int, [c_p] * 6 + [c_int] * 5 + [c_p]),
+    "mindiesd_mxfp8_linear": (c_int, [c_p, c_int, c_ll] + [c_p] * 6 + [c_int] * 5 + [c_p]),
 }
 
 

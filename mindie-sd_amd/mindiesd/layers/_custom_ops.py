@@ -381,11 +381,8 @@ def _fp8_attention_fwd_fake(query, key, value, scale_value=1.0, input_layout="BN
 def _mxfp8_gemm_swiglu_impl(x, weight, weight_scale, bias=None, swiglu=True):
     """x [.., K] bf16/fp16 (quantised here, per 32 values along K), weight E4M3 [Nw, K] with E8M0 scales
     [Nw, K/32]; ``swiglu``: weight rows are [gate | up] and the result is silu(gate) * up [.., Nw/2]."""
-    from .quant.mxfp8 import mx_quantize, mxfp8_matmul
-    x2 = x.reshape(-1, x.shape[-1])
-    xq, xs = mx_quantize(x2)
-    out = mxfp8_matmul(xq, xs, weight, weight_scale, bias, x.dtype, swiglu)
-    return out.view(*x.shape[:-1], out.shape[-1])
+    from .quant.mxfp8 import mxfp8_linear
+    return mxfp8_linear(x, weight, weight_scale, bias, x.dtype, swiglu)
 
 
 @register_ops.register_mindie_fake_op("mxfp8_gemm_swiglu")

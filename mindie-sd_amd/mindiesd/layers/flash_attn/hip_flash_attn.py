@@ -25,6 +25,11 @@ def _strides_bns(t, layout):
 
 
 def _check_qkv(query, key, value):
+    dtype, d = query.dtype, query.shape[-1]
+    if (query.is_cuda and key.is_cuda and value.is_cuda and dtype in _native.DTYPE_CODE and key.dtype is dtype
+            and value.dtype is dtype and d % 8 == 0 and 0 < d <= MAX_HEAD_DIM and key.shape[-1] == d
+            and value.shape[-1] == d):
+        return
     for name, t in (("query", query), ("key", key), ("value", value)):
         if not t.is_cuda:
             raise ParametersInvalid(f"The fused attention kernel needs GPU tensors, but {name} is on {t.device}.")
@@ -47,6 +52,15 @@ def _aligned(t):
     return t
 
 
+def _aligned_bns(t, layout):
+    """A 4-D tensor as the kernels take it (copied if it has to be), and its (batch, head, token) element strides."""
+    s0, s1, s2, s3 = t.stride()
+    if s3 != 1 or (s0 | s1 | s2) & 7 or t.data_ptr() & 15:
+        t = t.contiguous()
+        s0, s1, s2, _ = t.stride()
+    return t, ((s0, s1, s2) if layout == "BNSD" else (s0, s2, s1))
+
+
 def flash_attention(query, key, value, scale, layout="BNSD", return_lse=False, attn_mask=None, causal=False):
     """softmax(scale * Q K^T) V on the GPU.  ``layout`` is 'BNSD' or 'BSND'; the output has the
     input's layout and dtype.  Grouped-query attention is supported (N % N_kv == 0).
@@ -64,18 +78,22 @@ def flash_attention(query, key, value, scale, layout="BNSD", return_lse=False, a
         skv, nkv = key.shape[1], key.shape[2]
     if key.shape != value.shape or key.shape[0] != b or n % nkv != 0:
         raise ParametersInvalid("Inconsistent query/key/value shapes.")
-    query, key, value = _aligned(query), _aligned(key), _aligned(value)
-    out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
-    lse = torch.empty((b, n, sq), dtype=torch.float32, device=query.device) if return_lse else None
-    strides = (*_strides_bns(query, layout), *_strides_bns(key, layout), *_strides_bns(value, layout),
-               *_strides_bns(out, layout))
-    with _native.on_device(query.device):
+    device = query.device
+    query, q_st = _aligned_bns(query, layout)
+    key, k_st = _aligned_bns(key, layout)
+    value, v_st = _aligned_bns(value, layout)
+    out = torch.empty_like(query, memory_format=torch.contiguous_format)
+    o_st = (n * sq * d, sq * d, d) if layout == "BNSD" else (n * sq * d, d, n * d)
+    lse = torch.empty((b, n, sq), dtype=torch.float32, device=device) if return_lse else None
+    strides = (*q_st, *k_st, *v_st, *o_st)
+    with _native.on_device(device):
         if attn_mask is None and not causal:
             rc = _native.lib().mindiesd_flash_attention_fwd(
                 query.data_ptr(), key.data_ptr(), value.data_ptr(), out.data_ptr(),
                 lse.data_ptr() if lse is not None else None, _native.DTYPE_CODE[query.dtype],
-                b, n, nkv, sq, skv, d, *strides, float(scale), _native.stream_ptr(query.device))
-            _native.check(rc, "mindiesd_flash_attention_fwd")
+                b, n, nkv, sq, skv, d, *strides, float(scale), _native.stream_ptr(device))
+            if rc:
+                _native.check(rc, "mindiesd_flash_attention_fwd")
         else:
             mask, m_sb, m_sn, m_sq = None, 0, 0, 0
             if attn_mask is not None:

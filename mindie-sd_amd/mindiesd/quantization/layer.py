@@ -3,7 +3,7 @@ import torch
 from torch import nn
 
 from ..layers.quant.fp8_attention import fp8_attention_forward
-from ..layers.quant.mxfp8 import mx_quantize, mxfp8_matmul
+from ..layers.quant.mxfp8 import mxfp8_linear
 from ..utils.exception import ParametersInvalid
 
 
@@ -72,10 +72,13 @@ class W8A8MXFP8QuantLinear(nn.Module):
             x = x.to(self.dtype)
         if self.mul_scale is not None:
             x = x * self.mul_scale
-        x1, input_scale = mx_quantize(x)
-        return mxfp8_matmul(x1, input_scale, self.weight, self.weight_scale, self.bias, self.dtype, self.swiglu)
+        if x.dim() != 2:
+            raise ParametersInvalid("mx_quantize needs a 2-D bf16/fp16 GPU tensor.")
+        return mxfp8_linear(x, self.weight, self.weight_scale, self.bias, self.dtype, self.swiglu)
 
     def forward(self, x):
+        if x.ndim >= 3 and self.mul_scale is None and x.dtype == self.dtype:
+            return mxfp8_linear(x, self.weight, self.weight_scale, self.bias, self.dtype, self.swiglu)
         if x.ndim >= 3:  # the reference flattens to 2-D as well (layer.py:104-116)
             out = self.quant_matmul(x.reshape(x.shape[:-1].numel(), -1))
             return out.view(*x.shape[:-1], out.shape[1])

@@ -166,3 +166,44 @@ def test_quantize_injected_layers_match_direct_calls(cuda, tmp_path):
     a = model.attn.fa_quant(q, k, v, layout="BNSD")
     b = fp8_attention_forward(q, k, v, layout="BNSD", q_rot=rot.to(cuda), k_rot=rot.to(cuda))
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("form", ["2d", "4d", "1d", "row_stride", "column_stride", "transposed"])
+def test_linear_in_one_call_equals_quantise_then_multiply(cuda, form):
+    """``mxfp8_linear`` on every form of x that needs another way to its rows, with and without SwiGLU and bias: the bits of
+    ``mx_quantize`` followed by ``mxfp8_matmul``."""
+    from mindiesd.layers.quant.mxfp8 import mx_quantize, mxfp8_linear, mxfp8_matmul
+    g = torch.Generator().manual_seed(5)
+    rnd = lambda *shape: torch.randn(shape, generator=g).to(torch.bfloat16).to(cuda)
+    x = {"2d": lambda: rnd(70, 256), "4d": lambda: rnd(2, 5, 7, 256), "1d": lambda: rnd(256),
+         "row_stride": lambda: rnd(70, 264)[:, :256], "column_stride": lambda: rnd(70, 512)[:, ::2],
+         "transposed": lambda: rnd(7, 10, 256).transpose(0, 1)}[form]()
+    wq, ws = mx_quantize(rnd(528, 256))
+    bias = torch.randn(528, generator=g).to(torch.float16).to(cuda)
+    xq, xs = mx_quantize(x.reshape(-1, 256))
+    for swiglu in (False, True):
+        for b in (None, bias):
+            want = mxfp8_matmul(xq, xs, wq, ws, b, torch.float16, swiglu)
+            got = mxfp8_linear(x, wq, ws.reshape(528, -1, 2), b, torch.float16, swiglu)
+            assert got.shape == (*x.shape[:-1], want.shape[1]) and torch.equal(got.view(want.shape), want)
+
+
+def test_linear_in_one_call_refuses_what_its_parts_refuse(cuda):
+    import mindiesd
+    from mindiesd.layers.quant.mxfp8 import mx_quantize, mxfp8_linear
+    x = torch.ones(4, 256, dtype=torch.bfloat16, device=cuda)
+    wq, ws = mx_quantize(x.repeat(2, 1))
+    refused = mindiesd.ParametersInvalid
+    for bad in (lambda: mxfp8_linear(x.cpu(), wq, ws), lambda: mxfp8_linear(x.float(), wq, ws),
+                lambda: mxfp8_linear(x[:, :40], wq[:, :40], ws), lambda: mxfp8_linear(x[:, :160], wq[:, :160], ws),
+                lambda: mxfp8_linear(x, wq[:, :128], ws), lambda: mxfp8_linear(x, wq[:4], ws[:4]),
+                lambda: mxfp8_linear(x, wq, ws, out_dtype=torch.float32), lambda: mxfp8_linear(x, wq, ws, swiglu=True),
+                lambda: mxfp8_linear(x, wq.cpu(), ws), lambda: mxfp8_linear(x, wq, ws, torch.ones(7, device=cuda))):
+        with pytest.raises(refused):
+            bad()
+    with pytest.raises(RuntimeError):
+        mxfp8_linear(x, wq, ws[:, :4])       # fewer scales than the weight has blocks
+    for bad in (x[:0], torch.ones(1028, dtype=torch.bfloat16, device=cuda)[4:].view(4, 256)):     # empty; not 16-byte aligned
+        for call in (lambda: mxfp8_linear(bad, wq, ws), lambda: mx_quantize(bad)):
+            with pytest.raises(RuntimeError):
+                call()
