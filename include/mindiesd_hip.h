@@ -306,6 +306,18 @@ int mindiesd_fp8_attention_fwd(const void* q8, const void* k8, const void* v8t, 
                                int Sq, int Skv, int D, long long o_sb, long long o_sn, long long o_ss, float scale,
                                int flags, hipStream_t stream);
 
+/* The FP8 attention module on 16-bit tensors as one call of three launches: q and k rotated by q_rot / k_rot ([128][128] row
+ * major, the tensors' type; NULL: not rotated) and quantised per (head, 128 tokens), v quantised per (head, channel), then
+ * attention; out in the tensors' type.  Same bits as mindiesd_fa_rot_block_quant / mindiesd_fa_block_quant,
+ * mindiesd_fp8_v_quant and mindiesd_fp8_attention_fwd one after another (FP8RotateQuantFA.forward,
+ * mindiesd/quantization/layer.py:283-324).  flags: 0 or MSD_FP8_P_EXP2.  workspace: codes and scales, 16-byte aligned. */
+size_t mindiesd_fp8_rot_attention_workspace_size(int B, int N, int Sq, int Skv);
+int mindiesd_fp8_rot_attention_fwd(const void* q, const void* k, const void* v, const void* q_rot, const void* k_rot, void* out,
+                                   int dtype, int B, int N, int Sq, int Skv, int D, long long q_sb, long long q_sn,
+                                   long long q_ss, long long k_sb, long long k_sn, long long k_ss, long long v_sb,
+                                   long long v_sn, long long v_ss, long long o_sb, long long o_sn, long long o_ss, float scale,
+                                   int flags, void* workspace, size_t ws_bytes, hipStream_t stream);
+
 /* ---- MXFP8 linear layer --------------------------------------------------------------------------------
  * x [M][K] 16-bit (row stride x_stride elements) -> q [M][K] E4M3 + e8m0 [M][K/32]
  * (OCP MX: shared scale 2^(floor(log2(amax)) - 8) per 32 elements).  Replaces

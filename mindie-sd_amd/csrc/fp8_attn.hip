@@ -113,21 +113,15 @@ __global__ __launch_bounds__(256) void block_quant_kernel(const void* x_, unsign
 #endif
 }
 
+#if defined(__HIP_DEVICE_COMPILE__)
 // The same for blocks of BS = 128 or 256 tokens with the block held in registers: a thread requests its
 // BS / 16 rows x 8 channels at once (more requests in flight than the row loop above) and quantises them without a
-// second read.
+// second read.  x, q: the (batch, head) problem's rows; scale: the block's entry.
 template <int DT, int BS>
-__global__ __launch_bounds__(256) void block_quant_reg_kernel(const void* x_, unsigned char* q, float* scale,
-                                                             long long sb, long long sn, long long ss, int N, int S,
-                                                             float prescale, int pow2) {
-#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ void block_quant_body(const typename Elem<DT>::type* x, unsigned char* q, float* scale, long long ss,
+                                                 int S, int blk, float prescale, int pow2, float* red) {
   using T = typename Elem<DT>::type;
   constexpr int kRows = BS / 16;  // rows per thread
-  __shared__ float red[4];
-  const int blk = blockIdx.x, bn = blockIdx.y;
-  const int b = bn / N, n = bn - b * N;
-  const int nblk = gridDim.x;
-  const T* x = (const T*)x_ + b * sb + n * sn;
   const int row0 = blk * BS, rows = min(BS, S - row0);
   const int c16 = threadIdx.x & 15, rgrp = threadIdx.x >> 4;
   union { i32x4_t v; T e[8]; } u[kRows];
@@ -144,8 +138,8 @@ __global__ __launch_bounds__(256) void block_quant_reg_kernel(const void* x_, un
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(__fmul_rn((float)u[i].e[j], prescale)));
   amax = block_max_256(amax, red);
   const float sc = block_scale(amax, pow2);
-  if (threadIdx.x == 0) scale[(long long)bn * nblk + blk] = sc;
-  unsigned char* qo = q + ((long long)bn * S + row0) * 128 + c16 * 8;
+  if (threadIdx.x == 0) *scale = sc;
+  unsigned char* qo = q + (long long)row0 * 128 + c16 * 8;
 #pragma unroll
   for (int i = 0; i < kRows; ++i) {
     const int r = rgrp + 16 * i;
@@ -155,42 +149,32 @@ __global__ __launch_bounds__(256) void block_quant_reg_kernel(const void* x_, un
     const i32x2_t w = {pack4_e4m3(f[0], f[1], f[2], f[3]), pack4_e4m3(f[4], f[5], f[6], f[7])};
     if (r < rows) *(i32x2_t*)(qo + (long long)r * 128) = w;
   }
-#endif
 }
 
 // ---- rotation + block quantisation in one pass ------------------------------------------------------------------
 // y = x @ R (R a fixed [128][128] matrix, e.g. a Hadamard rotation that spreads outliers over the channels),
 // y rounded to the 16-bit input type as a separate matmul would leave it, then quantised like
-// block_quant_kernel with 128-token blocks.  x is read once and only the E4M3 codes are written: 3 bytes
+// block_quant_body with 128-token blocks.  x is read once and only the E4M3 codes are written: 3 bytes
 // per element instead of the 7 of matmul + quantisation.
-// One workgroup = one 128-token block; R^T sits in LDS (16-byte chunk c of row n at chunk c ^ (n & 15)); wave w
-// owns tokens 32w..32w+31.  R^T is the first matrix operand, so a lane holds one token and, per register
-// quad, four consecutive output channels = one dword of codes.
-// (launch bounds: at least 4 waves per SIMD = 128 registers per lane, so that the four workgroups whose LDS fits a CU
-// are resident together - the pass is bound by memory latency)
-template <int DT>
-__global__ __launch_bounds__(256, 4) void rot_block_quant_kernel(const void* x_, const void* rot_t_, unsigned char* q,
-                                                              float* scale, long long sb, long long sn, long long ss,
-                                                              int N, int S, float prescale, int pow2) {
-#if defined(__HIP_DEVICE_COMPILE__)
+// One workgroup = one 128-token block; wave w owns tokens 32w..32w+31.  R^T is the first matrix operand, so a lane holds
+// one token and, per register quad, four consecutive output channels = one dword of codes.
+// TRANSPOSED: `rot` is R^T, 16-byte chunk c of its row n sits in LDS at chunk c ^ (n & 15).  Otherwise it is R itself and the
+// operand comes out of its rows by transposing reads: 64-byte chunk c of row k at chunk c ^ (k & 3), so that the 4 rows of a
+// quarter-wave's read lie in different banks.  The matrix instruction gets the same operands either way.
+template <int DT, bool TRANSPOSED>
+__device__ __forceinline__ void rot_block_body(const typename Elem<DT>::type* x, const void* rot, unsigned char* q, float* scale,
+                                               long long ss, int S, int blk, float prescale, int pow2, char* r_lds, float* red) {
   using E = Elem<DT>;
-  using T = typename E::type;
   using X8 = typename E::x8;
-  __shared__ __attribute__((aligned(16))) char rt_lds[128 * 256];
-  __shared__ float red[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, h = lane >> 5;
-  const int blk = blockIdx.x, bn = blockIdx.y;
-  const int b = bn / N, n = bn - b * N;
-  const int nblk = gridDim.x;
-  const T* x = (const T*)x_ + b * sb + n * sn;
   const int row0 = blk * 128;
-  // R^T [out channel][in channel] -> LDS
-  const char* rt = (const char*)rot_t_;
+  const char* rg = (const char*)rot;
 #pragma unroll
   for (int pass = 0; pass < 8; ++pass) {
     const int row = pass * 16 + (tid >> 4), c = tid & 15;
-    *(i32x4_t*)(rt_lds + row * 256 + ((c ^ (row & 15)) << 4)) = *(const i32x4_t*)(rt + row * 256 + c * 16);
+    const int at = TRANSPOSED ? c ^ (row & 15) : c ^ ((row & 3) << 2);
+    *(i32x4_t*)(r_lds + row * 256 + (at << 4)) = *(const i32x4_t*)(rg + row * 256 + c * 16);
   }
   // this lane's token: in channels 16ks + 8h .. +7 for ks = 0..7
   const int tok = row0 + wave * 32 + l32;
@@ -202,6 +186,8 @@ __global__ __launch_bounds__(256, 4) void rot_block_quant_kernel(const void* x_,
     if (!ok) xf[ks] = X8{0};
   }
   __syncthreads();
+  const int k4 = (lane & 15) >> 2;  // the row of four that this lane points at
+  const char* r_tr = r_lds + (8 * h + k4) * 256 + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
   f32x16_t acc[4];
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb) {
@@ -210,7 +196,15 @@ __global__ __launch_bounds__(256, 4) void rot_block_quant_kernel(const void* x_,
     const int row = nb * 32 + l32;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      const X8 rf = *(const X8*)(rt_lds + row * 256 + (((2 * ks + h) ^ (row & 15)) << 4));
+      X8 rf;
+      if constexpr (TRANSPOSED) {
+        rf = *(const X8*)(r_lds + row * 256 + (((2 * ks + h) ^ (row & 15)) << 4));
+      } else {  // rows 16ks + 8h + 0..3 and + 4..7, columns 32nb + l32
+        union { s16x4_t s[2]; X8 x; } u;
+        u.s[0] = lds_read_tr16(r_tr + 16 * ks * 256 + ((nb ^ k4) << 6));
+        u.s[1] = lds_read_tr16(r_tr + (16 * ks + 4) * 256 + ((nb ^ k4) << 6));
+        rf = u.x;
+      }
       acc[nb] = E::mfma32(rf, xf[ks], acc[nb]);
     }
   }
@@ -225,8 +219,8 @@ __global__ __launch_bounds__(256, 4) void rot_block_quant_kernel(const void* x_,
     }
   amax = block_max_256(amax, red);
   const float sc = block_scale(amax, pow2);
-  if (tid == 0) scale[(long long)bn * nblk + blk] = sc;
-  // The codes of a token (128 bytes) are spread over the lanes in dwords; they go through LDS (R^T is no longer
+  if (tid == 0) *scale = sc;
+  // The codes of a token (128 bytes) are spread over the lanes in dwords; they go through LDS (R is no longer
   // needed: block_max_256 has synchronised the workgroup after the last matrix instruction) so that the stores to
   // global memory are whole 16-byte chunks of consecutive rows.  16-byte chunk c of token row r sits at chunk
   // c ^ (r & 7).
@@ -239,17 +233,125 @@ __global__ __launch_bounds__(256, 4) void rot_block_quant_kernel(const void* x_,
         const int w = pack4_e4m3(__fdiv_rn(acc[nb][4 * g], sc), __fdiv_rn(acc[nb][4 * g + 1], sc),
                                  __fdiv_rn(acc[nb][4 * g + 2], sc), __fdiv_rn(acc[nb][4 * g + 3], sc));
         const int byte = nb * 32 + 8 * g + 4 * h;
-        *(int*)(rt_lds + r * 128 + (((byte >> 4) ^ (r & 7)) << 4) + (byte & 15)) = w;
+        *(int*)(r_lds + r * 128 + (((byte >> 4) ^ (r & 7)) << 4) + (byte & 15)) = w;
       }
   }
   __syncthreads();
-  unsigned char* qo = q + ((long long)bn * S + row0) * 128;
+  unsigned char* qo = q + (long long)row0 * 128;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = (tid >> 3) + 32 * i, c = tid & 7;
-    const i32x4_t w = *(const i32x4_t*)(rt_lds + r * 128 + ((c ^ (r & 7)) << 4));
+    const i32x4_t w = *(const i32x4_t*)(r_lds + r * 128 + ((c ^ (r & 7)) << 4));
     if (row0 + r < S) *(i32x4_t*)(qo + (long long)r * 128 + c * 16) = w;
   }
+}
+
+// Largest magnitude of each of 128 channels over `rows` rows from v on: thread c < 128 returns channel c's.
+template <int DT>
+__device__ __forceinline__ float channel_amax_body(const typename Elem<DT>::type* v, long long ss, int rows, float (*part)[128]) {
+  using T = typename Elem<DT>::type;
+  const int c16 = threadIdx.x & 15, rgrp = threadIdx.x >> 4;
+  float m[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) m[j] = 0.f;
+  // 8 rows of a thread are requested before the first one is used (rows past the end read row 0 again)
+  for (int r0 = rgrp; r0 < rows; r0 += 128) {
+    union { i32x4_t v; T e[8]; } u[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = r0 + 16 * i;
+      u[i].v = *(const i32x4_t*)(v + (long long)(r < rows ? r : 0) * ss + c16 * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) m[j] = fmaxf(m[j], fabsf((float)u[i].e[j]));
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) part[rgrp][c16 * 8 + j] = m[j];
+  __syncthreads();
+  float a = 0.f;
+  if (threadIdx.x < 128) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) a = fmaxf(a, part[r][threadIdx.x]);
+  }
+  return a;
+}
+#endif
+
+template <int DT, int BS>
+__global__ __launch_bounds__(256) void block_quant_reg_kernel(const void* x_, unsigned char* q, float* scale,
+                                                             long long sb, long long sn, long long ss, int N, int S,
+                                                             float prescale, int pow2) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  using T = typename Elem<DT>::type;
+  __shared__ float red[4];
+  const int blk = blockIdx.x, bn = blockIdx.y;
+  const int b = bn / N, n = bn - b * N;
+  block_quant_body<DT, BS>((const T*)x_ + b * sb + n * sn, q + (long long)bn * S * 128, scale + (long long)bn * gridDim.x + blk, ss,
+                           S, blk, prescale, pow2, red);
+#endif
+}
+
+// (launch bounds: at least 4 waves per SIMD = 128 registers per lane, so that the four workgroups whose LDS fits a CU
+// are resident together - the pass is bound by memory latency)
+template <int DT>
+__global__ __launch_bounds__(256, 4) void rot_block_quant_kernel(const void* x_, const void* rot_t, unsigned char* q,
+                                                              float* scale, long long sb, long long sn, long long ss,
+                                                              int N, int S, float prescale, int pow2) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  using T = typename Elem<DT>::type;
+  __shared__ __attribute__((aligned(16))) char r_lds[128 * 256];
+  __shared__ float red[4];
+  const int blk = blockIdx.x, bn = blockIdx.y;
+  const int b = bn / N, n = bn - b * N;
+  rot_block_body<DT, true>((const T*)x_ + b * sb + n * sn, rot_t, q + (long long)bn * S * 128,
+                           scale + (long long)bn * gridDim.x + blk, ss, S, blk, prescale, pow2, r_lds, red);
+#endif
+}
+
+// ---- everything that reads 16-bit q, k and v first, as one launch ---------------------------------------------------
+// Workgroups are numbered: parts of V (per-channel maxima of v_rows keys of one head), then the 128-token blocks of q, then
+// those of k (codes and scale, behind the rotation if there is one).  The parts of V are the longest and start first.  Their
+// maxima leave as plain stores, one row of 128 per part, and v_quant_transpose_kernel takes the maximum over a head's rows: no
+// memory to clear, no atomics.  Before, this was six launches (two transposed copies of the rotation, two rotations, clearing,
+// maxima).  What bounds it: memory, and with few tokens its chain of loads, products, maximum and stores (12 us at 20 heads x
+// 1026 tokens, where the six took 32 us and their gaps); 40 heads x 7205 tokens 113 -> 74 us, 4.0 TB/s of the bytes it moves.  The
+// whole module: 1026 x 20 66 -> 39 us, 3114 x 12 93 -> 68, 5791 x 20 238 -> 219, 7205 x 40 660 -> 636 us, 32760 x 40 0.3 %.
+struct QkvQuantParams {
+  const void *q, *k, *v, *q_rot, *k_rot;  // rotations [128][128] row major, or null
+  unsigned char *q8, *k8;
+  float *q_scale, *k_scale, *v_max;       // v_max [B * N][v_parts][128]
+  long long q_sb, q_sn, q_ss, k_sb, k_sn, k_ss, v_sb, v_sn, v_ss;
+  int BN, N, Sq, Skv, q_blocks, k_blocks, v_parts, v_rows;
+};
+template <int DT>
+__global__ __launch_bounds__(256, 4) void qkv_quant_kernel(const QkvQuantParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  using T = typename Elem<DT>::type;
+  __shared__ __attribute__((aligned(16))) char lds[128 * 256];
+  __shared__ float red[4];
+  int i = blockIdx.x;
+  if (i < p.BN * p.v_parts) {
+    const int bn = i / p.v_parts, part = i - bn * p.v_parts, b = bn / p.N, n = bn - b * p.N;
+    const int row0 = part * p.v_rows;
+    const float a = channel_amax_body<DT>((const T*)p.v + b * p.v_sb + n * p.v_sn + row0 * p.v_ss, p.v_ss,
+                                          min(p.v_rows, p.Skv - row0), (float(*)[128])lds);
+    if (threadIdx.x < 128) p.v_max[(long long)i * 128 + threadIdx.x] = a;
+    return;
+  }
+  i -= p.BN * p.v_parts;
+  const bool is_q = i < p.BN * p.q_blocks;
+  if (!is_q) i -= p.BN * p.q_blocks;
+  const int nblk = is_q ? p.q_blocks : p.k_blocks, S = is_q ? p.Sq : p.Skv;
+  const int bn = i / nblk, blk = i - bn * nblk, b = bn / p.N, n = bn - b * p.N;
+  const T* x = is_q ? (const T*)p.q + b * p.q_sb + n * p.q_sn : (const T*)p.k + b * p.k_sb + n * p.k_sn;
+  const long long ss = is_q ? p.q_ss : p.k_ss;
+  const void* rot = is_q ? p.q_rot : p.k_rot;
+  unsigned char* codes = (is_q ? p.q8 : p.k8) + (long long)bn * S * 128;
+  float* scale = (is_q ? p.q_scale : p.k_scale) + i;
+  if (rot) rot_block_body<DT, false>(x, rot, codes, scale, ss, S, blk, 1.f, 0, lds, red);
+  else block_quant_body<DT, 128>(x, codes, scale, ss, S, blk, 1.f, 0, red);
 #endif
 }
 
@@ -267,34 +369,9 @@ __global__ __launch_bounds__(256) void channel_amax_kernel(const void* v_, unsig
   using T = typename Elem<DT>::type;
   __shared__ float part[16][128];
   const int bn = blockIdx.y, b = bn / N, n = bn - b * N;
-  const T* v = (const T*)v_ + b * sb + n * sn;
-  const int c16 = threadIdx.x & 15, rgrp = threadIdx.x >> 4;
-  const int row0 = blockIdx.x * 1024, rows = min(1024, S - row0);
-  float m[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) m[j] = 0.f;
-  // 8 rows of a thread are requested before the first one is used (rows past the end read row 0 again)
-  for (int r0 = rgrp; r0 < rows; r0 += 128) {
-    union { i32x4_t v; T e[8]; } u[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r = r0 + 16 * i;
-      u[i].v = *(const i32x4_t*)(v + (long long)(row0 + (r < rows ? r : 0)) * ss + c16 * 8);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) m[j] = fmaxf(m[j], fabsf((float)u[i].e[j]));
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) part[rgrp][c16 * 8 + j] = m[j];
-  __syncthreads();
-  if (threadIdx.x < 128) {
-    float a = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) a = fmaxf(a, part[r][threadIdx.x]);
-    atomicMax(amax_bits + (long long)bn * 128 + threadIdx.x, __builtin_bit_cast(unsigned, a));
-  }
+  const int row0 = blockIdx.x * 1024;
+  const float a = channel_amax_body<DT>((const T*)v_ + b * sb + n * sn + row0 * ss, ss, min(1024, S - row0), part);
+  if (threadIdx.x < 128) atomicMax(amax_bits + (long long)bn * 128 + threadIdx.x, __builtin_bit_cast(unsigned, a));
 #endif
 }
 
@@ -306,32 +383,24 @@ __host__ __device__ __forceinline__ int v8t_pos(int kk) {
   return 32 * h + 16 * blk32 + 4 * g8 + e;
 }
 
-// V [B][N][S][128] -> V8T [B][N][128][S128] bytes + per-channel scale [B][N][128] = amax/448.
+// V [B][N][S][128] -> V8T [B][N][128][S128] bytes + per-channel scale [B][N][128] = amax/448, amax being the maximum over
+// the head's amax_rows rows of 128.
 // One workgroup = 128 keys of one (batch, head): every channel row it writes is one full 128-byte line.
 // A thread takes 8 channels of two groups of 4 consecutive keys: 4 consecutive keys are 4 consecutive positions of
 // V8T (v8t_pos), so their codes of one channel leave as one dword.  LDS tile [channel][128 positions], 16-byte chunk
 // c of a row stored at chunk c ^ ((channel >> 3) & 7): the 16 threads of a key group, 8 channels apart, then write
 // to 8 different bank groups.
 template <int DT>
-__global__ __launch_bounds__(256) void v_quant_transpose_kernel(const void* v_, const unsigned* amax_bits,
+__global__ __launch_bounds__(256) void v_quant_transpose_kernel(const void* v_, const float* amax, int amax_rows,
                                                                 unsigned char* v8t, float* vscale, long long sb,
                                                                 long long sn, long long ss, int N, int S, int S128) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using T = typename Elem<DT>::type;
   __shared__ __attribute__((aligned(16))) unsigned char tile[128 * 128];
+  __shared__ float rows_max[2][128];
   const int grp = blockIdx.x, bn = blockIdx.y, b = bn / N, n = bn - b * N;
   const T* v = (const T*)v_ + b * sb + n * sn;
   const int c16 = threadIdx.x & 15, qd = threadIdx.x >> 4;
-  float sc[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float a = __builtin_bit_cast(float, amax_bits[(long long)bn * 128 + c16 * 8 + j]);
-    sc[j] = a > 0.f ? __fdiv_rn(a, kE4M3Max) : 1.0f;
-  }
-  if (grp == 0 && qd == 0) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) vscale[(long long)bn * 128 + c16 * 8 + j] = sc[j];
-  }
   // keys 4 * qd + j and 64 + 4 * qd + j (j < 4): all 8 rows are requested before the first one is used
   union { i32x4_t v; T e[8]; } u[2][4];
 #pragma unroll
@@ -342,6 +411,25 @@ __global__ __launch_bounds__(256) void v_quant_transpose_kernel(const void* v_, 
       u[half][j].v = i32x4_t{0, 0, 0, 0};
       if (key < S) u[half][j].v = *(const i32x4_t*)(v + (long long)key * ss + c16 * 8);
     }
+  // the scales: every row of maxima is read once by the workgroup
+  {
+    const int ch = threadIdx.x & 127, odd = threadIdx.x >> 7;
+    float a = 0.f;
+#pragma unroll 4
+    for (int r = odd; r < amax_rows; r += 2) a = fmaxf(a, amax[((long long)bn * amax_rows + r) * 128 + ch]);
+    rows_max[odd][ch] = a;
+  }
+  __syncthreads();
+  float sc[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float a = fmaxf(rows_max[0][c16 * 8 + j], rows_max[1][c16 * 8 + j]);
+    sc[j] = a > 0.f ? __fdiv_rn(a, kE4M3Max) : 1.0f;
+  }
+  if (grp == 0 && qd == 0) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) vscale[(long long)bn * 128 + c16 * 8 + j] = sc[j];
+  }
   const int swz = c16 & 7;  // (channel >> 3) & 7 of this thread's channels
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
@@ -795,11 +883,11 @@ static int v_quant_launch(const void* v, void* v8t, float* v_scale, int dtype, i
   dim3 g1((S + 1023) / 1024, B * N), g2(S128 / 128, B * N);
   if (dtype == MSD_DTYPE_BF16) {
     hipLaunchKernelGGL(channel_amax_kernel<MSD_DTYPE_BF16>, g1, dim3(256), 0, stream, v, amax, v_sb, v_sn, v_ss, N, S);
-    hipLaunchKernelGGL(v_quant_transpose_kernel<MSD_DTYPE_BF16>, g2, dim3(256), 0, stream, v, (const unsigned*)amax,
+    hipLaunchKernelGGL(v_quant_transpose_kernel<MSD_DTYPE_BF16>, g2, dim3(256), 0, stream, v, (const float*)amax, 1,
                        (unsigned char*)v8t, v_scale, v_sb, v_sn, v_ss, N, S, S128);
   } else {
     hipLaunchKernelGGL(channel_amax_kernel<MSD_DTYPE_F16>, g1, dim3(256), 0, stream, v, amax, v_sb, v_sn, v_ss, N, S);
-    hipLaunchKernelGGL(v_quant_transpose_kernel<MSD_DTYPE_F16>, g2, dim3(256), 0, stream, v, (const unsigned*)amax,
+    hipLaunchKernelGGL(v_quant_transpose_kernel<MSD_DTYPE_F16>, g2, dim3(256), 0, stream, v, (const float*)amax, 1,
                        (unsigned char*)v8t, v_scale, v_sb, v_sn, v_ss, N, S, S128);
   }
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
@@ -889,6 +977,88 @@ int mindiesd_fp8_attention_fwd(const void* q8, const void* k8, const void* v8t, 
                     : fp8_fa_launch<MSD_DTYPE_F16, false, true>(p, grid, stream);
   return bf ? fp8_fa_launch<MSD_DTYPE_BF16, false, false>(p, grid, stream)
             : fp8_fa_launch<MSD_DTYPE_F16, false, false>(p, grid, stream);
+}
+
+// ---- rotation, quantisation and attention as one call: three launches ---------------------------------------------
+namespace {
+struct Fp8Scratch {  // offsets into the workspace, each a multiple of 256
+  size_t q8, k8, v8t, q_scale, k_scale, v_scale, v_max, bytes;
+  int v_parts, v_rows;
+};
+Fp8Scratch fp8_scratch(int B, int N, int Sq, int Skv) {
+  Fp8Scratch w{};
+  const size_t BN = (size_t)B * N;
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t here = at;
+    at += (bytes + 255) / 256 * 256;
+    return here;
+  };
+  // V's maxima: parts of at least 512 keys, at most 16 to a head (every workgroup of the next launch reads all of its head's
+  // rows of maxima), whole multiples of the 128 keys that a workgroup has in flight
+  const int parts = Skv < 16 * 512 ? (Skv + 511) / 512 : 16;
+  w.v_rows = (Skv + parts * 128 - 1) / (parts * 128) * 128;
+  w.v_parts = (Skv + w.v_rows - 1) / w.v_rows;
+  w.q8 = take(BN * Sq * 128);
+  w.k8 = take(BN * Skv * 128);
+  w.v8t = take(BN * 128 * (((size_t)Skv + 127) / 128 * 128));
+  w.q_scale = take(BN * (((size_t)Sq + 127) / 128) * 4);
+  w.k_scale = take(BN * (((size_t)Skv + 127) / 128) * 4);
+  w.v_scale = take(BN * 128 * 4);
+  w.v_max = take(BN * w.v_parts * 128 * 4);
+  w.bytes = at;
+  return w;
+}
+}  // namespace
+
+size_t mindiesd_fp8_rot_attention_workspace_size(int B, int N, int Sq, int Skv) {
+  if (B <= 0 || N <= 0 || Sq <= 0 || Skv <= 0) return 0;
+  return fp8_scratch(B, N, Sq, Skv).bytes;
+}
+
+int mindiesd_fp8_rot_attention_fwd(const void* q, const void* k, const void* v, const void* q_rot, const void* k_rot, void* out,
+                                   int dtype, int B, int N, int Sq, int Skv, int D, long long q_sb, long long q_sn,
+                                   long long q_ss, long long k_sb, long long k_sn, long long k_ss, long long v_sb,
+                                   long long v_sn, long long v_ss, long long o_sb, long long o_sn, long long o_ss, float scale,
+                                   int flags, void* workspace, size_t ws_bytes, hipStream_t stream) {
+  if (!q || !k || !v || !out || !workspace || B <= 0 || N <= 0 || Sq <= 0 || Skv <= 0) return MSD_ERR_BAD_ARG;
+  if (D != 128 || !(scale > 0.f)) return MSD_ERR_UNSUPPORTED;
+  if (dtype != MSD_DTYPE_BF16 && dtype != MSD_DTYPE_F16) return MSD_ERR_BAD_ARG;
+  if (flags & ~MSD_FP8_P_EXP2) return MSD_ERR_BAD_ARG;
+  if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)q_rot | (uintptr_t)k_rot | (uintptr_t)out | (uintptr_t)workspace) & 15)
+    return MSD_ERR_BAD_ARG;
+  if ((q_sb | q_sn | q_ss | k_sb | k_sn | k_ss | v_sb | v_sn | v_ss | o_sb | o_sn | o_ss) & 7) return MSD_ERR_BAD_ARG;
+  const long long BN = (long long)B * N;
+  if (BN > 65535 || (long long)Sq * 128 >= (1ll << 31) || (long long)(Skv + 127) * 128 >= (1ll << 31)) return MSD_ERR_UNSUPPORTED;
+  const Fp8Scratch w = fp8_scratch(B, N, Sq, Skv);
+  if (ws_bytes < w.bytes) return MSD_ERR_WORKSPACE;
+  char* ws = (char*)workspace;
+  QkvQuantParams p{};
+  p.q = q; p.k = k; p.v = v; p.q_rot = q_rot; p.k_rot = k_rot;
+  p.q8 = (unsigned char*)ws + w.q8; p.k8 = (unsigned char*)ws + w.k8;
+  p.q_scale = (float*)(ws + w.q_scale); p.k_scale = (float*)(ws + w.k_scale); p.v_max = (float*)(ws + w.v_max);
+  p.q_sb = q_sb; p.q_sn = q_sn; p.q_ss = q_ss;
+  p.k_sb = k_sb; p.k_sn = k_sn; p.k_ss = k_ss;
+  p.v_sb = v_sb; p.v_sn = v_sn; p.v_ss = v_ss;
+  p.BN = (int)BN; p.N = N; p.Sq = Sq; p.Skv = Skv;
+  p.q_blocks = (Sq + 127) / 128; p.k_blocks = (Skv + 127) / 128;
+  p.v_parts = w.v_parts; p.v_rows = w.v_rows;
+  const long long grid = BN * ((long long)p.v_parts + p.q_blocks + p.k_blocks);
+  if (grid > 0x7ffffff0ll) return MSD_ERR_UNSUPPORTED;
+  const dim3 g2(p.k_blocks, B * N);
+  const int S128 = p.k_blocks * 128;
+  auto quantise = [&](auto dt) {
+    constexpr int DT = decltype(dt)::value;
+    hipLaunchKernelGGL(qkv_quant_kernel<DT>, dim3((unsigned)grid), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(v_quant_transpose_kernel<DT>, g2, dim3(256), 0, stream, v, (const float*)p.v_max, p.v_parts,
+                       (unsigned char*)ws + w.v8t, (float*)(ws + w.v_scale), v_sb, v_sn, v_ss, N, Skv, S128);
+    return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
+  };
+  const int rc = dtype == MSD_DTYPE_BF16 ? quantise(std::integral_constant<int, MSD_DTYPE_BF16>{})
+                                         : quantise(std::integral_constant<int, MSD_DTYPE_F16>{});
+  if (rc != MSD_OK) return rc;
+  return mindiesd_fp8_attention_fwd(p.q8, p.k8, ws + w.v8t, p.q_scale, p.k_scale, (const float*)(ws + w.v_scale), out, dtype, B, N,
+                                    Sq, Skv, D, o_sb, o_sn, o_ss, scale, flags, stream);
 }
 
 }  // extern "C"

@@ -255,3 +255,26 @@ def test_ops_match_the_python_functions_and_trace(cuda):
 
     o1, o2 = torch.compile(fn, backend="eager", fullgraph=True)(q, k, v, x)
     assert torch.equal(o1, out) and torch.equal(o2, y)
+
+
+@pytest.mark.parametrize("sq, skv, rotated, dtype, layout, rule", [
+    (1, 1, "qk", torch.bfloat16, "BNSD", "linear"), (127, 129, "qk", torch.float16, "BSND", "linear"),
+    (128, 512, "q", torch.bfloat16, "BNSD", "exp2"), (300, 513, "k", torch.bfloat16, "BSND", "linear"),
+    (1026, 1026, "", torch.float16, "BNSD", "linear"), (257, 8191, "qk", torch.bfloat16, "BNSD", "linear"),
+    (129, 8193, "qk", torch.bfloat16, "BSND", "linear"), (64, 20011, "q", torch.float16, "BNSD", "exp2")])
+def test_one_call_has_the_bits_of_its_parts(cuda, sq, skv, rotated, dtype, layout, rule):
+    """The fused quantisation launch against the separate passes: one part of V's maxima and the most there can be, parts and
+    blocks that end inside their rows, the rotation read row by row against its transposed copy, strided inputs."""
+    from mindiesd.layers.quant.block_quant import _block_quant, _rot_block_quant
+    from mindiesd.layers.quant.fp8_attention import fp8_attention_forward, fp8_attention_quantized, quantize_v_per_channel
+    g = torch.Generator().manual_seed(sq + skv)
+    def tensor(s):
+        shape = (2, 3, s, 2, 128) if layout == "BNSD" else (2, s, 3, 2, 128)
+        return (torch.randn(shape, generator=g) * torch.rand(shape[-1], generator=g) * 4).to(dtype).to(cuda)[..., 1, :]
+    q, k, v = tensor(sq), tensor(skv), tensor(skv)
+    rot = torch.linalg.qr(torch.randn(128, 128, generator=g))[0].to(cuda)          # fp32, converted by both sides
+    q_rot, k_rot = (rot if "q" in rotated else None), (rot.t() if "k" in rotated else None)
+    parts = [_block_quant(x, 128, layout) if r is None else _rot_block_quant(x, r, layout) for x, r in ((q, q_rot), (k, k_rot))]
+    want = fp8_attention_quantized(*parts[0], *parts[1], *quantize_v_per_channel(v, layout), 0.09, dtype, layout, p_rule=rule)
+    got = fp8_attention_forward(q, k, v, 0.09, layout, q_rot, k_rot, p_rule=rule)
+    assert torch.isfinite(got.float()).all() and torch.equal(got, want)
