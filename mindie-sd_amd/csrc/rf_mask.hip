@@ -145,27 +145,18 @@ struct MaskParams {
 constexpr int kMaxBlocks = 2048;
 
 // One workgroup = kMaskRows consecutive query-block rows of one (batch, head): the pooled keys of the head are read
-// once for all of them (with one row per workgroup the kernel was bound by those reads: 150 KiB from L2 per row),
-// then the rows are finished one after the other.
+// once for all of them (with one row per workgroup the kernel was bound by those reads: 150 KiB from L2 per row); then
+// every wave finishes one of the rows by itself.  The four waves working on one row after the other met at some 40
+// barriers per row: 20 heads x 26 blocks 19 -> 6 us, 40 heads x 591 blocks 311 -> 230 us.
 constexpr int kMaskRows = 4;
 
-template <int DT>
+// REGS: key blocks per lane that a row's wave keeps in registers from the scores on (NB <= 64 * REGS).
+template <int DT, int REGS>
 __global__ __launch_bounds__(256) void rf_block_mask_kernel(const MaskParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using T = typename Elem<DT>::type;
   __shared__ float qrow[kMaskRows][128];
-  __shared__ double red[256];
-  // per key block (dynamic LDS, 14 + 4 * kMaskRows bytes per block: a row of 591 blocks leaves room for 8
-  // workgroups per CU):
-  extern __shared__ __attribute__((aligned(16))) char mask_lds[];
-  const int NBp = (p.NB + 3) & ~3;
-  double* ex = (double*)mask_lds;                                  // exp(score - maximum)
-  unsigned short* key = (unsigned short*)(mask_lds + (size_t)NBp * 8);   // 16-bit pattern of the rounded probabilities
-  float* xs_all = (float*)(mask_lds + (size_t)NBp * 12);           // [kMaskRows][NBp] scaled scores, rounded to 16 bit
-  __shared__ int hist[256];
-  __shared__ int suf[257];
-  __shared__ int wave_cnt[4];
-  __shared__ int sel_bin, sel_rem, run_base;
+  extern __shared__ float xs_all[];  // [kMaskRows][NB] scaled scores, rounded to 16 bit
   const int row0 = blockIdx.x * kMaskRows, bn = blockIdx.y;
   const int b = bn / p.N, n = bn - b * p.N;
   const int tid = threadIdx.x;
@@ -208,89 +199,54 @@ __global__ __launch_bounds__(256) void rf_block_mask_kernel(const MaskParams p) 
       for (int o = 2; o > 0; o >>= 1) acc[r] += __shfl_xor(acc[r], o, 64);
       if (c < NB && sub == 0) {
         const float s16 = round16<DT>((float)acc[r]);
-        xs_all[r * NBp + c] = round16<DT>(__fmul_rn(s16, p.scale));
+        xs_all[r * NB + c] = round16<DT>(__fmul_rn(s16, p.scale));
       }
     }
   }
   __syncthreads();
 
-  for (int rr = 0; rr < nrows; ++rr) {
+  const int lane = tid & 63, rr = tid >> 6;
+  if (rr >= nrows) return;
   const int row = row0 + rr;
-  const float* xs = xs_all + rr * NBp;
-  float lmax = -INFINITY;
-  for (int c = tid; c < NB; c += 256) lmax = fmaxf(lmax, xs[c]);
-  red[tid] = (double)lmax;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (tid < s) red[tid] = fmax(red[tid], red[tid + s]);
-    __syncthreads();
+  const float* xs = xs_all + rr * NB;
+  float x[REGS], mx = -INFINITY;  // block 64 * i + lane in register i
+#pragma unroll
+  for (int i = 0; i < REGS; ++i) {
+    x[i] = 64 * i + lane < NB ? xs[64 * i + lane] : -INFINITY;
+    mx = fmaxf(mx, x[i]);
   }
-  const double mx = red[0];
-  __syncthreads();
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
 
   // ---- softmax in fp64, rounded to fp32 and then to 16 bit --------------------------------------
-  // (the exponentials are kept in LDS between the sum and the division: fp64 exp is the longest chain here)
-  double lsum = 0.0;
-  for (int c = tid; c < NB; c += 256) {
-    const double e = exp((double)xs[c] - mx);
-    ex[c] = e;
-    lsum += e;
-  }
-  red[tid] = lsum;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (tid < s) red[tid] += red[tid + s];
-    __syncthreads();
-  }
-  const double denom = red[0];
-  for (int c = tid; c < NB; c += 256) {
-    const float pr = (float)(ex[c] / denom);
-    const T p16 = Elem<DT>::from_float(pr);
-    key[c] = __builtin_bit_cast(unsigned short, p16);  // probabilities are >= 0: bit order == value order
-  }
-  hist[tid] = 0;
-  __syncthreads();
-
-  // ---- keep_len-th largest value: two-level radix select on the 16-bit patterns -------------------
-  // Per level: histogram of one byte, suffix sums over the 256 bins (one bin per thread, a scan inside the
-  // waves and a combine over the four of them), and the bin in which the wanted rank falls: the one with
-  // suffix(bin) >= need > suffix(bin + 1); the rank inside it is need - suffix(bin + 1).
-  const int lane = tid & 63, wv = tid >> 6;
-  auto pick_bin = [&](int need) {
-    int v = hist[tid];
+  // (the sum is a fixed tree over 256 partial sums, four of them in a lane)
+  double e[REGS], part[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int t = __shfl_down(v, o, 64);
-      if (lane + o < 64) v += t;
+  for (int i = 0; i < REGS; ++i)
+    if (64 * i + lane < NB) {
+      e[i] = exp((double)x[i] - (double)mx);
+      part[i & 3] += e[i];
     }
-    if (lane == 0) wave_cnt[wv] = v;
-    __syncthreads();
-    for (int w2 = wv + 1; w2 < 4; ++w2) v += wave_cnt[w2];
-    suf[tid] = v;
-    if (tid == 0) suf[256] = 0;
-    __syncthreads();
-    // bin 0 also takes what no other bin takes (the scan it replaces stopped there)
-    const bool mine = tid == 0 ? suf[1] < need : (suf[tid] >= need && suf[tid + 1] < need);
-    if (mine) {
-      sel_bin = tid;
-      sel_rem = need - suf[tid + 1];
-    }
-    __syncthreads();
-  };
-  for (int c = tid; c < NB; c += 256) atomicAdd(&hist[key[c] >> 8], 1);
-  __syncthreads();
-  pick_bin(p.keep_len);
-  const int hi_bin = sel_bin;
-  const int rem = sel_rem;
-  hist[tid] = 0;
-  __syncthreads();
-  for (int c = tid; c < NB; c += 256)
-    if ((key[c] >> 8) == hi_bin) atomicAdd(&hist[key[c] & 255], 1);
-  __syncthreads();
-  pick_bin(rem);
-  if (tid == 0) run_base = 0;
-  __syncthreads();
-  const unsigned thr = ((unsigned)hi_bin << 8) | (unsigned)sel_bin;
+  double denom = (part[0] + part[2]) + (part[1] + part[3]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) denom += __shfl_down(denom, o, 64);
+  denom = __shfl(denom, 0, 64);
+  unsigned key[REGS];  // 16-bit patterns of the rounded probabilities: these are >= 0, bit order == value order
+#pragma unroll
+  for (int i = 0; i < REGS; ++i) {
+    key[i] = 0;  // (blocks that do not exist: below every threshold that is tested)
+    if (64 * i + lane < NB) key[i] = __builtin_bit_cast(unsigned short, Elem<DT>::from_float((float)(e[i] / denom)));
+  }
+
+  // ---- keep_len-th largest value: the largest pattern that at least keep_len patterns reach, bit by bit -----------
+  unsigned thr = 0;
+  for (int bit = 15; bit >= 0; --bit) {
+    const unsigned t = thr | (1u << bit);
+    int reach = 0;
+#pragma unroll
+    for (int i = 0; i < REGS; ++i) reach += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key[i] >= t));
+    if (reach >= p.keep_len) thr = t;
+  }
 
   // ---- mask row (score >= threshold, forced rows / columns), ordered compaction -------------------
   const bool row_forced = row < p.ff_blocks || row >= NB - p.txt_blocks;
@@ -298,38 +254,31 @@ __global__ __launch_bounds__(256) void rf_block_mask_kernel(const MaskParams p) 
   signed char* mrow = p.mask ? p.mask + row_lin * NB : nullptr;
   int* irow = p.blk_idx ? p.blk_idx + row_lin * p.kb_stride : nullptr;
   long long* irow64 = (p.idx64 && b == 0) ? p.idx64 + ((long long)row * p.N + n) * NB : nullptr;
-  for (int c0 = 0; c0 < NB; c0 += 256) {
-    const int c = c0 + tid;
+  int total = 0;
+#pragma unroll
+  for (int i = 0; i < REGS; ++i) {
+    const int c = 64 * i + lane;
     bool keep = false;
     if (c < NB) {
-      keep = key[c] >= thr || row_forced || c < p.ff_blocks || c >= NB - p.txt_blocks || (p.keep_diag && c == row);
+      keep = key[i] >= thr || row_forced || c < p.ff_blocks || c >= NB - p.txt_blocks || (p.keep_diag && c == row);
       if (mrow) mrow[c] = keep ? 1 : 0;
     }
     const unsigned long long bal = __builtin_amdgcn_ballot_w64(keep);
-    if (lane == 0) wave_cnt[wv] = __builtin_popcountll(bal);
-    __syncthreads();
-    int off = run_base;
-    for (int w2 = 0; w2 < wv; ++w2) off += wave_cnt[w2];
-    off += __builtin_popcountll(bal & ((1ull << lane) - 1ull));
+    const int off = total + __builtin_popcountll(bal & ((1ull << lane) - 1ull));
     if (keep) {
       if (irow) irow[off] = c;
       if (irow64) irow64[off] = c;
     }
-    __syncthreads();
-    if (tid == 0) run_base += wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
-    __syncthreads();
+    total += __builtin_popcountll(bal);
   }
-  const int total = run_base;
   if (irow)
-    for (int c = total + tid; c < p.kb_stride; c += 256) irow[c] = -1;
+    for (int c = total + lane; c < p.kb_stride; c += 64) irow[c] = -1;
   if (irow64)
-    for (int c = total + tid; c < NB; c += 256) irow64[c] = -1;
-  if (tid == 0) {
+    for (int c = total + lane; c < NB; c += 64) irow64[c] = -1;
+  if (lane == 0) {
     if (p.blk_cnt) p.blk_cnt[row_lin] = total;
     if (p.cnt64 && b == 0) p.cnt64[(long long)row * p.N + n] = total;
   }
-  __syncthreads();
-  }  // rows of the workgroup
 #endif
 }
 
@@ -440,12 +389,19 @@ int mindiesd_rf_block_mask(const void* q_pool, const void* k_pool, int dtype, in
   p.keep_len = keep_len; p.txt_blocks = txt_blocks; p.ff_blocks = ff_blocks; p.keep_diag = keep_diag;
   p.scale = scale;
   dim3 grid((NB + kMaskRows - 1) / kMaskRows, B * N);
-  const size_t lds = (size_t)((NB + 3) & ~3) * (12 + 4 * kMaskRows);  // at most 56 KiB (NB <= kMaxBlocks)
-  if (dtype == MSD_DTYPE_BF16)
-    hipLaunchKernelGGL(rf_block_mask_kernel<MSD_DTYPE_BF16>, grid, dim3(256), lds, stream, p);
-  else
-    hipLaunchKernelGGL(rf_block_mask_kernel<MSD_DTYPE_F16>, grid, dim3(256), lds, stream, p);
-  return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
+  const int lds = NB * 4 * kMaskRows;  // at most 32 KiB (NB <= kMaxBlocks)
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, p);
+    return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
+  };
+  auto pick = [&](auto dt) {
+    constexpr int DT = decltype(dt)::value;
+    if (NB <= 128) return launch(rf_block_mask_kernel<DT, 2>);
+    if (NB <= 640) return launch(rf_block_mask_kernel<DT, 10>);
+    return launch(rf_block_mask_kernel<DT, kMaxBlocks / 64>);
+  };
+  return dtype == MSD_DTYPE_BF16 ? pick(std::integral_constant<int, MSD_DTYPE_BF16>{})
+                                 : pick(std::integral_constant<int, MSD_DTYPE_F16>{});
 }
 
 int mindiesd_mask_to_index(const signed char* mask, int BN, int QB, int KB, int* blk_idx, int* blk_cnt,

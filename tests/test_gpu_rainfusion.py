@@ -143,6 +143,22 @@ def test_block_mask_keep_diagonal_and_fp16(cuda):
     assert bool(torch.diagonal(got, dim1=-2, dim2=-1).all())
 
 
+@pytest.mark.parametrize("nb", [1, 3, 64, 65, 128, 129, 640, 641, 2048])
+def test_block_mask_sizes(cuda, nb):
+    """A row's key blocks in one register of its wave, in all of an instantiation's and one more; ties at the threshold
+    (pooled keys that repeat) and the smallest and largest number of blocks to keep."""
+    from mindiesd.layers.flash_attn import rainfusion as rf
+    g = torch.Generator().manual_seed(nb)
+    pool = torch.randn(3, 1, nb, 128, generator=g)
+    pool[1, 0, nb // 2:] = pool[1, 0, :nb - nb // 2].clone()
+    pool = pool.to(torch.bfloat16)
+    for sparsity in (0.0, 0.75, 1.0 - 1.0 / (nb + 1)):
+        for protect in (False, True):
+            args = (0, sparsity, 128 ** -0.5, 128, (2, 16, 16), (2, 16, 16), "BNSD")
+            got = rf.get_blockwise_mask(pool.to(cuda), *args, return_binary=True, protect_first_frame=protect).cpu()
+            assert torch.equal(got, orf.get_blockwise_mask(pool, *args, return_binary=True, protect_first_frame=protect))
+
+
 def test_get_mask_index_known_answers(cuda):
     """Reference KATs (test_sparse_flash_attn_rf_v2.py:198-216)."""
     from mindiesd.layers.flash_attn import rainfusion as rf
