@@ -167,6 +167,18 @@ int mindiesd_block_sparse_attention_paired_fwd(const void* q, const void* k, con
                                                float scale, const signed char* mask, const int* token_order,
                                                void* workspace, size_t ws_bytes, hipStream_t stream);
 
+/* The same call by whichever way suits its size: paired as above, or, for masks of at most 768 rows (B * N * ceil(Sq / 128)),
+ * one workgroup per mask row over its list, the longest lists first.  The result differs from the paired one by the order of
+ * accumulation only; arguments and workspace are the paired call's. */
+int mindiesd_block_sparse_attention_mask_fwd(const void* q, const void* k, const void* v, void* out, float* lse,
+                                               int dtype, int B, int N, int Nkv, int Sq, int Skv, int D,
+                                               long long q_sb, long long q_sn, long long q_ss,
+                                               long long k_sb, long long k_sn, long long k_ss,
+                                               long long v_sb, long long v_sn, long long v_ss,
+                                               long long o_sb, long long o_sn, long long o_ss,
+                                               float scale, const signed char* mask, const int* token_order,
+                                               void* workspace, size_t ws_bytes, hipStream_t stream);
+
 /* token_order[i] (int32, S entries) = row of the original [text | image (t,h,w)] sequence that holds the
  * token at position i of RainFusion's [image in 8x8-window order | text] sequence (the index map behind
  * rearrange_with_remaining, sparse_flash_attn_rf_v2.py:137-196, 297-312). */

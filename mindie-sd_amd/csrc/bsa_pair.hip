@@ -299,6 +299,70 @@ __global__ __launch_bounds__(1024) void bsa_pair_kernel(const unsigned* bits_g, 
 #endif
 }
 
+// ---- small masks: block lists in the order in which the workgroups should start ----------------------------------------
+// Workgroup x of 8 takes the mask rows that XCD x will work on (a run of consecutive rows, so that the XCD keeps its heads'
+// keys in its L2) and writes their ascending lists and counts, then order[8 * j + x] = the row with the j-th longest list of
+// the run (ties: the earlier row), so that the last workgroups to start are short ones.
+constexpr int kMaxRun = 1024;  // rows per XCD: one thread ranks one row
+__global__ __launch_bounds__(1024) void bsa_sorted_lists_kernel(const signed char* mask, int rows, int KB, int* idx, int* cnt,
+                                                                int* order) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(16))) int count[kMaxRun];
+  const int x = blockIdx.x, start = x * (rows / 8) + min(x, rows % 8), len = (rows - x + 7) / 8;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int kAhead = 4;  // rows of a wave whose bytes are requested together
+  for (int r0 = wave * kAhead; r0 < len; r0 += 16 * kAhead) {
+    int total[kAhead] = {0, 0, 0, 0};
+    for (int k0 = 0; k0 < KB; k0 += 128) {
+      bool on[kAhead][2];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int r = min(r0 + i, len - 1), k = k0 + 64 * j + lane;
+          on[i][j] = mask[(long long)(start + r) * KB + min(k, KB - 1)] != 0 && k < KB;
+        }
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const unsigned long long bal = __builtin_amdgcn_ballot_w64(on[i][j]);
+          if (on[i][j] && r0 + i < len)
+            idx[(long long)(start + r0 + i) * KB + total[i] + __builtin_popcountll(bal & ((1ull << lane) - 1ull))] = k0 + 64 * j + lane;
+          total[i] += __builtin_popcountll(bal);
+        }
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i)
+        if (r0 + i < len) cnt[start + r0 + i] = count[r0 + i] = total[i];
+    }
+  }
+  if ((int)threadIdx.x >= len) count[threadIdx.x] = -1;  // (a thread's own slot: the lists above fill those below len)
+  __syncthreads();
+  if ((int)threadIdx.x < len) {
+    const int me = threadIdx.x, mine = count[me];
+    int rank = 0;
+    for (int f = 0; f < len; f += 4) {
+      const i32x4_t c = *(const i32x4_t*)&count[f];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) rank += c[j] > mine || (c[j] == mine && f + j < me) ? 1 : 0;
+    }
+    order[8 * rank + x] = start + me;
+  }
+#endif
+}
+
+int bsa_build_sorted_lists(const signed char* mask, long long BN, int QB, int KB, int* ws, BsaSortedLists* t, hipStream_t stream) {
+  const long long rows = BN * QB;
+  if (rows <= 0 || rows > 8ll * kMaxRun) return MSD_ERR_UNSUPPORTED;
+  t->order = ws;
+  t->cnt = ws + rows;
+  t->idx = ws + 2 * rows;
+  hipLaunchKernelGGL(bsa_sorted_lists_kernel, dim3(8), dim3(1024), 0, stream, mask, (int)rows, KB, t->idx, t->cnt, t->order);
+  return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
+}
+
 // Workspace of the pairing (ints): bit rows + counts, candidates, pairs, shared lists + counts, exclusive lists +
 // counts, init counts.
 size_t bsa_pair_ints(long long BN, int QB, int KB) {

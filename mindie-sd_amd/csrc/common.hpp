@@ -281,6 +281,12 @@ struct BsaPairTables {
 size_t bsa_pair_ints(long long BN, int QB, int KB);
 bool bsa_pair_supported(int QB, int KB);
 int bsa_build_pairs(const signed char* mask, long long BN, int QB, int KB, int* ws, BsaPairTables* t, hipStream_t stream);
+struct BsaSortedLists {
+  int* order;  // [BN * QB] work order
+  int* cnt;    // [BN][QB]
+  int* idx;    // [BN][QB][KB]
+};
+int bsa_build_sorted_lists(const signed char* mask, long long BN, int QB, int KB, int* ws, BsaSortedLists* t, hipStream_t stream);
 
 // Lazy-rescale threshold of the online softmax, in log2 units.
 constexpr float kTau = 8.0f;

@@ -1558,6 +1558,47 @@ int mindiesd_block_sparse_attention_paired_fwd(const void* q, const void* k, con
                      : launch_fa<MSD_DTYPE_F16, 4, 32, 64, true, 1, 0, false, true>(p, stream);
 }
 
+// Block-sparse attention driven by the int8 mask: over paired query blocks as above, or, for small masks, one 128-row workgroup
+// per mask row, the longest rows of each XCD first (bsa_sorted_lists_kernel).  Pairing halves the K/V stream that bounds long
+// calls; with few rows the heads' keys stay in the L2 anyway, and what counts are the pairing's three launches (21 us) and the
+// 256-row workgroups, one to a CU, of which the longest end late.  rf_v3 / ada_bsa calls at sparsity 0.8, paired -> lists (the
+// former with the mask kernel's own gain of 12 us): 256 rows (8 heads x 4000 tokens) - / 78 -> 60 us, 520 (20 x 3264) 141 -> 108 /
+// 130 -> 108, 632 (8 x 10000) 286 -> 237 / 185 -> 157, 752 (8 x 12000) 331 -> 285 / 237 -> 208, 768 (24 x 4000) 164 -> 146 / 120 -> 102.
+// Above kListRows it depends on the mask: 800 (20 x 5000, sparsity 0.5) 228 -> 208 / 206 -> 207, 848 (8 x 13500) 450 -> 455 / 437 -> 469,
+// 1016 (8 x 16200, 0.6) 649 -> 597 / 463 -> 494; from 1700 rows on pairs win by up to 8 %.
+// Workspace as for the paired entry point.
+constexpr int kListRows = 3 * kCus;
+int mindiesd_block_sparse_attention_mask_fwd(const void* q, const void* k, const void* v, void* out, float* lse, int dtype, int B,
+                                             int N, int Nkv, int Sq, int Skv, int D, long long q_sb, long long q_sn,
+                                             long long q_ss, long long k_sb, long long k_sn, long long k_ss, long long v_sb,
+                                             long long v_sn, long long v_ss, long long o_sb, long long o_sn, long long o_ss,
+                                             float scale, const signed char* mask, const int* token_order, void* workspace,
+                                             size_t ws_bytes, hipStream_t stream) {
+  const int QB = Sq / 128 + (Sq % 128 != 0), KB = Skv / 128 + (Skv % 128 != 0);
+  if ((long long)B * N * QB > kListRows || !bsa_pair_supported(QB, KB))
+    return mindiesd_block_sparse_attention_paired_fwd(q, k, v, out, lse, dtype, B, N, Nkv, Sq, Skv, D, q_sb, q_sn, q_ss, k_sb, k_sn,
+                                                      k_ss, v_sb, v_sn, v_ss, o_sb, o_sn, o_ss, scale, mask, token_order,
+                                                      workspace, ws_bytes, stream);
+  const long long st[12] = {q_sb, q_sn, q_ss, k_sb, k_sn, k_ss, v_sb, v_sn, v_ss, o_sb, o_sn, o_ss};
+  int rc = check_common(q, k, v, out, dtype, B, N, Nkv, Sq, Skv, D, st, scale);
+  if (rc != MSD_OK) return rc;
+  if (!mask || !workspace || ((uintptr_t)workspace & 15)) return MSD_ERR_BAD_ARG;
+  if (token_order && Sq != Skv) return MSD_ERR_BAD_ARG;
+  if (ws_bytes < mindiesd_block_sparse_attention_paired_workspace_size(B, N, Sq, Skv)) return MSD_ERR_WORKSPACE;
+  BsaSortedLists l;
+  rc = bsa_build_sorted_lists(mask, (long long)B * N, QB, KB, (int*)workspace, &l, stream);
+  if (rc != MSD_OK) return rc;
+  FaParams p = make_params(q, k, v, out, lse, B, N, Nkv, Sq, Skv, st, scale);
+  p.blk_idx = l.idx; p.blk_cnt = l.cnt; p.kb_stride = KB; p.order = l.order;
+  p.tok = token_order;
+  p.QB = QB;
+  if (dtype == MSD_DTYPE_BF16)
+    return token_order ? launch_fa<MSD_DTYPE_BF16, 4, 32, 64, true, 1, 0, true>(p, stream)
+                       : launch_fa<MSD_DTYPE_BF16, 4, 32, 64, true, 1>(p, stream);
+  return token_order ? launch_fa<MSD_DTYPE_F16, 4, 32, 64, true, 1, 0, true>(p, stream)
+                     : launch_fa<MSD_DTYPE_F16, 4, 32, 64, true, 1>(p, stream);
+}
+
 // True when B x N x ceil(Sq / 256) workgroups of 256 rows would fill the 256 CUs badly - at most half of them busy, or
 // a second round for at most half of them - for the calls whose last round fa16_split does not cut: head dims below 64,
 // causal ones, and some at head_dim 64.  They run as 128-row workgroups of four waves, two to a CU.

@@ -40,6 +40,8 @@ SIGNATURES = {
     "mindiesd_block_sparse_attention_paired_workspace_size": (c_sz, [c_int] * 4),
     "mindiesd_block_sparse_attention_paired_fwd": (c_int, [c_p] * 5 + [c_int] * 7 + [c_ll] * 12 + [c_f, c_p, c_p, c_p, c_sz,
                                                                                           c_p]),
+    "mindiesd_block_sparse_attention_mask_fwd": (c_int, [c_p] * 5 + [c_int] * 7 + [c_ll] * 12 + [c_f, c_p, c_p, c_p, c_sz,
+                                                                                          c_p]),
     "mindiesd_block_sparse_attention_general_fwd": (c_int, [c_p] * 5 + [c_int] * 7 + [c_ll] * 12 + [c_f, c_p, c_p, c_int, c_p,
                                                                                            c_int, c_int, c_p]),
     "mindiesd_rf_token_order": (c_int, [c_p] + [c_int] * 5 + [c_p]),

@@ -372,7 +372,8 @@ def block_sparse_attention_mask(query, key, value, block_sparse_mask, scale, lay
     """Attention of every 128-row query block over the key blocks its mask row selects
     (``block_sparse_mask`` int8/bool [B, N, qb, kb], non-zero = attend; an all-zero row yields zeros).
     Runs the kernel over paired query blocks (query blocks with similar mask rows share their K/V
-    tiles); masks too large for the pairing kernels go through the block lists.  ``order`` as in
+    tiles), small masks one workgroup per mask row, the longest first; masks too large for the pairing
+    kernels go through the block lists.  ``order`` as in
     :func:`block_sparse_attention_lists`."""
     for name, t in (("query", query), ("key", key), ("value", value)):
         _check_gpu16(t, name)
@@ -397,7 +398,7 @@ def block_sparse_attention_mask(query, key, value, block_sparse_mask, scale, lay
     ws_bytes = lib.mindiesd_block_sparse_attention_paired_workspace_size(b, n, sq, skv)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
     with _native.on_device(q.device):
-        rc = lib.mindiesd_block_sparse_attention_paired_fwd(
+        rc = lib.mindiesd_block_sparse_attention_mask_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr() if return_lse else None,
             _native.DTYPE_CODE[q.dtype], b, n, nkv, sq, skv, q.shape[-1],
             *_strides_bns(q, layout), *_strides_bns(k, layout), *_strides_bns(v, layout), *_strides_bns(out, layout),
@@ -406,7 +407,7 @@ def block_sparse_attention_mask(query, key, value, block_sparse_mask, scale, lay
     if rc == 2 and q.shape[-1] == HEAD_DIM:  # mask too large for the pairing kernels
         idx, cnt = mask_to_lists(m8)
         return block_sparse_attention_lists(q, k, v, idx, cnt, scale, layout, return_lse, order)
-    _native.check(rc, "mindiesd_block_sparse_attention_paired_fwd")
+    _native.check(rc, "mindiesd_block_sparse_attention_mask_fwd")
     return (out, lse) if return_lse else out
 
 
