@@ -355,17 +355,28 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
     step(t + 6, std::integral_constant<int, 6>{}, fx, fq, fp);
     step(t + 7, std::integral_constant<int, 7>{}, fy, fq, fx);
   }
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // the trailing (empty) DMA requests
+  // the trailing (empty) DMA requests, mine and everybody's: the output is staged where they write
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  wg_barrier();
 
-  // ---- epilogue: bias, SwiGLU, 16-bit, straight from the accumulators ----------------------------------------------
+  // ---- epilogue: bias, SwiGLU, 16-bit, through LDS ------------------------------------------------------------------
   // W rows are the first matrix operand, so accumulator [a][w][mb][nb] register r holds
   // X row a*128 + wm*64 + mb*32 + l32 and W row (tile-local) w*128 + wn*64 + nb*32 + 8*(r/4) + 4*h + r%4:
-  // four consecutive output columns per register quad, written as one 8-byte store (the two halves of
-  // the wave complete 16 bytes, the four quads and two blocks the 128-byte line).  Output columns of the
-  // wave: SwiGLU: f0 + wn*64 + [0,64) (gate from w = 0, up from w = 1); plain: f0 + w*128 + wn*64 + [0,64).
+  // four consecutive output columns per register quad.  Output columns of the wave: SwiGLU: f0 + wn*64 + [0,64) (gate from
+  // w = 0, up from w = 1); plain: f0 + w*128 + wn*64 + [0,64).  Every 64 x 64 block goes through 8 KiB of LDS of its own, 16-byte
+  // chunk c of row r at chunk c ^ ((r >> 1) & 7), and leaves as full 128-byte lines: stored from the registers, 8 bytes to a
+  // row and instruction, the 32 rows of a store were 32 requests to the L2 for 16 bytes each, 4 us of a
+  // tile's 27 at K 1536.  Layers, before -> now: 39552 x 1536 x 4608 372 -> 318 us, 46344 x 1536 x 1536 190 -> 168, 4395 x 3072 x 12288
+  // 189 -> 170, 10261 x 5120 x 15360 760 -> 690; SwiGLU, half the output and two transcendental instructions for each:
+  // 7756 x 1536 x 2 x 3072 92 -> 88, 32760 x 5120 x 2 x 13824 3734 -> 3675 us.
   T* og = (T*)p.out;
+  int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));  // the lane's number anew: not kept through the loop
+  asm volatile("" : "+v"(el));
+  const int el32 = el & 31, eh = el >> 5;
+  MSD_LDS char* stage = smem + wave * 4 * 8192;
   auto write_tile = [&](auto bias_c) __attribute__((always_inline)) {
     constexpr bool BIAS = decltype(bias_c)::value;
+    constexpr int NWO = SWIGLU ? 1 : 2;  // output blocks per 64 rows
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
       // the bias of this block's columns, fetched once for all rows (columns past the end read column 0: never stored)
@@ -375,23 +386,18 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
         for (int w = 0; w < 2; ++w)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const int col = f0 + (SWIGLU ? 0 : w * 128) + wn * 64 + nb * 32 + 8 * j + 4 * h;
+            const int col = f0 + (SWIGLU ? 0 : w * 128) + wn * 64 + nb * 32 + 8 * j + 4 * eh;
             bias_r[w][j] = *(const f32x4_t*)(p.bias + (SWIGLU ? w * half : 0) + (col < p.Nout ? col : 0));
           }
       }
 #pragma unroll
       for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb) {
-          const int m = m0 + a * 128 + wm * 64 + mb * 32 + l32;
-          T* orow = og + (long long)m * p.Nout;
+        for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-          for (int w = 0; w < (SWIGLU ? 1 : 2); ++w)
+          for (int w = 0; w < NWO; ++w)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              const int ncol = wn * 64 + nb * 32 + 8 * j + 4 * h;  // first of the four columns, tile-local
-              const int col = f0 + (SWIGLU ? 0 : w * 128) + ncol;
-              const bool col_ok = col < p.Nout;
               float v[4];
               if (SWIGLU) {
                 f32x4_t bg = {0.f, 0.f, 0.f, 0.f}, bu = {0.f, 0.f, 0.f, 0.f};
@@ -411,13 +417,27 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = acc[a][w][mb][nb][4 * j + e] + bv[e];
               }
-              if (m < p.M && col_ok) {
-                T t4[4] = {E::from_float(v[0]), E::from_float(v[1]), E::from_float(v[2]), E::from_float(v[3])};
-                *(i32x2_t*)(orow + col) = *(const i32x2_t*)t4;
-              }
+              const T t4[4] = {E::from_float(v[0]), E::from_float(v[1]), E::from_float(v[2]), E::from_float(v[3])};
+              const int r = mb * 32 + el32;
+              *(MSD_LDS i32x2_t*)(stage + (a * 2 + w) * 8192 + r * 128 + (((nb * 4 + j) ^ ((r >> 1) & 7)) << 4) + 8 * eh) =
+                  *(const i32x2_t*)t4;
             }
-        }
     }
+    __builtin_amdgcn_wave_barrier();  // (a wave's LDS operations execute in order)
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int w = 0; w < NWO; ++w) {
+        __builtin_amdgcn_sched_barrier(0);
+        const int col = f0 + w * 128 + wn * 64 + (el & 7) * 8;  // (Nout is a multiple of 8: a chunk is inside or outside)
+        T* ob = og + (long long)(m0 + a * 128 + wm * 64) * p.Nout + col;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int r = i * 8 + (el >> 3);
+          const i32x4_t v = *(MSD_LDS const i32x4_t*)(stage + (a * 2 + w) * 8192 + r * 128 + (((el & 7) ^ ((r >> 1) & 7)) << 4));
+          if (m0 + a * 128 + wm * 64 + r < p.M && col < p.Nout) *(i32x4_t*)(ob + (long long)r * p.Nout) = v;
+        }
+      }
   };
   if (p.bias) write_tile(std::true_type{});
   else write_tile(std::false_type{});
@@ -603,7 +623,9 @@ __global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_smal
     if (kb + 2 < k_blocks) step(kb + 2, std::integral_constant<int, 2>{}, fx, fy);
     if (kb + 3 < k_blocks) step(kb + 3, std::integral_constant<int, 3>{}, fy, fx);
   }
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // the trailing (empty) requests
+  // the trailing (empty) requests, mine and everybody's: the output is staged where they write
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  wg_barrier();
 #undef MSD_WAIT_VM
 
   // lane: X row l32 of its blocks, W rows 8 * j + 4 * h + e of its blocks: four consecutive columns per quad
@@ -619,23 +641,31 @@ __global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_smal
         bias[nb][j] = *(const f32x4_t*)(p.bias + (row < p.Nw ? row : 0));
       }
   }
+  // through LDS as in mxfp8_gemm_kernel: the wave's TM/2 rows of kCols columns, full 64- or 128-byte lines to a row
+  constexpr int kCols = SWIGLU ? 32 : TN / 2, kRow = 2 * kCols, kChunks = kRow / 16;
+  MSD_LDS char* stage = smem + wave * (TM / 2) * kRow;
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int m = m0 + wm * (TM / 2) + mb * 32 + l32;
-    T* orow = (T*)p.out + (long long)m * p.Nout;
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int nb = 0; nb < (SWIGLU ? 1 : NB); ++nb)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int col = f0 + (SWIGLU ? wn * 32 : wn * (TN / 2) + nb * 32) + 8 * j + 4 * h;
         T t4[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float g = acc[mb][nb][4 * j + e] + bias[nb][j][e];
           t4[e] = E::from_float(SWIGLU ? silu_mul(g, acc[mb][NB - 1][4 * j + e] + bias[NB - 1][j][e]) : g);
         }
-        if (m < p.M && col < p.Nout) *(i32x2_t*)(orow + col) = *(const i32x2_t*)t4;
+        const int r = mb * 32 + l32;
+        *(MSD_LDS i32x2_t*)(stage + r * kRow + (((nb * 4 + j) ^ ((r >> 1) & (kChunks - 1))) << 4) + 8 * h) = *(const i32x2_t*)t4;
       }
+  __builtin_amdgcn_wave_barrier();
+  const int c = lane % kChunks, col = f0 + wn * kCols + c * 8;  // (Nout is a multiple of 8: a chunk is inside or outside)
+#pragma unroll
+  for (int i = 0; i < TM / 2 * kChunks / 64; ++i) {
+    const int r = i * (64 / kChunks) + lane / kChunks, m = m0 + wm * (TM / 2) + r;
+    const i32x4_t v = *(MSD_LDS const i32x4_t*)(stage + r * kRow + ((c ^ ((r >> 1) & (kChunks - 1))) << 4));
+    if (m < p.M && col < p.Nout) *(i32x4_t*)((T*)p.out + (long long)m * p.Nout + col) = v;
   }
 #endif
 }
