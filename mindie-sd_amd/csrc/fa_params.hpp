@@ -220,6 +220,11 @@ int launch_fa16_d64(const FaParams& p, int dtype, hipStream_t stream, int gen = 
 // head dims below 64 (multiples of 8), computed as 64
 int launch_fa16_d64_padded(const FaParams& p, int dtype, int D, hipStream_t stream, int gen = 0, int rows = 256);
 
+// Dense attention at head_dim 128 over at most 256 keys that a workgroup keeps in LDS (flash_attn_keys.hip); `preferred`:
+// the call has them, and enough query rows for it to pay.
+bool fa16_keys_preferred(const FaParams& p);
+int launch_fa16_keys(const FaParams& p, int dtype, hipStream_t stream);
+
 // Attention at head dims above 128 up to 256 (flash_attn_d256.hip; multiples of 8, computed as 256); `gen` as for
 // launch_fa16_d64 (its packed tiles are 128 rows); `supported` as above.
 bool fa16_d256_supported(const FaParams& p);

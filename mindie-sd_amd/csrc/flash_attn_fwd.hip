@@ -1643,7 +1643,9 @@ int mindiesd_flash_attention_fwd(const void* q, const void* k, const void* v, vo
   // A few key tiles per query tile (cross attention over a short text): the launch is mostly reading Q and writing O,
   // and two 4-wave workgroups per CU overlap one's memory phases with the other's tiles better than one 8-wave
   // workgroup does (75600 queries x 40 heads: 0.42 vs 0.53 ms at 77 keys, 0.62 vs 0.70 at 226, equal at 512).
+  // At most 256 keys and enough rows: the kernel that keeps them in LDS (flash_attn_keys.hip).
   // (More keys than that: launch_fa16_rounds, but for the grids that rest_on_four_waves describes.)
+  if (forced_tile_rows() == 0 && fa16_keys_preferred(p)) return launch_fa16_keys(p, dtype, stream);
   if (Skv <= kShortKv || forced_tile_rows() == 128 || rest_on_four_waves(p)) {
     if (dtype == MSD_DTYPE_BF16) return launch_fa<MSD_DTYPE_BF16, 4, 32, 64, false, 1, 1>(p, stream);
     return launch_fa<MSD_DTYPE_F16, 4, 32, 64, false, 1, 1>(p, stream);
