@@ -1243,9 +1243,20 @@ __global__ __launch_bounds__(NWAVES * 64, 1) void fa_fwd16_kernel(const FaParams
       }
     }
   } else {
-    for (int t = 0; t < tiles; t += 2) {
+    // Causal: of the tiles that the workgroup's last rows see, the last ones lie beyond this wave's last row; it only helps to
+    // stage them and meets the others at the barrier (short sequences spend a third of their
+    // tiles on the diagonal: 5 sequences of 9000 tokens, 24 heads, 150.6 -> 146.6 us, 11 of 12755, 20 heads, 141 -> 135 us).
+    const int mine = causal ? min(tiles, max(0, (row0 + 31 + causal_shift + BN) / BN)) : tiles;
+    for (int t = 0; t < mine; t += 2) {
       tile_step(std::integral_constant<int, 0>{}, t * BN, t + 1 < tiles ? (t + 1) * BN : -1);
-      if (t + 1 < tiles) tile_step(std::integral_constant<int, 1>{}, (t + 1) * BN, t + 2 < tiles ? (t + 2) * BN : -1);
+      if (t + 1 < mine) tile_step(std::integral_constant<int, 1>{}, (t + 1) * BN, t + 2 < tiles ? (t + 2) * BN : -1);
+    }
+    if constexpr (gen && !keymask) {
+      for (int t = mine; t < tiles; ++t) {
+        if (t + 1 < tiles) load_tile((t + 1) * BN, (t + 1) & 1);
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        __syncthreads();
+      }
     }
   }
 
