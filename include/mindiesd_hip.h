@@ -97,6 +97,11 @@ int mindiesd_flash_attention_packed_fwd(const void* q, const void* k, const void
 int mindiesd_varlen_meta(const int* cu_seqlens_q, const int* cu_seqlens_k, int B, int total_q, int total_k,
                          int max_q, int max_k, int* seq_meta, hipStream_t stream);
 
+/* The same, and zeros for the rows of `out` ([total_q] rows of row_bytes, a multiple of 16, without gaps) that no sequence
+ * covers; every row when the query table decreases, leaves the tensor or names a sequence longer than max_q. */
+int mindiesd_varlen_meta_fill(const int* cu_seqlens_q, const int* cu_seqlens_k, int B, int total_q, int total_k, int max_q,
+                              int max_k, int* seq_meta, void* out, int row_bytes, hipStream_t stream);
+
 /* ---- block-sparse attention ------------------------------------------------------------------------
  * Query block i (128 rows) of (b, n) attends to the 128-key blocks blk_idx[b][n][i][0 .. blk_cnt[b][n][i])
  * (ascending ids, int32, row pitch kb_stride); an empty list gives zeros.  `order` (optional,

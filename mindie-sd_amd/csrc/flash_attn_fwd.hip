@@ -1411,14 +1411,42 @@ static int launch_fa(const FaParams& p, hipStream_t stream) {
 }
 
 // cumulative lengths (device) -> the [B][4] table of the packed / general entry points, clamped to the tensors
-__global__ void varlen_meta_kernel(const int* cu_q, const int* cu_k, int B, int total_q, int total_k, int max_q,
-                                   int max_k, int* meta) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
+__device__ __forceinline__ void varlen_meta_entry(const int* cu_q, const int* cu_k, int b, int total_q, int total_k, int max_q,
+                                                  int max_k, int* meta) {
   const int q0 = min(max(cu_q[b], 0), total_q), k0 = min(max(cu_k[b], 0), total_k);
   const int lq = min(min(max(cu_q[b + 1] - cu_q[b], 0), total_q - q0), max_q);
   const int lk = min(min(max(cu_k[b + 1] - cu_k[b], 0), total_k - k0), max_k);
   *(i32x4_t*)(meta + 4 * b) = i32x4_t{q0, lq, k0, lk};
+}
+__global__ void varlen_meta_kernel(const int* cu_q, const int* cu_k, int B, int total_q, int total_k, int max_q,
+                                   int max_k, int* meta) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b < B) varlen_meta_entry(cu_q, cu_k, b, total_q, total_k, max_q, max_k, meta);
+}
+
+// The same, and zeros for the rows of `out` (row_chunks x 16 bytes each, no gaps) that no sequence covers.  A table whose entries
+// do not decrease, stay inside the tensor and lie at most max_q apart covers the rows from its first entry to its last; with any
+// other one every row is cleared, as sequences that overlap or were cut may leave tiles uncomputed.  A workgroup looks after
+// kFillRows rows and reads the table; where all of its rows are covered that is all it does.  Clearing the whole output in a
+// launch of its own, 65 MB for 12755 tokens x 20 heads, was 10 us and a gap of
+// 149, now 3: 24 heads x 10028 tokens 300 -> 291 us, 8 x 2973 26.4 -> 23.3 us.
+constexpr int kFillRows = 32;
+__global__ __launch_bounds__(256) void varlen_meta_fill_kernel(const int* cu_q, const int* cu_k, int B, int total_q, int total_k,
+                                                               int max_q, int max_k, int* meta, i32x4_t* out, int row_chunks) {
+  const int t = threadIdx.x;
+  for (int b = blockIdx.x * 256 + t; b < B; b += gridDim.x * 256) varlen_meta_entry(cu_q, cu_k, b, total_q, total_k, max_q, max_k, meta);
+  bool regular = true;
+  for (int b = t; b < B; b += 256) {
+    const int first = cu_q[b], next = cu_q[b + 1];
+    regular = regular && first >= 0 && next >= first && next <= total_q && next - first <= max_q;
+  }
+  regular = __syncthreads_and(regular) != 0;
+  const int covered0 = regular ? cu_q[0] : 0, covered1 = regular ? cu_q[B] : 0;
+  const int row0 = blockIdx.x * kFillRows, row1 = min(row0 + kFillRows, total_q);
+  for (int r = row0; r < row1; ++r) {
+    if (r >= covered0 && r < covered1) continue;
+    for (int c = t; c < row_chunks; c += 256) out[(long long)r * row_chunks + c] = i32x4_t{0, 0, 0, 0};
+  }
 }
 
 }  // namespace msd
@@ -1782,6 +1810,16 @@ int mindiesd_varlen_meta(const int* cu_seqlens_q, const int* cu_seqlens_k, int B
   if ((uintptr_t)seq_meta & 15) return MSD_ERR_BAD_ARG;
   hipLaunchKernelGGL(varlen_meta_kernel, dim3((B + 255) / 256), dim3(256), 0, stream, cu_seqlens_q, cu_seqlens_k, B,
                      total_q, total_k, max_q, max_k, seq_meta);
+  return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
+}
+
+int mindiesd_varlen_meta_fill(const int* cu_seqlens_q, const int* cu_seqlens_k, int B, int total_q, int total_k, int max_q,
+                              int max_k, int* seq_meta, void* out, int row_bytes, hipStream_t stream) {
+  if (!cu_seqlens_q || !cu_seqlens_k || !seq_meta || !out || B <= 0 || total_q <= 0 || total_k < 0 || max_q < 0 || max_k < 0)
+    return MSD_ERR_BAD_ARG;
+  if ((((uintptr_t)seq_meta | (uintptr_t)out) & 15) || row_bytes <= 0 || (row_bytes & 15)) return MSD_ERR_BAD_ARG;
+  hipLaunchKernelGGL(varlen_meta_fill_kernel, dim3((total_q + kFillRows - 1) / kFillRows), dim3(256), 0, stream, cu_seqlens_q,
+                     cu_seqlens_k, B, total_q, total_k, max_q, max_k, seq_meta, (i32x4_t*)out, row_bytes / 16);
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
 }
 

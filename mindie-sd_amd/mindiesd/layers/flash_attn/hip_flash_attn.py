@@ -120,16 +120,20 @@ def flash_attention(query, key, value, scale, layout="BNSD", return_lse=False, a
     return (out, lse) if return_lse else out
 
 
-def _varlen_meta(cu_q, cu_k, total_q, total_k, device, max_q=None, max_k=None):
+def _on_gpu(cu):
+    return isinstance(cu, torch.Tensor) and cu.is_cuda
+
+
+def _varlen_meta(cu_q, cu_k, total_q, total_k, device, max_q=None, max_k=None, out=None):
     """Cumulative lengths -> (int32 [B, 4] device table {first query token, query count, first key token, key
     count}, longest query count, longest key count, B).  Host lists / CPU tensors are validated and give exact
     bounds; device tensors are turned into the table on the device without a host synchronisation - the bounds
     are then the token totals (workgroups past a sequence's end return at once) unless the caller names the longest
     sequences (``max_q`` / ``max_k``), and the entries are clamped to the tensors instead of validated: a malformed
     device table cannot be rejected without reading it back, so it yields clamped sequences, never an access outside
-    the tensors."""
-    on_device = isinstance(cu_q, torch.Tensor) and cu_q.is_cuda and isinstance(cu_k, torch.Tensor) and cu_k.is_cuda
-    if on_device:
+    the tensors.  With ``out`` (device tables only, contiguous [total_q, ...]) the rows that no sequence covers are cleared in the
+    same launch."""
+    if _on_gpu(cu_q) and _on_gpu(cu_k):
         if cu_q.dim() != 1 or cu_k.dim() != 1 or cu_q.shape[0] != cu_k.shape[0] or cu_q.shape[0] < 2:
             raise ParametersInvalid("cu_seqlens_q and cu_seqlens_k must be 1-D with batch_size + 1 entries each.")
         cq = cu_q.to(device=device, dtype=torch.int32).contiguous()   # no copies when they already are int32
@@ -137,9 +141,13 @@ def _varlen_meta(cu_q, cu_k, total_q, total_k, device, max_q=None, max_k=None):
         bound_q = total_q if max_q is None else max(min(int(max_q), total_q), 1)
         bound_k = total_k if max_k is None else max(min(int(max_k), total_k), 0)
         meta = torch.empty((cq.shape[0] - 1, 4), dtype=torch.int32, device=device)
+        args = (cq.data_ptr(), ck.data_ptr(), cq.shape[0] - 1, total_q, total_k, bound_q, bound_k, meta.data_ptr())
         with _native.on_device(device):
-            rc = _native.lib().mindiesd_varlen_meta(cq.data_ptr(), ck.data_ptr(), cq.shape[0] - 1, total_q, total_k,
-                                                    bound_q, bound_k, meta.data_ptr(), _native.stream_ptr(device))
+            if out is None:
+                rc = _native.lib().mindiesd_varlen_meta(*args, _native.stream_ptr(device))
+            else:
+                rc = _native.lib().mindiesd_varlen_meta_fill(*args, out.data_ptr(), out.numel() // total_q * out.element_size(),
+                                                             _native.stream_ptr(device))
         _native.check(rc, "mindiesd_varlen_meta")
         return meta, bound_q, max(bound_k, 1), cq.shape[0] - 1
     def lengths(cu, name):
@@ -174,12 +182,14 @@ def flash_attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, scale, causal=Fa
     if q.dim() != 3 or k.shape != v.shape or k.dim() != 3 or q.shape[1] % k.shape[1] != 0:
         raise ParametersInvalid("Inconsistent query/key/value shapes.")
     q, k, v = _aligned(q), _aligned(k), _aligned(v)
-    unchecked = isinstance(cu_seqlens_q, torch.Tensor) and cu_seqlens_q.is_cuda
-    out = (torch.zeros if unchecked else torch.empty)(q.shape, dtype=q.dtype, device=q.device)
+    unchecked = _on_gpu(cu_seqlens_q)
+    # rows outside of a device table: cleared by the launch that reads it (every workgroup of it reads all of the table)
+    fill = unchecked and _on_gpu(cu_seqlens_k) and q.shape[1] > 0 and cu_seqlens_q.numel() <= 4096
+    out = (torch.zeros if unchecked and not fill else torch.empty)(q.shape, dtype=q.dtype, device=q.device)
     if q.shape[0] == 0:
         return out
     meta_t, max_q, max_k, nseq = _varlen_meta(cu_seqlens_q, cu_seqlens_k, q.shape[0], k.shape[0], q.device,
-                                              max_seqlen_q, max_seqlen_k)
+                                              max_seqlen_q, max_seqlen_k, out if fill else None)
     if max_q == 0:
         return out
     tn = lambda t: (0, t.stride(1), t.stride(0))  # (batch, head, token) strides of a [T, N, D] tensor

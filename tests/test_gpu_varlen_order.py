@@ -35,3 +35,28 @@ def test_longest_first(nseq, d, on_gpu):
         elif lens_q[i]:
             want = reference(*(x.transpose(0, 1).unsqueeze(0) for x in (q[cu_q[i]:cu_q[i + 1]], k[ks], v[ks])))
             check(part.transpose(0, 1).unsqueeze(0), want, v[ks], torch.bfloat16)
+
+
+@pytest.mark.parametrize("table, total, max_q, covered", [
+    ([0, 40, 100], 100, None, (0, 100)),             # all rows
+    ([0, 40, 97], 100, None, (0, 97)),               # a rest, inside a workgroup's rows
+    ([33, 33, 64, 64], 97, None, (33, 64)),          # a gap on either side, empty sequences
+    ([0, 0], 70, None, (0, 0)),                      # nothing
+    ([0, 60, 40, 100], 100, None, (0, 0)),           # decreasing: sequences overlap
+    ([-5, 40, 100], 100, None, (0, 0)),              # outside of the tensor
+    ([0, 40, 101], 100, None, (0, 0)),
+    ([0, 40, 100], 100, 59, (0, 0)),                 # a sequence longer than the longest one named
+    ([0, 40, 100], 100, 60, (0, 100)),
+    (list(range(0, 2001, 4)), 2003, None, (0, 2000)),  # more sequences than a workgroup has threads
+])
+def test_rows_outside_of_a_device_table_are_cleared(cuda, table, total, max_q, covered):
+    """The launch that builds the table clears exactly the rows that no sequence covers, and every row when the table is not one
+    that the attention kernels cover whole; the table itself is that of mindiesd_varlen_meta."""
+    from mindiesd.layers.flash_attn.hip_flash_attn import _varlen_meta
+    cu = torch.tensor(table, dtype=torch.int32, device=cuda)
+    out = torch.ones(total, 3, 24, dtype=torch.float16, device=cuda)
+    meta, *_ = _varlen_meta(cu, cu, total, total, cu.device, max_q, None, out)
+    want, *_ = _varlen_meta(cu, cu, total, total, cu.device, max_q, None)
+    assert torch.equal(meta, want)
+    assert (out[covered[0]:covered[1]] == 1).all()
+    assert not out[:covered[0]].any() and not out[covered[1]:].any()
