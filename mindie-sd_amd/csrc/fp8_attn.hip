@@ -20,6 +20,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "fa16_work.hpp"
 
 // (batch x head) pairs that mindiesd_fp8_v_quant_static accepts: its scratch is a fixed device array
 #define MINDIESD_FP8_V_QUANT_STATIC_MAX_HEADS 4096
@@ -465,6 +466,7 @@ struct Fp8Params {
   int B, N, Sq, Skv, S128;
   float scale_log2;  // softmax scale * log2(e)
   int k_shift;       // a K scale covers 128 << k_shift keys
+  int tail_full;     // tiles of 256 rows that an XCD computes whole; each of the others of its run goes as two workgroups
 };
 
 // Two rules for the E4M3 probabilities of a tile (x = score - reference maximum, in log2 units):
@@ -511,14 +513,13 @@ __global__ __launch_bounds__(512, 2) void fp8_fa_fwd_kernel(const Fp8Params p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, h = lane >> 5;
 
-  const int q_tiles = (p.Sq + BM - 1) / BM;
-  const int total = p.B * p.N * q_tiles;
-  const int per_xcd = (total + 7) / 8;
-  const int work = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (work >= total) return;
-  const int bn = work / q_tiles, qt = work - bn * q_tiles;
-  const int b = bn / p.N, n = bn - b * p.N;
-  const int q0 = qt * BM;
+  const fa16::Part work = fa16::runs_tail(blockIdx.x, p.B * p.N, (p.Sq + BM - 1) / BM, p.tail_full, 2);
+  if (work.group < 0) return;
+  const int bn = work.group, b = bn / p.N, n = bn - b * p.N;
+  const int q0 = work.tile * BM + (work.part == 1 ? BM / 2 : 0);
+  if (q0 >= p.Sq) return;
+  // of a half tile's workgroup the waves 4 .. 7 own no rows: they stage keys with the others, which then have their SIMD alone
+  const bool busy = work.part < 0 || wave < NW / 2;
   const int qblocks = (p.Sq + 127) / 128, kblocks = (p.Skv + 127) / 128;
   const int n_tiles = kblocks;
 
@@ -764,14 +765,22 @@ __global__ __launch_bounds__(512, 2) void fp8_fa_fwd_kernel(const Fp8Params p) {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
-  for (int t = 0; t < n_tiles; t += 3) {
+  const int my_tiles = busy ? n_tiles : 0;
+  for (int t = 0; t < my_tiles; t += 3) {
     tile_step(t, std::integral_constant<int, 0>{});
     if (t + 1 < n_tiles) tile_step(t + 1, std::integral_constant<int, 1>{});
     if (t + 2 < n_tiles) tile_step(t + 2, std::integral_constant<int, 2>{});
   }
+  for (int t = my_tiles, stage = 2; t < n_tiles; ++t) {
+    load_tile(t + 2, stage);
+    stage = stage == 2 ? 0 : stage + 1;
+    __builtin_amdgcn_s_waitcnt(0x0f74);
+    __builtin_amdgcn_s_barrier();
+  }
   // the requests past the last tile still write into the stages, which the output staging reuses
   __builtin_amdgcn_s_waitcnt(0x0f70);
   __syncthreads();
+  if (!busy) return;
 
   // ---- epilogue: 1/l, per-channel V scale, transpose through LDS, coalesced store -----------------------------------
   // (the 2^kPShift factor is in both the accumulator and the running sum, so it cancels)
@@ -964,9 +973,16 @@ int mindiesd_fp8_attention_fwd(const void* q8, const void* k8, const void* v8t, 
   p.B = B; p.N = N; p.Sq = Sq; p.Skv = Skv; p.S128 = S128;
   p.scale_log2 = scale * 1.4426950408889634f;
   p.k_shift = (flags & MSD_FP8_K_BLOCK_256) ? 1 : 0;
-  const int q_tiles = (Sq + 255) / 256;
-  const int total = B * N * q_tiles;
-  const int grid = (total + 7) / 8 * 8;
+  // An XCD runs its tiles in rounds of 32, one to a CU.  A last round of at most 16 goes as half tiles, which still is one round,
+  // and takes 0.7 of a whole one (one wave to a SIMD); a row's bits are the same in either.  The module, whole -> cut: 4 / 8 / 16
+  // tiles per XCD (8 heads x 1024 / 2000 / 4000) 30.6 -> 26.3, 46.2 -> 38.4, 74.9 -> 60.7 us, 64 + 1 (40 x 3300) 200 -> 188, 96 + 14
+  // (40 x 5500) 397 -> 379, 192 + 6 (20 x 20000) 2096 -> 2031, 256 + 2 (24 x 22000) 2990 -> 2919; from 16 whole rounds on it would be 1 %.
+  const long long q_tiles = (Sq + 255) / 256, per_xcd = ((long long)B * N * q_tiles + 7) / 8;
+  if (per_xcd >= (1ll << 27)) return MSD_ERR_UNSUPPORTED;
+  const int rest = (int)(per_xcd % (kCus / 8));
+  const bool cut = rest != 0 && 2 * rest <= kCus / 8 && per_xcd < 16 * (kCus / 8);
+  p.tail_full = (int)(cut ? per_xcd - rest : per_xcd);
+  const int grid = (int)fa16::runs_tail_grid((long long)B * N, q_tiles, p.tail_full, 2);
   const bool bf = out_dtype == MSD_DTYPE_BF16;
   const bool p2 = (flags & MSD_FP8_LOG2_DOMAIN) != 0, pl = (flags & MSD_FP8_P_EXP2) == 0;
   if (p2 && pl) return bf ? fp8_fa_launch<MSD_DTYPE_BF16, true, true>(p, grid, stream)

@@ -278,3 +278,18 @@ def test_one_call_has_the_bits_of_its_parts(cuda, sq, skv, rotated, dtype, layou
     want = fp8_attention_quantized(*parts[0], *parts[1], *quantize_v_per_channel(v, layout), 0.09, dtype, layout, p_rule=rule)
     got = fp8_attention_forward(q, k, v, 0.09, layout, q_rot, k_rot, p_rule=rule)
     assert torch.isfinite(got.float()).all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rule", ["linear", "exp2"])
+@pytest.mark.parametrize("s", [1, 128, 129, 256, 257, 385, 700, 2000, 4096])
+def test_half_tiles_have_the_bits_of_whole_ones(cuda, s, rule):
+    """8 heads: at most 16 tiles of 256 rows per XCD, which go as half tiles; the same heads among so many that each XCD has 17
+    to 32 tiles, which stay whole."""
+    from mindiesd.layers.quant.fp8_attention import fp8_attention_forward
+    tiles = -(-s // 256)
+    heads = 8 * -(-17 // tiles)
+    assert 1 <= tiles <= 16 < tiles * heads // 8 <= 32
+    q, k, v = (t.to(cuda) for t in _outlier_inputs((1, heads, s, 128), seed=s))
+    many = fp8_attention_forward(q, k, v, p_rule=rule)
+    few = fp8_attention_forward(q[:, :8], k[:, :8], v[:, :8], p_rule=rule)
+    assert torch.isfinite(few.float()).all() and torch.equal(few, many[:, :8])
