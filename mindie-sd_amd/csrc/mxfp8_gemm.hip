@@ -449,8 +449,8 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
 }
 
 // ---- GEMM on smaller tiles, for grids that 256 x 256 tiles leave mostly empty -------------------------------------------
-// Same operand formats, LDS swizzle and matrix instruction as mxfp8_gemm_kernel.  4 waves own a TM x TN tile (TM, TN 64 or
-// 128; a wave TM/2 x TN/2), K is walked in blocks of 128 codes: a stage holds the block of all TM + TN rows, four stages
+// Same operand formats, LDS swizzle and matrix instruction as mxfp8_gemm_kernel.  4 waves own a TM x TN tile (64 x 64,
+// 64 x 128 and 128 x 128: a wave half of it either way; 128 x 96: a wave 32 rows of it), K is walked in blocks of 128 codes: a stage holds the block of all TM + TN rows, four stages
 // form a ring (one being read into registers, one landed, two in flight), operands of the next block are read from LDS
 // while the matrix core works on the current one (two register sets).
 //
@@ -460,14 +460,16 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
 // the matrix pipe is busy 30 % of those CUs' cycles.  Neither deeper prefetch into the L2 by a fifth wave nor a split of K over
 // several workgroups (fp32 sums through memory, 29 to 47 us) was faster.  Plain GEMM, M x N x K, 256 x 256 tiles before -> now:
 // 512 x 5120 x 5120 57.5 -> 23.8 us, 128 x 5120 x 5120 51.5 -> 12.4 us, 64 x 1536 x 1536 19.5 -> 4.9 us, the weights in the
-// memory-side cache; the layer with its quantisation 62.7 -> 29.6 us at 512 x 5120 x 5120, and 70.7 -> 37.4 with weights in no cache.
+// memory-side cache; the layer with its quantisation 62.7 -> 29.6 us at 512 x 5120 x 5120 (24.8 with 96 columns to a tile, full lines
+// stored, one native call), and 70.7 -> 37.4 with weights in no cache (before those three).
 template <int DT, bool SWIGLU, int TM, int TN>
 __global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_small_kernel(const GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using E = Elem<DT>;
   using T = typename E::type;
   constexpr int BK = 128, NS = 4, ROWS = TM + TN;
-  constexpr int MB = TM / 64, NB = TN / 64;   // 32 x 32 blocks of a wave
+  constexpr int WN = TN % 64 == 0 ? 2 : 1, WM = 4 / WN;     // waves beside and below one another
+  constexpr int MB = TM / (32 * WM), NB = TN / (32 * WN);   // 32 x 32 blocks of a wave
   constexpr int kStage = ROWS * BK;
   constexpr int kDma = ROWS / 32;             // DMA instructions of a wave and stage (8 rows of 128 bytes each)
   static_assert(!SWIGLU || NB == 2, "gate and up rows of an output column are the two column blocks of a wave");
@@ -476,7 +478,7 @@ __global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_smal
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, h = lane >> 5;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / WN, wn = wave % WN;
 
   // tile order: consecutive tiles of an XCD share their W panel (X is the small operand here)
   const int per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
@@ -538,7 +540,7 @@ __global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_smal
     i32x8_t a[MB][2], w[NB][2];  // [block][k step]
     int as[MB], ws[NB];
   };
-  const int a_row = wm * (TM / 2) + l32, wr_row = TM + wn * (TN / 2) + l32;
+  const int a_row = wm * (TM / WM) + l32, wr_row = TM + wn * (TN / WN) + l32;
   // one of the 16-byte reads of a block's operands (X blocks, then W blocks; k step 0 first) or, index -1, its scales
   constexpr int kReads = 4 * (MB + NB);
   auto read_piece = [&](int kb, int slot, Frag& f, auto r_c) __attribute__((always_inline)) {
@@ -641,13 +643,15 @@ __global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_smal
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int row = w_row(wn * (TN / 2) + nb * 32 + 8 * j + 4 * h);  // rows past the end: never stored
+        const int row = w_row(wn * (TN / WN) + nb * 32 + 8 * j + 4 * h);  // rows past the end: never stored
         bias[nb][j] = *(const f32x4_t*)(p.bias + (row < p.Nw ? row : 0));
       }
   }
   // through LDS as in mxfp8_gemm_kernel: the wave's TM/2 rows of kCols columns, full 64- or 128-byte lines to a row
-  constexpr int kCols = SWIGLU ? 32 : TN / 2, kRow = 2 * kCols, kChunks = kRow / 16;
-  MSD_LDS char* stage = smem + wave * (TM / 2) * kRow;
+  // (96 columns: rows padded by a chunk instead of the XOR)
+  constexpr int kCols = SWIGLU ? 32 : TN / WN, kChunks = kCols / 8;
+  constexpr int kSwz = (kChunks & (kChunks - 1)) == 0 ? kChunks - 1 : 0, kRow = 16 * (kSwz ? kChunks : kChunks + 1), kRows = TM / WM;
+  MSD_LDS char* stage = smem + wave * kRows * kRow;
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -661,14 +665,14 @@ __global__ __launch_bounds__(256, (TM + TN <= 128 ? 2 : 1)) void mxfp8_gemm_smal
           t4[e] = E::from_float(SWIGLU ? silu_mul(g, acc[mb][NB - 1][4 * j + e] + bias[NB - 1][j][e]) : g);
         }
         const int r = mb * 32 + l32;
-        *(MSD_LDS i32x2_t*)(stage + r * kRow + (((nb * 4 + j) ^ ((r >> 1) & (kChunks - 1))) << 4) + 8 * h) = *(const i32x2_t*)t4;
+        *(MSD_LDS i32x2_t*)(stage + r * kRow + (((nb * 4 + j) ^ ((r >> 1) & kSwz)) << 4) + 8 * h) = *(const i32x2_t*)t4;
       }
   __builtin_amdgcn_wave_barrier();
-  const int c = lane % kChunks, col = f0 + wn * kCols + c * 8;  // (Nout is a multiple of 8: a chunk is inside or outside)
 #pragma unroll
-  for (int i = 0; i < TM / 2 * kChunks / 64; ++i) {
-    const int r = i * (64 / kChunks) + lane / kChunks, m = m0 + wm * (TM / 2) + r;
-    const i32x4_t v = *(MSD_LDS const i32x4_t*)(stage + r * kRow + ((c ^ ((r >> 1) & (kChunks - 1))) << 4));
+  for (int i = 0; i < kRows * kChunks / 64; ++i) {
+    const int r = (i * 64 + lane) / kChunks, c = (i * 64 + lane) % kChunks;
+    const int m = m0 + wm * kRows + r, col = f0 + wn * kCols + c * 8;  // (Nout is a multiple of 8: a chunk is inside or outside)
+    const i32x4_t v = *(MSD_LDS const i32x4_t*)(stage + r * kRow + ((c ^ ((r >> 1) & kSwz)) << 4));
     if (m < p.M && col < p.Nout) *(i32x4_t*)((T*)p.out + (long long)m * p.Nout + col) = v;
   }
 #endif
@@ -726,13 +730,16 @@ int mindiesd_mxfp8_gemm(const void* a, const void* a_scale, const void* w, const
   p.M = M; p.K = K; p.Nw = Nw; p.Nout = swiglu ? Nw / 2 : Nw;
   // Tile choice.  A workgroup walks all of K whatever its tile, so a launch takes (rounds over the 256 CUs) x (time of a
   // tile): 64 x 64, 64 x 128, 128 x 128 and 256 x 256 tiles take 4.9 / 7.0 / 10 / 26 us at K 1536, 8 / 11 / 15.5 / 38.5 us at
-  // K 3072 and 12 / 17.5 / 23.5 / 57 us at K 5120.  Hence the smallest tile whose grid is one round; 128 x 128 tiles still win
+  // K 3072 and 12 / 17.5 / 23.5 / 57 us at K 5120.  Hence the smallest tile whose grid is one round, 128 x 96 among them for the
+  // plain product (layers at K 5120, 216 of these instead of 160 workgroups: M 512 26.2 -> 24.8 us, M 400 25.1 -> 23.9; at K 1536 and
+  // 3072 and at 240 to 256 workgroups equal within 1 %); 128 x 128 tiles still win
   // in two rounds against one round of 256 x 256 (N K 5120, M 1024: 47 against 58 us, M 1536, 480 tiles: 52 against 59), not in
   // three (M 2048, 640 tiles: 82 against 61 us).
   auto count = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((p.Nout + (swiglu ? tn / 2 : tn) - 1) / (swiglu ? tn / 2 : tn)); };
   int tm = 256, tn = 256;
   if (!swiglu && count(64, 64) <= kCus) tm = tn = 64;
   else if (count(64, 128) <= kCus) tm = 64, tn = 128;
+  else if (!swiglu && count(128, 96) <= kCus) tm = 128, tn = 96;
   else if (count(128, 128) <= (count(256, 256) <= kCus ? 2 * kCus : kCus)) tm = tn = 128;
   p.tiles_m = (M + tm - 1) / tm;
   p.tiles_n = swiglu ? (p.Nout + tn / 2 - 1) / (tn / 2) : (Nw + tn - 1) / tn;
@@ -750,6 +757,7 @@ int mindiesd_mxfp8_gemm(const void* a, const void* a_scale, const void* w, const
     constexpr int DT = decltype(dt)::value;
     if (tm == 64 && tn == 64) return launch(mxfp8_gemm_small_kernel<DT, false, 64, 64>);
     if (tm == 64) return swiglu ? launch(mxfp8_gemm_small_kernel<DT, true, 64, 128>) : launch(mxfp8_gemm_small_kernel<DT, false, 64, 128>);
+    if (tn == 96) return launch(mxfp8_gemm_small_kernel<DT, false, 128, 96>);
     if (tm == 128) return swiglu ? launch(mxfp8_gemm_small_kernel<DT, true, 128, 128>) : launch(mxfp8_gemm_small_kernel<DT, false, 128, 128>);
     return swiglu ? launch(mxfp8_gemm_kernel<DT, true>) : launch(mxfp8_gemm_kernel<DT, false>);
   };

@@ -118,6 +118,16 @@ def test_gemm_tiles_vs_oracle(cuda, m, k, nw, swiglu, want_tile, dtype):
     assert (err <= half_ulp * (1 + 2.0 ** -6) + slack + tiny).all(), float((err - half_ulp - slack).max())
 
 
+# Plain products that the rule above gives 128 x 128 tiles in one round: where 96 columns to a tile are still one round they run
+# as 128 x 96, the others do not.  Columns past a tile's edge by 8, 40 and 88, exactly 256 workgroups of either.
+@pytest.mark.parametrize("m,k,nw,columns", [(385, 1408, 5000, 96), (129, 640, 12200, 96), (512, 128, 5128, 96), (1000, 1152, 2056, 96),
+                                            (900, 640, 3080, 128), (1000, 128, 4088, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gemm_tiles_of_96_columns(cuda, m, k, nw, columns, dtype):
+    assert columns == (96 if -(-m // 128) * -(-nw // 96) <= 256 else 128)
+    test_gemm_tiles_vs_oracle(cuda, m, k, nw, False, (128, 128), dtype)
+
+
 def test_gemm_errors(cuda):
     from mindiesd import ParametersInvalid
     from mindiesd.layers.quant import mx_quantize, mxfp8_matmul
