@@ -66,6 +66,13 @@ def fp8_attention_quantized(q8, q_scale, k8, k_scale, v8t, v_scale, scale, out_d
     return out
 
 
+def _rotation(rot, device, dtype):
+    """A rotation as the kernel reads it: row major in the inputs' type, 16-byte loads (a view into a packed buffer of weights
+    may start anywhere: it is copied)."""
+    rot = rot.to(device=device, dtype=dtype).contiguous()
+    return rot.clone() if rot.data_ptr() & 15 else rot
+
+
 def _fp8_attention_one_call(query, key, value, scale, layout, q_rot, k_rot, p_rule):
     """Three launches and two allocations instead of eight and nine (20 heads x 1026 tokens: 66 us, all of it host time, now
     39 us)."""
@@ -73,7 +80,7 @@ def _fp8_attention_one_call(query, key, value, scale, layout, q_rot, k_rot, p_ru
     query, q_st = _aligned_bns(query, layout)
     key, k_st = _aligned_bns(key, layout)
     value, v_st = _aligned_bns(value, layout)
-    rots = [rot if rot is None else rot.to(device=device, dtype=dtype).contiguous() for rot in (q_rot, k_rot)]
+    rots = [rot if rot is None else _rotation(rot, device, dtype) for rot in (q_rot, k_rot)]
     b, n, sq = (query.shape[0], query.shape[1], query.shape[2]) if layout == "BNSD" else (query.shape[0], query.shape[2],
                                                                                           query.shape[1])
     skv = key.shape[2 if layout == "BNSD" else 1]

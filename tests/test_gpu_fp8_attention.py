@@ -280,6 +280,26 @@ def test_one_call_has_the_bits_of_its_parts(cuda, sq, skv, rotated, dtype, layou
     assert torch.isfinite(got.float()).all() and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("offset", [1, 4, 7])
+@pytest.mark.parametrize("rotated", ["q", "k", "qk"])
+def test_rotations_that_start_anywhere(cuda, rotated, offset):
+    """Rotations that are contiguous views into a packed buffer, off the 16 bytes that the kernel loads at a time: the bits of
+    aligned ones, through the function and through the module."""
+    from mindiesd.layers.quant.fp8_attention import fp8_attention_forward
+    from mindiesd.quantization import FP8RotateQuantFA
+    q, k, v = (t.to(cuda) for t in _outlier_inputs((1, 2, 300, 128), seed=offset))
+    buf = torch.randn(2 * 128 * 128 + 16, generator=torch.Generator().manual_seed(offset)).mul_(0.1).to(torch.bfloat16).to(cuda)
+    views = [buf[offset + at:offset + at + 128 * 128].view(128, 128) for at in (0, 128 * 128)]
+    assert all(r.is_contiguous() and r.data_ptr() % 16 for r in views)
+    pick = lambda rots: [r if name in rotated else None for name, r in zip("qk", rots)]
+    want = fp8_attention_forward(q, k, v, None, "BNSD", *pick([r.clone() for r in views]))
+    assert torch.isfinite(want.float()).all()
+    assert torch.equal(fp8_attention_forward(q, k, v, None, "BNSD", *pick(views)), want)
+    if rotated == "qk":
+        module = FP8RotateQuantFA(prefix="a", weights={"a.q_rot": views[0], "a.k_rot": views[1]})
+        assert torch.equal(module(q, k, v), want)
+
+
 @pytest.mark.parametrize("rule", ["linear", "exp2"])
 @pytest.mark.parametrize("s", [1, 128, 129, 256, 257, 385, 700, 2000, 4096])
 def test_half_tiles_have_the_bits_of_whole_ones(cuda, s, rule):
