@@ -77,8 +77,6 @@ class W8A8MXFP8QuantLinear(nn.Module):
         return mxfp8_linear(x, self.weight, self.weight_scale, self.bias, self.dtype, self.swiglu)
 
     def forward(self, x):
-        if x.ndim >= 3 and self.mul_scale is None and x.dtype == self.dtype:
-            return mxfp8_linear(x, self.weight, self.weight_scale, self.bias, self.dtype, self.swiglu)
         if x.ndim >= 3:  # the reference flattens to 2-D as well (layer.py:104-116)
             out = self.quant_matmul(x.reshape(x.shape[:-1].numel(), -1))
             return out.view(*x.shape[:-1], out.shape[1])

@@ -198,3 +198,29 @@ def test_add_fa_quant_only_for_fp8_dynamic():
     other = nn.Linear(10, 10)
     add_fa_quant(other, QuantAlgorithm.NO_QUANT, "test_layer", weights)
     assert not hasattr(other, "fa_quant")
+
+
+@pytest.mark.parametrize("replace", ["subclass", "instance"])
+@pytest.mark.parametrize("shape", [(6, 256), (2, 3, 256), (2, 1, 3, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_every_linear_call_goes_through_quant_matmul(replace, shape, dtype):
+    """A quant_matmul of a subclass, or put on a layer, sees every input as rows, whatever the input's dimensions and type, and
+    the layer gives its result the input's leading dimensions."""
+    seen = []
+
+    def rows(x):
+        seen.append(x)
+        return x[:, :24].to(torch.bfloat16) * 2
+
+    class Layer(W8A8MXFP8QuantLinear):
+        def quant_matmul(self, x):
+            return rows(x)
+
+    weights = {"a.weight": torch.zeros(24, 256, dtype=torch.uint8), "a.weight_scale": torch.zeros(24, 4, 2, dtype=torch.uint8)}
+    layer = (Layer if replace == "subclass" else W8A8MXFP8QuantLinear)(256, 24, bias=False, weights=weights, prefix="a")
+    if replace == "instance":
+        layer.quant_matmul = rows
+    x = torch.arange(6 * 256).view(shape).to(dtype)
+    out = layer(x)
+    assert len(seen) == 1 and seen[0].shape == (6, 256) and seen[0].dtype == dtype
+    assert out.shape == (*shape[:-1], 24) and torch.equal(out, (x[..., :24].to(torch.bfloat16) * 2))
