@@ -61,6 +61,14 @@ def _aligned_bns(t, layout):
     return t, ((s0, s1, s2) if layout == "BNSD" else (s0, s2, s1))
 
 
+def _empty_out(query):
+    """A contiguous tensor of the query's shape, type and device for the output; a plain one also where the query is of a
+    subclass (empty_like, the cheaper of the two, would carry the class over)."""
+    if type(query) is torch.Tensor:
+        return torch.empty_like(query, memory_format=torch.contiguous_format)
+    return torch.empty(query.shape, dtype=query.dtype, device=query.device)
+
+
 def flash_attention(query, key, value, scale, layout="BNSD", return_lse=False, attn_mask=None, causal=False):
     """softmax(scale * Q K^T) V on the GPU.  ``layout`` is 'BNSD' or 'BSND'; the output has the
     input's layout and dtype.  Grouped-query attention is supported (N % N_kv == 0).
@@ -82,7 +90,7 @@ def flash_attention(query, key, value, scale, layout="BNSD", return_lse=False, a
     query, q_st = _aligned_bns(query, layout)
     key, k_st = _aligned_bns(key, layout)
     value, v_st = _aligned_bns(value, layout)
-    out = torch.empty_like(query, memory_format=torch.contiguous_format)
+    out = _empty_out(query)
     o_st = (n * sq * d, sq * d, d) if layout == "BNSD" else (n * sq * d, d, n * d)
     lse = torch.empty((b, n, sq), dtype=torch.float32, device=device) if return_lse else None
     strides = (*q_st, *k_st, *v_st, *o_st)

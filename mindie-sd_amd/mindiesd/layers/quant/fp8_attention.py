@@ -8,7 +8,7 @@ import torch
 
 from ... import _native
 from ...utils.exception import ParametersInvalid
-from ..flash_attn.hip_flash_attn import HEAD_DIM, _aligned_bns, _strides_bns
+from ..flash_attn.hip_flash_attn import HEAD_DIM, _aligned_bns, _empty_out, _strides_bns
 from .block_quant import _block_quant, _rot_block_quant
 
 
@@ -84,7 +84,7 @@ def _fp8_attention_one_call(query, key, value, scale, layout, q_rot, k_rot, p_ru
     b, n, sq = (query.shape[0], query.shape[1], query.shape[2]) if layout == "BNSD" else (query.shape[0], query.shape[2],
                                                                                           query.shape[1])
     skv = key.shape[2 if layout == "BNSD" else 1]
-    out = torch.empty_like(query, memory_format=torch.contiguous_format)
+    out = _empty_out(query)
     o_st = (n * sq * HEAD_DIM, sq * HEAD_DIM, HEAD_DIM) if layout == "BNSD" else (n * sq * HEAD_DIM, HEAD_DIM, n * HEAD_DIM)
     lib = _native.lib()
     ws_bytes = lib.mindiesd_fp8_rot_attention_workspace_size(b, n, sq, skv)

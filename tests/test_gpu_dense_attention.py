@@ -204,3 +204,21 @@ def test_tail_tile_reads_nothing_past_the_sequence(cuda, s):
     out = mindiesd.attention_forward(q.to(cuda), slabs[0], slabs[1], attn_mask=keep.to(cuda), head_first=True).cpu()
     assert not out.isnan().any()
     _check(out, ref)
+
+
+class _Tokens(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("layout", ["BNSD", "BSND"])
+@pytest.mark.parametrize("strided", [False, True])
+def test_a_query_of_a_tensor_subclass_gives_a_plain_output(cuda, layout, strided):
+    """Dense and FP8 attention: the type of the output does not follow the query's class, its bits are those of a plain query."""
+    from mindiesd.layers.flash_attn.hip_flash_attn import flash_attention
+    from mindiesd.layers.quant.fp8_attention import fp8_attention_forward
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(1, 130, 2, 256, generator=g).to(torch.bfloat16).to(cuda) for _ in range(3))
+    q, k, v = (x[..., ::2] if strided else x[..., :128] for x in (q, k, v))
+    for attend in (lambda t: flash_attention(t, k, v, 0.1, layout), lambda t: fp8_attention_forward(t, k, v, 0.1, layout)):
+        got = attend(q.as_subclass(_Tokens))
+        assert type(got) is torch.Tensor and got.is_contiguous() and torch.equal(got, attend(q))
