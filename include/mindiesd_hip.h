@@ -172,8 +172,8 @@ int mindiesd_block_sparse_attention_paired_fwd(const void* q, const void* k, con
                                                float scale, const signed char* mask, const int* token_order,
                                                void* workspace, size_t ws_bytes, hipStream_t stream);
 
-/* The same call by whichever way suits its size: paired as above, or, for masks of at most 768 rows (B * N * ceil(Sq / 128)),
- * one workgroup per mask row over its list, the longest lists first.  The result differs from the paired one by the order of
+/* The same call by whichever way suits its size: paired as above, or, for small masks (at most 768 rows, B * N * ceil(Sq / 128),
+ * of at most 64 key blocks; fewer rows over more), one workgroup per mask row over its list, the longest lists first.  The result differs from the paired one by the order of
  * accumulation only; arguments and workspace are the paired call's. */
 int mindiesd_block_sparse_attention_mask_fwd(const void* q, const void* k, const void* v, void* out, float* lse,
                                                int dtype, int B, int N, int Nkv, int Sq, int Skv, int D,

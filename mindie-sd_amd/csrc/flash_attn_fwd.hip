@@ -1597,16 +1597,25 @@ int mindiesd_block_sparse_attention_paired_fwd(const void* q, const void* k, con
                      : launch_fa<MSD_DTYPE_F16, 4, 32, 64, true, 1, 0, false, true>(p, stream);
 }
 
-// Block-sparse attention driven by the int8 mask: over paired query blocks as above, or, for small masks, one 128-row workgroup
-// per mask row, the longest rows of each XCD first (bsa_sorted_lists_kernel).  Pairing halves the K/V stream that bounds long
-// calls; with few rows the heads' keys stay in the L2 anyway, and what counts are the pairing's three launches (21 us) and the
-// 256-row workgroups, one to a CU, of which the longest end late.  rf_v3 / ada_bsa calls at sparsity 0.8, paired -> lists (the
-// former with the mask kernel's own gain of 12 us): 256 rows (8 heads x 4000 tokens) - / 78 -> 60 us, 520 (20 x 3264) 141 -> 108 /
-// 130 -> 108, 632 (8 x 10000) 286 -> 237 / 185 -> 157, 752 (8 x 12000) 331 -> 285 / 237 -> 208, 768 (24 x 4000) 164 -> 146 / 120 -> 102.
-// Above kListRows it depends on the mask: 800 (20 x 5000, sparsity 0.5) 228 -> 208 / 206 -> 207, 848 (8 x 13500) 450 -> 455 / 437 -> 469,
-// 1016 (8 x 16200, 0.6) 649 -> 597 / 463 -> 494; from 1700 rows on pairs win by up to 8 %.
+// Block-sparse attention driven by the int8 mask: over paired query blocks as above, or one 128-row workgroup per mask row, two to
+// a CU, the longest rows of each XCD first (bsa_sorted_lists_kernel).  Pairing costs three launches (21 us) and its 256-row
+// workgroups go one to a CU, of which the longest end late, but it halves the K/V stream.  Lists therefore win where the keys
+// stay in the L2 (a head's K and V take 64 KiB per key block, an XCD has 4 MiB: 64 blocks) and else only where pairs leave the
+// chip far from full.  paired / lists over rf_v3 and ada_bsa calls, sparsities 0.5 to 0.9:
+//   up to 64 key blocks, up to 768 rows (1.5 rounds): 0.98 (9 heads x 7168 tokens) to 1.6, 20 x 3264 141 -> 108 / 130 -> 108 us, 24 x 4000
+//     164 -> 146 / 120 -> 102; above, 800 rows (20 x 5000) 228 -> 208 / 206 -> 207 us and falling, from 1700 rows on 0.92 to 1;
+//   up to 96 key blocks: up to 192 pairs 1.02 to 1.3, 196 to 256 pairs 0.97 to 1.2 (5 heads x 11392 tokens 315 -> 323 / 223 -> 217 us),
+//     257 to 320 pairs, a second round almost empty, 1.0 to 1.5 (8 x 10000 286 -> 237 / 185 -> 157 us), more 0.95 to 1.2;
+//   beyond: up to 128 pairs, half the CUs, 1.03 to 1.4 (1 head x 32760 749 -> 550 / 287 -> 208 us), more 0.92 to 1.2
+//     (2 x 46800, sparsity 0.5, 1333 -> 1445 us; 4 x 24400 742 -> 766 us; 1 x 49152 ada_bsa 732 -> 767 us).
 // Workspace as for the paired entry point.
-constexpr int kListRows = 3 * kCus;
+static bool prefers_lists(long long BN, int QB, int KB) {
+  const long long rows = BN * QB, pairs = BN * ((QB + 1) / 2);
+  if (KB <= 64) return rows <= 3 * kCus;
+  if (KB <= 96) return pairs <= 192 || (pairs > kCus && pairs <= 320);
+  return pairs <= kCus / 2;
+}
+
 int mindiesd_block_sparse_attention_mask_fwd(const void* q, const void* k, const void* v, void* out, float* lse, int dtype, int B,
                                              int N, int Nkv, int Sq, int Skv, int D, long long q_sb, long long q_sn,
                                              long long q_ss, long long k_sb, long long k_sn, long long k_ss, long long v_sb,
@@ -1614,7 +1623,7 @@ int mindiesd_block_sparse_attention_mask_fwd(const void* q, const void* k, const
                                              float scale, const signed char* mask, const int* token_order, void* workspace,
                                              size_t ws_bytes, hipStream_t stream) {
   const int QB = Sq / 128 + (Sq % 128 != 0), KB = Skv / 128 + (Skv % 128 != 0);
-  if ((long long)B * N * QB > kListRows || !bsa_pair_supported(QB, KB))
+  if (!prefers_lists((long long)B * N, QB, KB) || !bsa_pair_supported(QB, KB))
     return mindiesd_block_sparse_attention_paired_fwd(q, k, v, out, lse, dtype, B, N, Nkv, Sq, Skv, D, q_sb, q_sn, q_ss, k_sb, k_sn,
                                                       k_ss, v_sb, v_sn, v_ss, o_sb, o_sn, o_ss, scale, mask, token_order,
                                                       workspace, ws_bytes, stream);

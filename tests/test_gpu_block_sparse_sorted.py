@@ -49,3 +49,26 @@ def test_paired_kernel_on_small_masks(cuda, monkeypatch, case, args):
     from mindiesd import _native
     monkeypatch.setattr(_native, "_lib", _Paired(_native.lib()))
     getattr(paired_cases, case)(cuda, *args)
+
+
+@pytest.mark.parametrize("n, qb, kb, lists", [
+    (8, 96, 64, True), (8, 97, 64, False),            # keys that stay in the L2: by the rows
+    (8, 64, 64, True), (8, 64, 65, False),            # 256 pairs, one whole round
+    (4, 96, 65, True), (4, 97, 65, False),            # 192 pairs, and 196
+    (6, 85, 65, True), (8, 80, 96, True), (8, 81, 96, False),   # odd rows: 258 pairs; 320; 328
+    (4, 96, 96, True), (4, 96, 97, False),
+    (2, 128, 97, True), (1, 255, 130, True), (2, 129, 97, False),   # 128 pairs; 130
+])
+def test_which_kernel_a_mask_takes(cuda, monkeypatch, n, qb, kb, lists):
+    """The lines of the dispatch, told by the bits: the two kernels add a row's key blocks up in different orders."""
+    from mindiesd import _native
+    from mindiesd.layers.flash_attn import rainfusion as rf
+    g = torch.Generator(device="cuda").manual_seed(100 * qb + kb)
+    q, k, v = (torch.randn(1, n, s, 128, generator=g, device=cuda).to(torch.bfloat16) for s in (128 * qb, 128 * kb, 128 * kb))
+    mask = torch.rand(1, n, qb, kb, generator=g, device=cuda) < 0.3
+    got = rf.block_sparse_attention_mask(q, k, v, mask, 0.09)
+    listed = rf.block_sparse_attention_lists(q, k, v, *rf.mask_to_lists(mask), 0.09)
+    monkeypatch.setattr(_native, "_lib", _Paired(_native.lib()))
+    paired = rf.block_sparse_attention_mask(q, k, v, mask, 0.09)
+    assert not torch.equal(listed, paired)
+    assert torch.equal(got, listed if lists else paired)
