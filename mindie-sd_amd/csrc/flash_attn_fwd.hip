@@ -1427,12 +1427,15 @@ __global__ void varlen_meta_kernel(const int* cu_q, const int* cu_k, int B, int 
 // The same, and zeros for the rows of `out` (row_chunks x 16 bytes each, no gaps) that no sequence covers.  A table whose entries
 // do not decrease, stay inside the tensor and lie at most max_q apart covers the rows from its first entry to its last; with any
 // other one every row is cleared, as sequences that overlap or were cut may leave tiles uncomputed.  A workgroup looks after
-// kFillRows rows and reads the table; where all of its rows are covered that is all it does.  Clearing the whole output in a
-// launch of its own, 65 MB for 12755 tokens x 20 heads, was 10 us and a gap of
-// 149, now 3: 24 heads x 10028 tokens 300 -> 291 us, 8 x 2973 26.4 -> 23.3 us.
-constexpr int kFillRows = 32;
+// kFillBytes of the output, however many rows that is, and reads the table; where all of its rows are covered that is all it does.
+// Clearing the whole output in a launch of its own, 65 MB for 12755 tokens x 20 heads, was 10 us and a gap of 149, now 3:
+// 24 heads x 10028 tokens 300 -> 291 us, 8 x 2973 26.4 -> 23.3 us.  Shares of 32 rows, a few KiB where the rows are narrow, cost more
+// workgroups, each with the whole table to read, than the launch saved: one head, 65536 rows, 255 sequences 32.5 us apart,
+// 33.3 with 32 rows, 28.4 with 64 KiB; 4095 sequences in 262144 rows 416, 438, 410 us (32, 128 and 256 KiB: within 1 % of that).
+constexpr int kFillBytes = 65536;
 __global__ __launch_bounds__(256) void varlen_meta_fill_kernel(const int* cu_q, const int* cu_k, int B, int total_q, int total_k,
-                                                               int max_q, int max_k, int* meta, i32x4_t* out, int row_chunks) {
+                                                               int max_q, int max_k, int* meta, i32x4_t* out, int row_chunks,
+                                                               int rows) {
   const int t = threadIdx.x;
   for (int b = blockIdx.x * 256 + t; b < B; b += gridDim.x * 256) varlen_meta_entry(cu_q, cu_k, b, total_q, total_k, max_q, max_k, meta);
   bool regular = true;
@@ -1442,11 +1445,13 @@ __global__ __launch_bounds__(256) void varlen_meta_fill_kernel(const int* cu_q, 
   }
   regular = __syncthreads_and(regular) != 0;
   const int covered0 = regular ? cu_q[0] : 0, covered1 = regular ? cu_q[B] : 0;
-  const int row0 = blockIdx.x * kFillRows, row1 = min(row0 + kFillRows, total_q);
-  for (int r = row0; r < row1; ++r) {
-    if (r >= covered0 && r < covered1) continue;
-    for (int c = t; c < row_chunks; c += 256) out[(long long)r * row_chunks + c] = i32x4_t{0, 0, 0, 0};
-  }
+  const int row0 = blockIdx.x * rows, row1 = row0 + min(rows, total_q - row0);
+  auto clear = [&](int from, int to) {
+    const long long end = (long long)to * row_chunks;
+    for (long long c = (long long)from * row_chunks + t; c < end; c += 256) out[c] = i32x4_t{0, 0, 0, 0};
+  };
+  clear(row0, min(row1, covered0));
+  clear(max(row0, covered1), row1);
 }
 
 }  // namespace msd
@@ -1827,8 +1832,9 @@ int mindiesd_varlen_meta_fill(const int* cu_seqlens_q, const int* cu_seqlens_k, 
   if (!cu_seqlens_q || !cu_seqlens_k || !seq_meta || !out || B <= 0 || total_q <= 0 || total_k < 0 || max_q < 0 || max_k < 0)
     return MSD_ERR_BAD_ARG;
   if ((((uintptr_t)seq_meta | (uintptr_t)out) & 15) || row_bytes <= 0 || (row_bytes & 15)) return MSD_ERR_BAD_ARG;
-  hipLaunchKernelGGL(varlen_meta_fill_kernel, dim3((total_q + kFillRows - 1) / kFillRows), dim3(256), 0, stream, cu_seqlens_q,
-                     cu_seqlens_k, B, total_q, total_k, max_q, max_k, seq_meta, (i32x4_t*)out, row_bytes / 16);
+  const int rows = (kFillBytes + row_bytes - 1) / row_bytes, grid = total_q / rows + (total_q % rows != 0);
+  hipLaunchKernelGGL(varlen_meta_fill_kernel, dim3(grid), dim3(256), 0, stream, cu_seqlens_q, cu_seqlens_k, B, total_q, total_k,
+                     max_q, max_k, seq_meta, (i32x4_t*)out, row_bytes / 16, rows);
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_ERR_LAUNCH;
 }
 

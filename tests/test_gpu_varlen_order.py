@@ -60,3 +60,21 @@ def test_rows_outside_of_a_device_table_are_cleared(cuda, table, total, max_q, c
     assert torch.equal(meta, want)
     assert (out[covered[0]:covered[1]] == 1).all()
     assert not out[:covered[0]].any() and not out[covered[1]:].any()
+
+
+@pytest.mark.parametrize("heads, d, total", [(1, 8, 12290), (1, 128, 769), (3, 24, 1400), (24, 128, 40), (300, 128, 9)])
+@pytest.mark.parametrize("where", ["none", "all", "tail", "head", "inside", "backwards"])
+def test_rows_outside_of_a_device_table_in_every_share(cuda, heads, d, total, where):
+    """The same over several workgroups' shares of the output: 4096, 256, 456 and 11 rows, one row; covered rows that end at a
+    share's edge and one row beside it."""
+    from mindiesd.layers.flash_attn.hip_flash_attn import _varlen_meta
+    share = -(-65536 // (2 * heads * d))
+    table = {"none": [0, 0], "all": [0, total // 2, total], "tail": [share, total], "head": [0, 1, total - 1],
+             "inside": [share - 1, share + 1, 2 * share], "backwards": [0, total, total - 1]}[where]
+    first, last = (0, 0) if where == "backwards" else (table[0], table[-1])
+    cu = torch.tensor(table, dtype=torch.int32, device=cuda)
+    guard = torch.ones(total + 8, heads, d, dtype=torch.bfloat16, device=cuda)
+    _varlen_meta(cu, cu, total, total, cu.device, None, None, guard[4:total + 4])
+    assert 2 * share < total and (guard[:4] == 1).all() and (guard[total + 4:] == 1).all()
+    out = guard[4:total + 4]
+    assert (out[first:last] == 1).all() and not out[:first].any() and not out[last:].any()
