@@ -8,12 +8,15 @@
 // (c = lane % 16, g = lane / 16) owns query columns 16 * nq + c, S^T blocks of 16 keys come from one 16-byte K read, V^T from
 // transposing reads.
 //
-// What bounds it: up to 128 keys reading Q and writing O (40 heads x 32760 queries x 128 keys 156 us = 3.5 TB/s), beyond that the
-// products and the LDS reads behind them, every wave all keys for its 32 rows (256 keys 204 us, 0.84 PFLOP/s).  Against the 4-wave
+// What bounds it: up to 128 keys reading Q and writing O (40 heads x 32760 queries x 128 keys 154 us, 676 MB behind the L2 = 4.4 TB/s,
+// the matrix pipe busy 25 % of the cycles), beyond that the products and the LDS reads behind them, every wave all keys for its 32
+// rows, and at 7 and 8 blocks the wait for queries that are not requested ahead (256 keys 204 us, 0.84 PFLOP/s, 41 %).  Against the 4-wave
 // kernel, which stages every key tile for each 128 rows: 40 heads x 32760 queries over 64 / 91 / 128 / 188 / 226 / 256 keys 160 / 177 /
 // 176 / 221 / 253 / 251 -> 154 / 155 / 156 / 168 / 200 / 204 us, 16 x 19666 33 / 41 / 41 / 50 / 57 / 57 -> 29 / 32 / 34 / 42 / 47 / 48 us,
-// 16 x 5000 13.6 / 16.3 / 16.1 / 19.2 / 21.1 / 21.2 -> 11.9 / 12.8 / 13.9 / 16.4 / 18.0 / 18.2 us.  Error against 64 bits 0.98 to 1.00 of
-// that kernel's (no rescaling).  Registers: 219 to 246, none spilled.
+// 16 x 5000 13.6 / 16.3 / 16.1 / 19.2 / 21.1 / 21.2 -> 11.9 / 12.8 / 13.9 / 16.4 / 18.0 / 18.2 us.  At most 64 keys (one key tile there)
+// over more than a million rows are the same copy of Q to O in both: 0.95 (2 x 12 heads x 60000) to 1.14 (8 x 40 x 4096), by heads and
+// layout.  Error against 64 bits 0.98 to 1.00 of that kernel's (no rescaling).  Vector registers: 160 with one block of 32 keys, 219 to
+// 246 with more, none spilled; scalar ones spilled 3 (two blocks) to 22 (eight), outside of the loop over the rows.
 #include <type_traits>
 #include <utility>
 

@@ -30,8 +30,10 @@ constexpr float kE4M3MaxMx = 448.0f;
 // ---- MX quantisation of a [M][K] 16-bit matrix along K -----------------------------------------------------
 // 4 lanes share one 32-element block (8 elements = 16 bytes each).  PACKED: rows follow one another without gaps, and as K is a
 // multiple of 32 the position in x alone gives those in the codes and scales; otherwise the row comes out of a 64-bit division,
-// some hundred instructions beside the fifty of the quantisation: 46344 x 1536 40.5 -> 36.6 us = 5.9 TB/s of the bytes moved (two or four pieces per thread, requested together,
-// are no faster: 165.3 and 166.3 against 164.6 us for the layer with 46344 x 1536 x 1536.)
+// some hundred instructions beside the fifty of the quantisation: 46344 x 1536 40.5 -> 36.6 us = 5.9 TB/s of the bytes moved,
+// 4096 x 5120 12.7 -> 11.4, 512 x 5120 3.6 -> 3.2 us by itself and 4.7 either way behind a GEMM, whose operands have taken x out of
+// the L2 (two or four pieces per thread, requested together, are no faster: 165.3 and 166.3 against 164.6 us for the layer with
+// 46344 x 1536 x 1536).
 template <int DT, bool PACKED>
 __global__ __launch_bounds__(256) void mx_quant_kernel(const void* x_, unsigned char* q, unsigned char* e8m0,
                                                        long long M, int K, long long x_stride) {
@@ -372,7 +374,8 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(const GemmParams p) 
   // row and instruction, the 32 rows of a store were 32 requests to the L2 for 16 bytes each, 4 us of a
   // tile's 27 at K 1536.  Layers, before -> now: 39552 x 1536 x 4608 372 -> 318 us, 46344 x 1536 x 1536 190 -> 168, 4395 x 3072 x 12288
   // 189 -> 170, 10261 x 5120 x 15360 760 -> 690; SwiGLU, half the output and two transcendental instructions for each:
-  // 7756 x 1536 x 2 x 3072 92 -> 88, 32760 x 5120 x 2 x 13824 3734 -> 3675 us.
+  // 7756 x 1536 x 2 x 3072 92 -> 88, 32760 x 5120 x 2 x 13824 3734 -> 3675 us.  The plain form spills 2 of its 512 vector registers
+  // around these stores, outside of the loop; the SwiGLU form and the smaller tiles none.
   T* og = (T*)p.out;
   int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));  // the lane's number anew: not kept through the loop
   asm volatile("" : "+v"(el));

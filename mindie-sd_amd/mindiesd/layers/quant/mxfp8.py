@@ -85,8 +85,8 @@ _CODE_DTYPES = (torch.uint8, torch.float8_e4m3fn, torch.float8_e8m0fnu)
 def mxfp8_linear(x, w_q, w_scale, bias=None, out_dtype=torch.bfloat16, swiglu=False):
     """``mxfp8_matmul(*mx_quantize(x), w_q, w_scale, bias, out_dtype, swiglu)`` as one native call, for x [..., K] bf16/fp16
     with any leading dimensions; result [..., Nw] or [..., Nw/2].  A layer on a few hundred tokens is
-    over sooner than the host has made the two calls with their tensors, views and checks (28 us a layer, this one call:
-    15 us), so the codes and scales share one allocation, and only what is not contiguous is viewed or copied."""
+    over sooner than the host has made the two calls with their tensors, views and checks (28 us a layer, with this one call
+    17 us, of which 2 are the layer's views), so the codes and scales share one allocation, and only what is not contiguous is viewed or copied."""
     if not isinstance(x, torch.Tensor) or x.dim() < 1 or not x.is_cuda or x.dtype not in _native.DTYPE_CODE:
         raise ParametersInvalid("mx_quantize needs a 2-D bf16/fp16 GPU tensor.")
     *lead, k = x.shape
